@@ -156,8 +156,10 @@ int lbq_weight_info(const lbq_weight *w, uint32_t *ggml_type, int64_t *n, int64_
  * adds when y is plain device memory (hipMalloc; checked once per allocation),
  * else through partial sums in the workspace; either way y = a + b for the two
  * halves, the same bits for finite normal-range halves.  Dense F32/F16/BF16
- * weights are candle's dense variant: no quantisation, an f32 matmul.  m == 0 is
- * a no-op. */
+ * weights are candle's dense variant: no quantisation, an f32 matmul (F16 / BF16
+ * at m > 8: x as 16-bit operands that add up to it, in the context's scratch;
+ * under a graph capture that would have to grow that scratch, the f32 matrix
+ * cores).  m == 0 is a no-op. */
 int lbq_qmatmul_f32(lbq_ctx *ctx, const lbq_weight *w, const float *d_x, int64_t m, float *d_y, void *stream);
 
 /* lbq_qmatmul_f32's result (the same kernels, the same bits), allocating
@@ -170,7 +172,8 @@ int lbq_qmatmul_f32(lbq_ctx *ctx, const lbq_weight *w, const float *d_x, int64_t
  * call), resolved by lbq_init and held until the process ends.  A call that needs more (roughly
  * m * k * 2 bytes of fp16 operands plus split-k partials above m = 8; every
  * Llama-3-8B projection fits up to m = 512, down_proj up to m = 2048) returns
- * LBQ_ERR_LIMIT before launching anything.  All contexts on a device share the
+ * LBQ_ERR_LIMIT before launching anything; a dense weight's call that needs more
+ * runs lbq_qmatmul_f32's form without scratch instead (f32 matrix cores).  All contexts on a device share the
  * one array, which keeps the last call's contents: calls that overlap on one
  * device (on different streams or threads) race and must be ordered by the
  * caller. */

@@ -14,6 +14,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "../../include/lbq.h"
 #include "lbq_device.hpp"
@@ -41,6 +42,13 @@ struct lbq_ctx {
     size_t ws_bytes;
     uint8_t *tmp;         // gate and up outputs when their product is not fused
     size_t tmp_bytes;
+    // dense F16 / BF16 at m > 8: operand pieces and split-k partials.  Outgrown buffers
+    // stay until the context goes (their sizes double, so they add up to less than the
+    // current one): a captured graph may still use them.
+    uint8_t *dense_ws;
+    size_t dense_ws_bytes;
+    std::vector<uint8_t *> dense_old;
+    hipStream_t dense_stream;  // the last call's
     uint32_t *tile_counters;  // KS_COUNTERS zeroed words of the k-sliced GEMM (each launch leaves them zero)
 };
 
@@ -363,17 +371,65 @@ int run_dot(Scratch &sc, const lbq_weight *w, const lbq::ActView &av, int64_t m,
     return LBQ_OK;
 }
 
+// The operand workspace of a dense call, or null where the f32 kernel has to run
+// without one: types and m that have no such path, fixed scratch that is too small,
+// and a stream under capture whose buffer would have to be allocated.  The dense
+// path keeps its own buffer: a call on another stream than the last one's waits for
+// the device first, as the buffer may still be in use there.
+uint8_t *dense_workspace(Scratch &sc, const lbq_weight *w, int64_t m, hipStream_t st) {
+    const size_t need = lbq::dense_workspace_bytes(w->type, w->n, w->k, m);
+    if (!need) return nullptr;
+    if (sc.fixed) return need <= sc.fixed_bytes ? sc.fixed : nullptr;
+    lbq_ctx *c = sc.ctx;
+    const bool grow = need > c->dense_ws_bytes, moved = c->dense_ws && st != c->dense_stream;
+    if (grow || moved) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (cap != hipStreamCaptureStatusNone) return grow ? nullptr : c->dense_ws;
+        if (moved && hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (grow) {
+            const size_t want = align_up(std::max(need, 2 * c->dense_ws_bytes), 1 << 20);
+            void *p = nullptr;
+            try {
+                c->dense_old.reserve(c->dense_old.size() + 1);
+            } catch (...) {
+                return nullptr;
+            }
+            if (hipMalloc(&p, want) != hipSuccess) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
+            if (c->dense_ws) c->dense_old.push_back(c->dense_ws);
+            c->dense_ws = static_cast<uint8_t *>(p);
+            c->dense_ws_bytes = want;
+        }
+    }
+    c->dense_stream = st;
+    return c->dense_ws;
+}
+
+// candle's dense variant: an f32 matmul, no activation quantisation.  `mu`: as forward's.
+int dense_forward(const lbq_weight *w, const float *d_x, int64_t m, float *d_y, hipStream_t st, Scratch &sc,
+                  std::mutex *mu) {
+    std::unique_lock<std::mutex> lock;
+    if (mu && m > 8) lock = std::unique_lock<std::mutex>(*mu);
+    hipError_t e = lbq::launch_dense(w->type, w->d_blocks, w->n, w->k, d_x, m, d_y, dense_workspace(sc, w, m, st), st);
+    return e == hipSuccess ? LBQ_OK : hip_fail(e, "dense matmul launch");
+}
+
 // QMatMul::forward after the argument checks, on the caller's device; `mu`
 // (the context's lock, null for the fixed region) is taken before any buffer is
 // touched.
 int forward(lbq_ctx *ctx, const lbq_weight *w, const float *d_x, int64_t m, float *d_y, hipStream_t st, Scratch &sc,
             std::mutex *mu) {
     const int act_type = lbq::vec_dot_type(w->type);
-    if (lbq::is_dense(w->type)) {
-        // candle's dense variant: an f32 matmul, no activation quantisation
-        hipError_t e = lbq::launch_dense(w->type, w->d_blocks, w->n, w->k, d_x, m, d_y, st);
-        return e == hipSuccess ? LBQ_OK : hip_fail(e, "dense matmul launch");
-    }
+    if (lbq::is_dense(w->type)) return dense_forward(w, d_x, m, d_y, st, sc, mu);
     const ActLayout L = act_layout(act_type, m, w->k);
     if (m <= 8 && !uses_mx(w, m) && lbq::gemv_fuses_quant(w->type, w->n, w->k, (int)m, d_x)) {
         // decode: the GEMV quantises x in its own prologue -- one launch, no scratch
@@ -567,6 +623,9 @@ int lbq_init(int device, lbq_ctx **out_ctx) {
     c->ws_bytes = 0;
     c->tmp = nullptr;
     c->tmp_bytes = 0;
+    c->dense_ws = nullptr;
+    c->dense_ws_bytes = 0;
+    c->dense_stream = nullptr;
     c->tile_counters = nullptr;
     e = hipMalloc(&c->tile_counters, NOALLOC_COUNTER_BYTES);
     if (e == hipSuccess) e = hipMemset(c->tile_counters, 0, NOALLOC_COUNTER_BYTES);
@@ -587,6 +646,8 @@ int lbq_ctx_destroy(lbq_ctx *ctx) {
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     if (ctx->ws) (void)hipFree(ctx->ws);
     if (ctx->tmp) (void)hipFree(ctx->tmp);
+    if (ctx->dense_ws) (void)hipFree(ctx->dense_ws);
+    for (uint8_t *p : ctx->dense_old) (void)hipFree(p);
     if (ctx->tile_counters) (void)hipFree(ctx->tile_counters);
     delete ctx;
     return LBQ_OK;
@@ -737,9 +798,11 @@ int group_f32(lbq_ctx *ctx, const lbq_weight *const *ws, int count, const float 
     lbq::TuningScope tsc(&ctx->tune);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (lbq::is_dense(w0->type)) {
+        Scratch sc;
+        sc.ctx = ctx;
         for (int i = 0; i < count; i++) {
-            hipError_t e = lbq::launch_dense(ws[i]->type, ws[i]->d_blocks, ws[i]->n, ws[i]->k, d_x, m, d_ys[i], st);
-            if (e != hipSuccess) return hip_fail(e, "dense matmul launch");
+            const int s = dense_forward(ws[i], d_x, m, d_ys[i], st, sc, &ctx->mu);
+            if (s) return s;
         }
         return LBQ_OK;
     }

@@ -10,10 +10,13 @@
 //           the next unit's 16-byte loads in flight, x staged in LDS, f32 FMA
 //           against up to 8 activation rows, DPP row sums -- HBM-bound like the
 //           quantised decode GEMV;
-//   m > 8   k_dense_gemm: 64 x 128 output tiles on v_mfma_f32_32x32x2_f32
-//           (f32 operands, f32 accumulation), operands staged through LDS.
-// Both compute in f32 throughout; only the summation order differs from
-// candle's, so results agree to f32 rounding (~1e-6 relative on a row).
+//   m > 8   k_dense_mm (F16 / BF16): x as two fp16 or three bf16 operands that add
+//           up to it, on the 16-bit matrix cores with f32 accumulation;
+//           k_dense_gemm (F32 weights, and calls without a workspace): 64 x 128
+//           output tiles on v_mfma_f32_32x32x2_f32, operands staged through LDS.
+// Every product is formed at f32 precision or better and summed in f32; only the
+// summation order differs from candle's, so results agree to f32 rounding (~1e-6
+// relative on a row).
 #include <algorithm>
 
 #include "lbq_device.hpp"
@@ -277,6 +280,371 @@ __global__ __launch_bounds__(256) void k_dense_gemm(const uint8_t *__restrict__ 
         }
 }
 
+
+// ---------------------------------------------------------------------------
+// m > 8 with F16 / BF16 weights: the weights are fp16 / bf16 MFMA operands as they
+// lie in memory, and x enters as P operands of the same type that add up to it:
+//   F16   P = 2: x * 2^-e = hi + lo, e the row's exponent (largest finite |x| in
+//         [2^14, 2^15) after it), hi and lo rounded to nearest: 22 bits and the
+//         rounding sign of x (lo is exact to 2^-25, so what a value loses below
+//         that is 2^-39 of the row's largest);
+//   BF16  P = 3: x = hi + mid + lo by truncation, 3 x 8 bits: exact, no exponent.
+// Every product is exact in the f32 accumulator of v_mfma_f32_32x32x16_{f16,bf16},
+// so only the f32 summation rounds.  P MFMAs of 16 k-values replace eight
+// v_mfma_f32_32x32x2_f32, at 16 times their rate.  Bound by the matrix cores and
+// their clock from M = 512 (0.9-1.1 PFLOP/s of operand products), by the launches
+// below.  Against k_dense_gemm, us per call and relative error against 64 bits:
+//   F16 4096^2    M = 9 / 64 / 512   237 / 241 / 244 -> 15.6 / 21.1 / 47.7, 1.1e-6 -> 4.1e-7
+//   F16 8192^2    M = 2048           3003 -> 503,  1.6e-6 -> 8.2e-7
+//   BF16 4096^2   M = 32 / 512       239 / 246 -> 17.1 / 57.2, 1.1e-6 -> 5.0e-7
+//   BF16 8192^2   M = 2048           3003 -> 955,  1.6e-6 -> 1.0e-6
+//   F16 512^2     M = 9              32.2 -> 14.0, 4e-7 -> 1.6e-7
+//
+// Tiles.  A workgroup of WM x WN waves owns BM = 32 WM TM rows of x and
+// BN = 32 WN TN weight rows; a wave its TM x TN tiles of 32 x 32.  k advances in
+// stages of 64: the P x BM x 64 pieces and the BN x 64 weights go into LDS by
+// buffer loads to LDS (16 B a lane, 8 rows of 128 B an instruction), two buffers;
+// row r's 16-byte chunk c sits in slot c ^ ((r >> 1) & 7), so the 32 rows of an
+// operand read spread over the banks.  One barrier a stage, before its last k-step:
+// there every wave has read the whole stage (and its own loads of the next one have
+// landed), so the buffer is refilled, and the next stage's first operands are
+// read, under the last k-step's MFMAs.  Rows past N and k past K read as zero
+// (outside the buffer resource); rows past M are never stored.
+// Few tiles: k is split over workgroups whose partial sums k_dense_sum adds in
+// slice order.
+//
+// A result that is not finite is formed again from x and W by f32 FMAs in k order
+// (dense_dot): an infinity in x or W would otherwise meet the zero lo pieces.
+// ---------------------------------------------------------------------------
+constexpr int DK = 64;  // values of k per stage
+
+typedef _Float16 dhalf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 dbf8 __attribute__((ext_vector_type(8)));
+
+template <bool BF>
+__device__ __forceinline__ floatx16 dense_mfma(uint4 a, uint4 b, floatx16 c) {
+    if constexpr (BF)
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(dbf8, a), __builtin_bit_cast(dbf8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(dhalf8, a), __builtin_bit_cast(dhalf8, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ bool dense_finite(float v) { return fabsf(v) <= 3.4028234664e38f; }  // false for NaN
+
+template <bool BF>
+__device__ __attribute__((noinline)) float dense_dot(const float *x, const uint8_t *w, int64_t K) {
+    float s = 0.f;
+    for (int64_t i = 0; i < K; i++) s = fmaf(w16<BF>(reinterpret_cast<const unsigned short *>(w)[i]), x[i], s);
+    return s;
+}
+
+// x [M][K] -> pieces [P][rows][Kp] (Kp = K up to a multiple of DK, zero filled) and,
+// for F16, the row exponents; one workgroup per row of x.
+template <bool BF>
+__global__ __launch_bounds__(256) void k_dense_pieces(const float *__restrict__ x, int64_t K, int64_t Kp, int64_t rows,
+                                                      unsigned short *__restrict__ A, int *__restrict__ erow) {
+    const int64_t m = blockIdx.x;
+    const int t = threadIdx.x;
+    const bool xv = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    const float *xr = x + m * K;
+    int e = 0;
+    if constexpr (!BF) {
+        __shared__ float wmax[4];
+        float mx = 0.f;
+        for (int64_t c = 8 * t; c < K; c += 2048) {
+            float v[8];
+            load_x8(xr + c, xv, v);
+#pragma unroll
+            for (int i = 0; i < 8; i++) mx = fmaxf(mx, dense_finite(v[i]) ? fabsf(v[i]) : 0.f);
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+        if ((t & 63) == 0) wmax[t >> 6] = mx;
+        __syncthreads();
+        mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+        e = mx > 0.f ? __builtin_amdgcn_frexp_expf(mx) - 15 : 0;
+        if (t == 0) erow[m] = e;
+    }
+    unsigned short *a = A + m * Kp;
+    const int64_t ps = rows * Kp;
+    for (int64_t c = 8 * t; c < Kp; c += 2048) {
+        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (c < K) load_x8(xr + c, xv, v);
+        uint32_t pc[3][4];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            uint32_t b[3];
+            if constexpr (BF) {
+                const uint32_t u0 = __float_as_uint(v[i]);
+                const bool fin = dense_finite(v[i]);
+                // a NaN keeps a mantissa bit in the upper half
+                b[0] = (u0 >> 16) | (v[i] != v[i] ? 0x40u : 0u);
+                const float r1 = v[i] - __uint_as_float(u0 & 0xffff0000u);
+                const uint32_t u1 = fin ? __float_as_uint(r1) : 0u;
+                b[1] = u1 >> 16;
+                b[2] = fin ? __float_as_uint(r1 - __uint_as_float(u1 & 0xffff0000u)) >> 16 : 0u;
+            } else {
+                const float s = __builtin_amdgcn_ldexpf(v[i], -e);
+                const _Float16 hi = (_Float16)s;
+                const _Float16 lo = (_Float16)(dense_finite(s) ? s - (float)hi : 0.f);
+                b[0] = __builtin_bit_cast(unsigned short, hi);
+                b[1] = __builtin_bit_cast(unsigned short, lo);
+                b[2] = 0u;
+            }
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                if (i & 1) pc[p][i >> 1] |= b[p] << 16;
+                else pc[p][i >> 1] = b[p];
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < (BF ? 3 : 2); p++)
+            *reinterpret_cast<uint4 *>(a + p * ps + c) = make_uint4(pc[p][0], pc[p][1], pc[p][2], pc[p][3]);
+    }
+}
+
+// a buffer resource over [p, p + bytes), wave-uniform
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dense_rsrc(const void *p, int64_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
+                       ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32);
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(u), (short)0,
+                                             __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+
+struct DenseGrid {
+    int tiles_m, tiles_n, splits, sps;  // sps: stages of k per split
+    int64_t rows, Kp;                   // rows of a piece, its row length
+    int64_t split_stride;               // partials apart (0: out is y)
+};
+
+template <bool BF, int P, int WM, int WN, int TM, int TN>
+__global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__restrict__ W, int64_t N, int64_t K,
+                                                           const unsigned short *__restrict__ A,
+                                                           const int *__restrict__ erow, const float *__restrict__ x,
+                                                           int64_t M, float *__restrict__ out, DenseGrid g) {
+    constexpr int NW = WM * WN, BM = 32 * WM * TM, BN = 32 * WN * TN;
+    constexpr int RA = BM / 8 / NW, RB = BN / 8 / NW;  // staging instructions per wave: RA per piece, RB
+    static_assert(RA * 8 * NW == BM && RB * 8 * NW == BN && NW % 2 == 0, "whole staging instructions per wave");
+    __shared__ __align__(1024) uint8_t As0[P * BM * 128], As1[P * BM * 128];
+    __shared__ __align__(1024) uint8_t Bs0[BN * 128], Bs1[BN * 128];
+    // tiles that share weight rows on one XCD
+    const int G = (int)gridDim.x, L = (int)blockIdx.x;
+    const int T = (G & 7) == 0 ? (L & 7) * (G >> 3) + (L >> 3) : L;
+    const int tm = T % g.tiles_m, tn = (T / g.tiles_m) % g.tiles_n, z = T / (g.tiles_m * g.tiles_n);
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+    const int s0 = z * g.sps, ns = min(g.sps, (int)(g.Kp / DK) - s0);  // ns >= 1
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5, lr = lane & 31;
+    const int wm = wave / WN, wn = wave % WN;
+
+    const __amdgpu_buffer_rsrc_t a0 = dense_rsrc(A + m0 * g.Kp, BM * g.Kp * 2);
+    const __amdgpu_buffer_rsrc_t a1 = dense_rsrc(A + (g.rows + m0) * g.Kp, BM * g.Kp * 2);
+    const __amdgpu_buffer_rsrc_t a2 = dense_rsrc(A + ((P - 1) * g.rows + m0) * g.Kp, BM * g.Kp * 2);
+    const __amdgpu_buffer_rsrc_t br = dense_rsrc(W + n0 * K * 2, (N - n0 < BN ? N - n0 : BN) * K * 2);
+    // lane l of an instruction fills row l/8, slot l%8 of its 8 rows; the rows' number
+    // / 8 has the wave's parity (NW is even)
+    const int ch = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
+    const uint32_t va = (uint32_t)((lane >> 3) * (int)g.Kp * 2 + 16 * ch);
+    const uint32_t vb = (uint32_t)((lane >> 3) * (int)K * 2 + 16 * ch);
+    // stage s (of the slice) into buffer `buf`; past the slice, zeros (no memory access).
+    // Straight-line code with the buffers' names in it: a load to LDS that the compiler
+    // cannot tell from a read's buffer makes it wait for the load before the read.
+    auto stage_in = [&](int s, int buf) __attribute__((always_inline)) {
+        const int k0 = (s0 + s) * DK;
+        const uint32_t v0 = s < ns ? va : 0x80000000u;
+#pragma unroll
+        for (int p = 0; p < P; p++)
+#pragma unroll
+            for (int j = 0; j < RA; j++) {
+                const int rb = wave + NW * j;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    p == 0 ? a0 : p == 1 ? a1 : a2, (__attribute__((address_space(3))) void *)((buf ? As1 : As0) + (p * BM + 8 * rb) * 128), 16, v0,
+                    (8 * rb * (int)g.Kp + k0) * 2, 0, 0);
+            }
+        const uint32_t v1 = s < ns && k0 + 8 * ch < (int)K ? vb : 0x80000000u;  // past K: zero
+#pragma unroll
+        for (int j = 0; j < RB; j++) {
+            const int rb = wave + NW * j;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                br, (__attribute__((address_space(3))) void *)((buf ? Bs1 : Bs0) + 8 * rb * 128), 16, v1,
+                (8 * rb * (int)K + k0) * 2, 0, 0);
+        }
+    };
+    // byte offsets of a lane's operands of k-step ks, kept as plain numbers (a chain of
+    // pointer steps hides from the compiler which buffer it points into)
+    int oa[4], ob[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) {
+        const int o = lr * 128 + 16 * ((2 * ks + h) ^ ((lr >> 1) & 7));
+        oa[ks] = o + wm * TM * 4096;
+        ob[ks] = o + wn * TN * 4096;
+        asm volatile("" : "+v"(oa[ks]), "+v"(ob[ks]));
+    }
+
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+    // operands of this k-step and the next; operand q of a k-step: its TN B, then its P TM A
+    constexpr int NO = TN + P * TM, NM = P * TM * TN;  // operands, MFMAs per k-step
+    uint4 op[2][NO];
+    auto read = [&](int buf, int ks, int r, int q) __attribute__((always_inline)) {
+        if (q < TN) op[r][q] = *reinterpret_cast<const uint4 *>((buf ? Bs1 : Bs0) + (ob[ks] + q * 4096));
+        else
+            op[r][q] = *reinterpret_cast<const uint4 *>((buf ? As1 : As0) +
+                                                        (oa[ks] + (q - TN) / TM * (BM * 128) + (q - TN) % TM * 4096));
+    };
+    // the MFMAs of the k-step in op[r], each followed by its share of the next one's reads
+    auto step = [&](int r, int buf, int ks) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < NM; u++) {
+            const int j = u % TN, i = u / TN % TM, p = u / TN / TM;
+            acc[i][j] = dense_mfma<BF>(op[r][TN + p * TM + i], op[r][j], acc[i][j]);
+#pragma unroll
+            for (int q = u * NO / NM; q < (u + 1) * NO / NM; q++) read(buf, ks, r ^ 1, q);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    stage_in(0, 0);
+    stage_in(1, 1);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NO; q++) read(0, 0, 0, q);
+    auto stage = [&](int s, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ks = 0; ks < 3; ks++) step(ks & 1, buf, ks + 1);
+        __builtin_amdgcn_s_waitcnt(0);  // this wave's operands, and its loads of stage s + 1
+        __syncthreads();
+        stage_in(s + 2, buf);
+        __builtin_amdgcn_sched_barrier(0);
+        step(1, buf ^ 1, 0);
+    };
+    for (int s = 0; s < ns; s += 2) {  // an odd count ends with a stage of zeros
+        stage(s, 0);
+        stage(s + 1, 1);
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // the loads past the slice
+    // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
+    float *y = out + (int64_t)z * g.split_stride;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int64_t n = n0 + 32 * (wn * TN + j) + lr;
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int64_t m = m0 + 32 * (wm * TM + i) + 8 * (v >> 2) + 4 * h + (v & 3);
+                if (m >= M || n >= N) continue;
+                float r = acc[i][j][v];
+                if (g.split_stride == 0) {
+                    if constexpr (!BF) r = __builtin_amdgcn_ldexpf(r, erow[m]);
+                    if (!dense_finite(r)) r = dense_dot<BF>(x + m * K, W + n * K * 2, K);
+                }
+                y[m * N + n] = r;
+            }
+        }
+}
+
+// y[m][n] = 2^e_m * (sum over the slices, in order); blockIdx.y: row m
+template <bool BF>
+__global__ __launch_bounds__(256) void k_dense_sum(const float *__restrict__ part, int S, int64_t M, int64_t N,
+                                                   const int *__restrict__ erow, const float *__restrict__ x,
+                                                   const uint8_t *__restrict__ W, int64_t K, float *__restrict__ y) {
+    const int64_t m = blockIdx.y, st = M * N;
+    const int e = BF ? 0 : erow[m];
+    const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (n >= N) return;
+    const float *p = part + m * N + n;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    if ((N & 3) == 0) {
+        for (int z0 = 0; z0 < S; z0 += 8) {
+            float4 v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (z0 + j < S) v[j] = *reinterpret_cast<const float4 *>(p + (z0 + j) * st);
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (z0 + j < S) { s[0] += v[j].x; s[1] += v[j].y; s[2] += v[j].z; s[3] += v[j].w; }
+        }
+    } else {
+        for (int i = 0; i < 4 && n + i < N; i++)
+            for (int z = 0; z < S; z++) s[i] += p[z * st + i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if (n + i >= N) break;
+        float r = BF ? s[i] : __builtin_amdgcn_ldexpf(s[i], e);
+        if (!dense_finite(r)) r = dense_dot<BF>(x + m * K, W + (n + i) * K * 2, K);
+        y[m * N + n + i] = r;
+    }
+}
+
+namespace {
+struct DensePlan {
+    int bm, bn;
+    DenseGrid g;
+    size_t a_off, e_off, part_off, total;
+};
+// Tile by m (32, 64, 128 rows; 128 x 256 for F16 where such tiles fill the chip by
+// themselves), then k split until the resident workgroups (LDS: three of the 32-row
+// tiles a CU, two of the 64-row, one of the 128-row) are there, at least four
+// stages a slice.
+DensePlan dense_plan(int type, int64_t n, int64_t k, int64_t m) {
+    DensePlan p;
+    const int P = type == TYPE_BF16 ? 3 : 2;
+    p.bm = m <= 32 ? 32 : m <= 64 ? 64 : 128;
+    p.bn = 128;
+    const int64_t cus = num_cus();
+    if (p.bm == 128 && P == 2 && ((m + 127) / 128) * ((n + 255) / 256) * 4 >= 3 * cus) p.bn = 256;
+    p.g.tiles_m = (int)((m + p.bm - 1) / p.bm);
+    p.g.tiles_n = (int)((n + p.bn - 1) / p.bn);
+    p.g.rows = (int64_t)p.g.tiles_m * p.bm;
+    p.g.Kp = (k + DK - 1) / DK * DK;
+    const int64_t ns = p.g.Kp / DK, tiles = (int64_t)p.g.tiles_m * p.g.tiles_n;
+    const int64_t slots = cus * (p.bm == 32 ? 3 : p.bm == 64 ? 2 : 1);
+    const int64_t s = std::max<int64_t>(1, std::min(slots / tiles, ns / 4));
+    p.g.sps = (int)((ns + s - 1) / s);
+    p.g.splits = (int)((ns + p.g.sps - 1) / p.g.sps);
+    p.g.split_stride = p.g.splits > 1 ? m * n : 0;
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    p.a_off = 0;
+    p.e_off = up((size_t)P * (size_t)p.g.rows * (size_t)p.g.Kp * 2);
+    p.part_off = p.e_off + up((size_t)m * 4);
+    p.total = p.part_off + (p.g.splits > 1 ? up((size_t)p.g.splits * (size_t)(m * n) * 4) : 0);
+    return p;
+}
+}  // namespace
+
+size_t dense_workspace_bytes(int type, int64_t n, int64_t k, int64_t m) {
+    // the pieces' buffer resources: 128 rows of k within 2^31 bytes
+    if ((type != TYPE_F16 && type != TYPE_BF16) || m <= 8 || k % 8 || k > (1 << 22) || m > 65535) return 0;
+    return dense_plan(type, n, k, m).total;
+}
+
+template <bool BF>
+static hipError_t dense_pieces(int type, const uint8_t *w, int64_t n, int64_t k, const float *x, int64_t m, float *y,
+                               uint8_t *ws, hipStream_t st) {
+    const DensePlan p = dense_plan(type, n, k, m);
+    unsigned short *a = reinterpret_cast<unsigned short *>(ws + p.a_off);
+    int *e = reinterpret_cast<int *>(ws + p.e_off);
+    float *out = p.g.splits > 1 ? reinterpret_cast<float *>(ws + p.part_off) : y;
+    k_dense_pieces<BF><<<(unsigned)m, 256, 0, st>>>(x, k, p.g.Kp, p.g.rows, a, e);
+    const unsigned grid = (unsigned)(p.g.tiles_m * p.g.tiles_n * p.g.splits);
+    constexpr int P = BF ? 3 : 2;
+    if (p.bm == 32) k_dense_mm<BF, P, 1, 4, 1, 1><<<grid, 256, 0, st>>>(w, n, k, a, e, x, m, out, p.g);
+    else if (p.bm == 64) k_dense_mm<BF, P, 2, 4, 1, 1><<<grid, 512, 0, st>>>(w, n, k, a, e, x, m, out, p.g);
+    else if (p.bn == 128) k_dense_mm<BF, P, 4, 2, 1, 2><<<grid, 512, 0, st>>>(w, n, k, a, e, x, m, out, p.g);
+    else if constexpr (!BF) k_dense_mm<BF, P, 2, 4, 2, 2><<<grid, 512, 0, st>>>(w, n, k, a, e, x, m, out, p.g);
+    if (p.g.splits > 1)
+        k_dense_sum<BF><<<dim3((unsigned)((n + 1023) / 1024), (unsigned)m), 256, 0, st>>>(out, p.g.splits, m, n, e, x, w,
+                                                                                        k, y);
+    return hipGetLastError();
+}
+
 template <bool F16, bool BF = false>
 static hipError_t dense_typed(const uint8_t *w, int64_t n, int64_t k, const float *x, int64_t m, float *y,
                               hipStream_t st) {
@@ -302,8 +670,11 @@ static hipError_t dense_typed(const uint8_t *w, int64_t n, int64_t k, const floa
 }
 
 hipError_t launch_dense(int type, const uint8_t *w, int64_t n, int64_t k, const float *x, int64_t m, float *y,
-                        hipStream_t st) {
+                        void *ws, hipStream_t st) {
     if (k % 8 || m > 65535LL * DBM) return hipErrorInvalidValue;
+    if (ws && dense_workspace_bytes(type, n, k, m))
+        return type == TYPE_BF16 ? dense_pieces<true>(type, w, n, k, x, m, y, static_cast<uint8_t *>(ws), st)
+                                 : dense_pieces<false>(type, w, n, k, x, m, y, static_cast<uint8_t *>(ws), st);
     if (type == TYPE_F16) return dense_typed<true>(w, n, k, x, m, y, st);
     if (type == TYPE_F32) return dense_typed<false>(w, n, k, x, m, y, st);
     if (type == TYPE_BF16) return dense_typed<true, true>(w, n, k, x, m, y, st);

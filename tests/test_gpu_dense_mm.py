@@ -1,0 +1,137 @@
+"""Dense F16 / BF16 weights at m > 8: x as 16-bit operands that add up to it, on the
+matrix cores, against a float64 product.
+
+Bound: every product is exact in the f32 accumulator, so a row's relative L2 error is
+that of adding P k/16 partial sums one after the other, each rounded to half an ulp
+(2^-24) of the running sum: 2^-24 sqrt(P k / 16) for errors of independent sign, taken
+twice, and never below f32's own rounding of a handful of steps.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_parity import to_dev
+
+pytestmark = pytest.mark.gpu
+F16, BF16 = 1, 30
+
+
+def _weight(t, n, k, rng, dev, w=None):
+    from lightbulb_amd.quantized import GgmlDType, QMatMul, QTensor
+    w = torch.from_numpy((rng.standard_normal((n, k)) * 0.05).astype(np.float32) if w is None else w)
+    w = w.to(torch.float16 if t == F16 else torch.bfloat16)
+    qm = QMatMul.from_qtensor(QTensor(w.reshape(-1).view(torch.uint8).to(dev), GgmlDType(t), (n, k)))
+    return qm, w.to(torch.float64).numpy()
+
+
+def _bound(t, k):
+    return 2.0 ** -23 * max(4.0, ((3 if t == BF16 else 2) * k / 16) ** 0.5)
+
+
+def _assert_rows(y, ref, bound):
+    err = np.linalg.norm(y.astype(np.float64) - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert err.max() <= bound, (err.max(), bound)
+
+
+@pytest.mark.parametrize("t", [F16, BF16])
+# each row tile's edges (32, 64, 128 rows), column tiles of 128 and 256, k that is no
+# multiple of a stage (64) or of two, one stage, slices of k and none
+@pytest.mark.parametrize("m,n,k", [(9, 1, 8), (32, 130, 520), (33, 300, 4096), (64, 127, 72), (65, 257, 1000),
+                                   (128, 640, 2048), (129, 4096, 64), (700, 8200, 200), (300, 64, 14336)])
+def test_dense_mm_shapes(lbq, dev, t, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    qm, w = _weight(t, n, k, rng, dev)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[rng.random(x.shape) < 0.01] *= 20
+    _assert_rows(qm.forward(to_dev(x, dev)).cpu().numpy(), x.astype(np.float64) @ w.T, _bound(t, k))
+
+
+@pytest.mark.parametrize("t", [F16, BF16])
+def test_dense_mm_range_and_alignment(lbq, dev, t):
+    # rows of very different size, subnormal rows, zero rows; x only 4-byte aligned
+    rng = np.random.default_rng(7)
+    m, n, k = 40, 200, 264
+    qm, w = _weight(t, n, k, rng, dev)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x *= (10.0 ** rng.integers(-30, 30, (m, 1))).astype(np.float32)
+    x[3] = 0
+    base = to_dev(np.concatenate([[0], x.reshape(-1)]).astype(np.float32), dev)
+    y = qm.forward(base[1:].reshape(m, k)).cpu().numpy()
+    rows = [r for r in range(m) if r != 3]
+    _assert_rows(y[rows], (x.astype(np.float64) @ w.T)[rows], _bound(t, k))
+    assert not y[3].any()
+
+
+@pytest.mark.parametrize("t", [F16, BF16])
+@pytest.mark.parametrize("m,n,k", [(20, 140, 64), (20, 140, 2048)])  # unsplit, and slices of k
+def test_dense_mm_nonfinite(lbq, dev, t, m, n, k):
+    # an infinity gives the infinities and NaN of the f32 product, nowhere else
+    rng = np.random.default_rng(11)
+    w = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1, 5], x[2, 9], x[4, 60], x[4, 61] = np.inf, np.nan, np.inf, -np.inf
+    x[6, 3] = 3e38
+    w[7, 20], w[9, 5], w[11, 30] = np.inf, 0.0, np.nan
+    x[8, 20] = 0.0
+    qm, w = _weight(t, n, k, rng, dev, w)
+    y = qm.forward(to_dev(x, dev)).cpu().numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = (x[:, None, :].astype(np.float64) * w[None]).sum(2)
+        ref = np.where(np.abs(ref) > 3.4028235e38, np.copysign(np.inf, ref), ref)
+    fin = np.isfinite(ref)
+    assert np.array_equal(np.isnan(ref), np.isnan(y))
+    assert np.array_equal(ref[~fin & ~np.isnan(ref)], y[~fin & ~np.isnan(ref)])
+    for r in range(m):
+        c = fin[r]
+        if c.any():
+            assert np.linalg.norm(y[r][c] - ref[r][c]) <= _bound(t, k) * np.linalg.norm(ref[r][c])
+
+
+def test_dense_mm_streams_growth_and_capture(lbq, dev):
+    # the operand buffer: two streams in turn, a larger call while a captured graph
+    # uses the smaller buffer, and replays between eager calls
+    rng = np.random.default_rng(13)
+    qm, w = _weight(F16, 512, 1024, rng, dev)
+    big, wb = _weight(F16, 1024, 8192, rng, dev)
+    x = rng.standard_normal((48, 1024)).astype(np.float32)
+    xb = rng.standard_normal((600, 8192)).astype(np.float32)
+    xd, xbd = to_dev(x, dev), to_dev(xb, dev)
+    want, wantb = qm.forward(xd).cpu().numpy(), big.forward(xbd).cpu().numpy()
+    _assert_rows(want, x.astype(np.float64) @ w.T, _bound(F16, 1024))
+    _assert_rows(wantb, xb.astype(np.float64) @ wb.T, _bound(F16, 8192))
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    ys = []
+    torch.cuda.synchronize()
+    for i in range(6):
+        with torch.cuda.stream((s1, s2)[i % 2]):
+            ys.append((big.forward(xbd), wantb) if i % 3 == 0 else (qm.forward(xd), want))
+    torch.cuda.synchronize()
+    for y, ref in ys:
+        assert np.array_equal(y.cpu().numpy(), ref)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        yg = qm.forward(xd)
+    huge, wh = _weight(F16, 256, 16384, rng, dev)
+    xh = to_dev(rng.standard_normal((2000, 16384)).astype(np.float32), dev)
+    for _ in range(3):
+        huge.forward(xh)
+        yg.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(yg.cpu().numpy(), want)
+
+
+def test_dense_mm_noalloc_beyond_scratch(lbq, dev):
+    # operands beyond the fixed scratch: the f32 matrix cores, as accurate
+    from lightbulb_amd.quantized import context
+    rng = np.random.default_rng(17)
+    n, k, m = 64, 16384, 1100
+    qm, w = _weight(F16, n, k, rng, dev)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    xd, y = to_dev(x, dev), torch.empty(m, n, device=dev)
+    st = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    assert lbq.lbq_qmatmul_f32_noalloc(context(dev), qm._handle, xd.data_ptr(), m, y.data_ptr(), st) == 0
+    # k/2 sums of two products, one after the other
+    _assert_rows(y.cpu().numpy(), x.astype(np.float64) @ w.T, 2.0 ** -23 * (k / 2) ** 0.5)
