@@ -150,7 +150,11 @@ int lbq_weight_info(const lbq_weight *w, uint32_t *ggml_type, int64_t *n, int64_
  *   - m > 8 otherwise, for every quantised type when k % 256 == 0 (Q4_0, Q4_1,
  *     Q5_0, Q5_1, Q8_0, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K): MFMA on fp16 roundings of
  *     the same activation and weight values (about 4e-4 relative on a row);
- *   - m > 8 with k % 256 != 0: the integer GEMV over chunks of 8 rows.
+ *   - m > 8 with k % 256 != 0: integer block sums on the fp16 matrix cores (the
+ *     codes and scales exact in fp16, f32 combine; ~1e-7 relative), with operands
+ *     in the context's scratch; where that cannot be had (a graph capture that
+ *     would have to grow it, the allocation-free scratch exceeded) the integer
+ *     GEMV over chunks of 8 rows.
  * Where the matrix-core decode kernel (m = 2..64) splits a 32-row
  * tile between two workgroups, their halves are added into y with f32 atomic
  * adds when y is plain device memory (hipMalloc; checked once per allocation),

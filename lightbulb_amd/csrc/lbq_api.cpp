@@ -288,6 +288,28 @@ struct Scratch {
     }
 };
 
+// `bytes` of GEMM workspace for a path that has another to fall back on, or null: fixed
+// scratch that is too small, a stream under capture whose buffer would have to grow, or
+// no memory.  (The caller holds ctx->mu and has its activation scratch already.)
+uint8_t *optional_ws(Scratch &sc, size_t bytes, hipStream_t st) {
+    if (!bytes) return nullptr;
+    if (sc.fixed) {
+        if (sc.act_used + bytes > sc.fixed_bytes) return nullptr;
+    } else if (sc.ctx->ws_bytes < bytes) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
+    uint8_t *ws = nullptr;
+    if (sc.ws(bytes, &ws)) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return ws;
+}
+
 // Batch decode on the matrix cores for this weight and row count
 static bool uses_mx(const lbq_weight *w, int64_t m) { return m <= 64 && lbq::gemv_mx_serves(w->type, w->n, w->k, (int)m); }
 // ... with its two split halves added into y, which the quantisation launch zeroes
@@ -359,7 +381,7 @@ int run_dot(Scratch &sc, const lbq_weight *w, const lbq::ActView &av, int64_t m,
         e = lbq::launch_gemv(w->type, w->d_blocks, w->n, w->k, w->row_bytes, av, (int)m, d_y, st);
     } else {
         const size_t wsb = lbq::gemm_workspace_bytes(w->type, w->n, w->k, m);
-        uint8_t *ws = nullptr;
+        uint8_t *ws = optional_ws(sc, lbq::gemm_b32_workspace_bytes(w->type, w->n, w->k, m), st);
         if (wsb) {
             int s = sc.ws(wsb, &ws);
             if (s) return s;
@@ -451,6 +473,15 @@ int forward(lbq_ctx *ctx, const lbq_weight *w, const float *d_x, int64_t m, floa
                                         sc.counters(), st);
         if (e != hipSuccess) return hip_fail(e, "quantized matmul launch");
         return LBQ_OK;
+    }
+    if (m > 8 && lbq::gemm_b32_serves(w->type, w->k, m) && lbq::gemm_b32_quantises(d_x)) {
+        // k % 256 != 0: the operand pre-pass quantises x itself, where its workspace is to be had
+        uint8_t *ws = optional_ws(sc, lbq::gemm_b32_workspace_bytes(w->type, w->n, w->k, m), st);
+        if (ws) {
+            const lbq::ActView none{nullptr, nullptr, nullptr, w->k, L.nb};
+            hipError_t e = lbq::launch_gemm_b32(w->type, w->d_blocks, w->n, w->k, w->row_bytes, none, d_x, m, d_y, ws, st);
+            return e == hipSuccess ? LBQ_OK : hip_fail(e, "quantized matmul launch");
+        }
     }
     uint8_t *abuf = nullptr;
     int s = sc.act(L.total, &abuf);

@@ -270,6 +270,11 @@ __global__ __launch_bounds__(256) void k_split_sum(const float *__restrict__ par
     }
 }
 
+hipError_t launch_split_sum(const float *part, int S, int64_t count, float *y, hipStream_t st) {
+    k_split_sum<<<(unsigned)((count + 1023) / 1024), 256, 0, st>>>(part, S, count, y);
+    return hipGetLastError();
+}
+
 // The k-sliced layout's operand rows with Q8_K activations: one wave per (row m,
 // exponent group g of KS_BLOCKS blocks), 16 lanes per block.  Each block is
 // quantised as k_quant_f16 does (q8k_lane16) or read from Q8_K codes; the group's
@@ -605,9 +610,7 @@ hipError_t gemm_main(int type, const uint8_t *w, const int8_t *rexp, int64_t n, 
     default: return hipErrorInvalidValue;
     }
     if (e != hipSuccess || p.splits == 1 || cnt) return e;
-    const int64_t count = m * n;
-    k_split_sum<<<(unsigned)((count + 1023) / 1024), 256, 0, st>>>(part, p.splits, count, y);
-    return hipGetLastError();
+    return launch_split_sum(part, p.splits, m * n, y, st);
 }
 
 hipError_t launch_gemm(int type, const uint8_t *w, const int8_t *rexp, int64_t n, int64_t k, int64_t row_bytes,
@@ -620,8 +623,9 @@ hipError_t launch_gemm(int type, const uint8_t *w, const int8_t *rexp, int64_t n
         if (e != hipSuccess) return e;
         return gemm_main(type, w, rexp, n, k, row_bytes, m, y, ws, counters, nullptr, st);
     }
+    if (ws && gemm_b32_serves(type, k, m)) return launch_gemm_b32(type, w, n, k, row_bytes, act, x, m, y, ws, st);
     if (x) return hipErrorInvalidValue;  // the GEMV over row chunks takes quantised activations
-    // k % 256 != 0: the decode GEMV over row chunks of 8
+    // k % 256 != 0 without a workspace: the decode GEMV over row chunks of 8
     for (int64_t m0 = 0; m0 < m; m0 += 8) {
         const int mc = (int)(m - m0 < 8 ? m - m0 : 8);
         ActView a = act;

@@ -24,7 +24,7 @@ constexpr bool has_fast_gemv(int t) { return t == TYPE_Q4_K || t == TYPE_Q5_K ||
 // weight types the MFMA GEMM serves at m > 8: every quantised weight type
 constexpr bool has_mfma_gemm(int t) { return is_kquant(t) || is_legacy(t) || t == TYPE_Q8_0; }
 // ... at this k: the GEMM steps through k in 256-value super-blocks (32-value
-// types: 8 blocks); other k run the decode GEMV over row chunks of 8
+// types: 8 blocks); other k run the 32-value block kernel (lbq_gemm_b32.hip)
 constexpr bool gemm_serves(int t, int64_t k) { return has_mfma_gemm(t) && k % 256 == 0; }
 // types whose per-lane weight state (raw bytes + expanded operands) is large: one
 // workgroup per CU for the 32-row-tile kernels, no 128-row k_gemm tiles, one
@@ -214,6 +214,16 @@ bool gemm_quantises_in_kernel(int type, int64_t n, int64_t k, int64_t m, const f
 hipError_t launch_gemm(int type, const uint8_t *w, const int8_t *rexp, int64_t n, int64_t k, int64_t row_bytes,
                        const ActView &act, const float *x, int64_t m, float *y, void *ws, uint32_t *counters,
                        hipStream_t st);
+// The 32-value types at m > 8 with k % 256 != 0 (lbq_gemm_b32.hip), with
+// gemm_b32_workspace_bytes (else 0) bytes at ws: from f32 x where gemm_b32_quantises(x)
+// (act supplies k and the block count only), else (x == nullptr) from act's codes.
+bool gemm_b32_serves(int type, int64_t k, int64_t m);
+bool gemm_b32_quantises(const float *x);
+size_t gemm_b32_workspace_bytes(int type, int64_t n, int64_t k, int64_t m);
+hipError_t launch_gemm_b32(int type, const uint8_t *w, int64_t n, int64_t k, int64_t row_bytes, const ActView &act,
+                           const float *x, int64_t m, float *y, void *ws, hipStream_t st);
+// y[i] = sum over s < S of part[s][i] in slice order, count values
+hipError_t launch_split_sum(const float *part, int S, int64_t count, float *y, hipStream_t st);
 // Per-row operand exponents of a weight the MFMA GEMM serves (gemm_serves):
 // rexp[i] = e such that every value row i's blocks can produce is below
 // 2^(15 + e), so the GEMM's fp16 weight operands, scaled by 2^-e, stay clear
