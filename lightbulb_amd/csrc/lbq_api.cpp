@@ -87,7 +87,8 @@ Tuning tuning_from_env() {
     t.gemm_no_ks = getenv("LBQ_GEMM_NO_KS") != nullptr;
     t.gemm_no_tall = getenv("LBQ_GEMM_NO_TALL") != nullptr;
     t.gemm_ks = std::max(0, env_int("LBQ_GEMM_KS"));
-    if (const char *e = getenv("LBQ_GEMM_BIG")) t.gemm_big = e[0] == 't' ? 2 : 1;
+    if (const char *e = getenv("LBQ_GEMM_BIG")) t.gemm_big = e[0] == 's' ? 3 : e[0] == 't' ? 2 : 1;
+    t.gemm_pair_off = getenv("LBQ_GEMM_PAIR_OFF") != nullptr;
     t.gemm_splits = std::max(0, env_int("LBQ_GEMM_SPLITS"));
     if (const char *e = getenv("LBQ_GEMM_WIDE7")) t.gemm_wide7 = e[0] == '0' ? -1 : 1;
     t.gemm_split_launch = getenv("LBQ_GEMM_SPLIT_LAUNCH") != nullptr;
@@ -982,6 +983,28 @@ int gate_up_f32(lbq_ctx *ctx, const lbq_weight *w_gate, const lbq_weight *w_up, 
         if (e == hipSuccess)
             e = lbq::launch_gemv_mx_pair(w_gate->type, w_gate->d_blocks, w_up->d_blocks, w_gate->n, w_gate->k,
                                          w_gate->row_bytes, av, (int)m, d_out, st);
+        return e == hipSuccess ? LBQ_OK : hip_fail(e, "gate/up launch");
+    }
+    if (!nm && m > 64 && !lbq::is_dense(w_gate->type) && lbq::gemm_pair_serves(w_gate->type, w_gate->n, w_gate->k, m)) {
+        // one operand pre-pass, then both weights and the product in one launch
+        std::lock_guard<std::mutex> lock(ctx->mu);
+        int s = ensure_buffer(&ctx->ws, &ctx->ws_bytes,
+                              lbq::gemm_pair_workspace_bytes(w_gate->type, w_gate->n, w_gate->k, m), "GEMM workspace");
+        if (s) return s;
+        const int act_type = lbq::vec_dot_type(w_gate->type);
+        const ActLayout L = act_layout(act_type, m, w_gate->k);
+        lbq::ActView av{nullptr, nullptr, nullptr, w_gate->k, L.nb};
+        const bool fused = lbq::gemm_prepass_fuses_quant(w_gate->type, w_gate->k, d_x);
+        hipError_t e = hipSuccess;
+        if (!fused) {
+            if ((s = ensure_scratch(ctx, L.total))) return s;
+            av = view_of(ctx->scratch, L, w_gate->k);
+            e = quant_into(act_type, d_x, m, w_gate->k, av, st);
+        }
+        if (e == hipSuccess) e = lbq::gemm_prepass(w_gate->type, w_gate->k, av, fused ? d_x : nullptr, m, ctx->ws, st);
+        if (e == hipSuccess)
+            e = lbq::gemm_pair(w_gate->type, w_gate->d_blocks, w_gate->d_rexp, w_up->d_blocks, w_up->d_rexp, w_gate->n,
+                               w_gate->k, w_gate->row_bytes, m, d_out, ctx->ws, st);
         return e == hipSuccess ? LBQ_OK : hip_fail(e, "gate/up launch");
     }
     // otherwise gate and up through the grouped path into context memory, then

@@ -399,6 +399,14 @@ hipError_t launch_row_exponents(int type, const uint8_t *w, int64_t n, int64_t k
 namespace {
 
 
+// Whether the square tiles can run: from 256 rows.  (Q4_K up to 512 rows at larger k:
+// the pre-pass's rows then stay whole 128-row tiles, so that what fitted a fixed
+// scratch of 64 MB still does.)
+bool square_ok(int type, int64_t k, int64_t m) {
+    return gemm_square(type) && m >= 256 && k * 2 * XBM < (int64_t(1) << 31) && (m > 512 || k <= 24576) && !tuning().gemm_no_tall;
+}
+int square_tiles(int64_t n, int64_t m, int cols) { return (int)((m + XBM - 1) / XBM * ((n + cols - 1) / cols)); }
+
 // mt, rt and tile_rows depend on (type, k, m) only -- the pre-pass plans with n = 1
 Plan plan_for(int type, int64_t n, int64_t k, int64_t m) {
     Plan p;
@@ -478,6 +486,22 @@ Plan plan_for(int type, int64_t n, int64_t k, int64_t m) {
     }
     p.bps = (nb + s - 1) / s;
     p.splits = (nb + p.bps - 1) / p.bps;
+    // square tiles, k whole, where their rounds of the chip are the shorter ones: a
+    // square tile takes about 8.2 us per block of k with every CU busy, the wide and
+    // tall tiles of half its size 5.0 (Q4_K 14336x4096 M = 2048 / 4096 302 / 590 ->
+    // 261 / 545 us, Q8_0 8192^2 M = 2048 371 -> 329; with fewer tiles than half the
+    // CUs and k split they lose: 14336x4096 M = 512 76 -> 92)
+    if (square_ok(type, k, m) && (!tu.gemm_big || tu.gemm_big == 3)) {
+        const int64_t tiles = square_tiles(n, m, XBN), half = (int64_t)p.tiles_m * p.tiles_n * p.splits;
+        const int64_t rs = (tiles + slots - 1) / slots * nb * 82, rh = (half + slots - 1) / slots * p.bps * 50;
+        if (tu.gemm_big == 3 || (2 * tiles > slots && rs < rh)) {
+            p.mt = MT_SQ;
+            p.tiles_m = (int)((m + XBM - 1) / XBM);
+            p.tiles_n = (int)((n + XBN - 1) / XBN);
+            p.bps = nb;
+            p.splits = 1;
+        }
+    }
     return p;
 }
 
@@ -490,7 +514,8 @@ struct WsLayout {
 // exponents and the partials, for whole row tiles like the operand rows
 WsLayout ws_layout(int type, const Plan &p, int64_t n, int64_t k, int64_t m) {
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-    const size_t rows = (size_t)p.tiles_m * tile_rows(p);
+    // whole row tiles, of the square kernel too where a weight of the call may run it
+    const size_t rows = square_ok(type, k, m) ? (size_t)((m + XBM - 1) / XBM * XBM) : (size_t)p.tiles_m * tile_rows(p);
     WsLayout L;
     L.a_off = 0;
     L.e_off = L.a_off + up(rows * (size_t)k * sizeof(_Float16));  // whole row tiles
@@ -573,6 +598,53 @@ bool gemm_quantises_in_kernel(int type, int64_t n, int64_t k, int64_t m, const f
     return p.mt == MT_KS && p.tiles_n <= KS_FX_MAX_TILES && ks_fx_shape(p.bps, ks_fx_rows(m, p.rt));
 }
 
+namespace {
+hipError_t launch_any(int type, const Plan &p, const uint8_t *w, const int8_t *rexp, int64_t n, int64_t row_bytes,
+                      const _Float16 *a, const int *erow, const _Float16 *ofs, int64_t k, int64_t m, float *out,
+                      int64_t stride, uint32_t *cnt, float *y, const float *x, hipStream_t st) {
+    switch (type) {
+#define LBQ_GEMM_GO(T) case T: return launch_typed<T>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st);
+    LBQ_GEMM_GO(TYPE_Q4_K) LBQ_GEMM_GO(TYPE_Q5_K) LBQ_GEMM_GO(TYPE_Q6_K) LBQ_GEMM_GO(TYPE_Q8_0) LBQ_GEMM_GO(TYPE_Q4_0)
+    LBQ_GEMM_GO(TYPE_Q4_1) LBQ_GEMM_GO(TYPE_Q5_0) LBQ_GEMM_GO(TYPE_Q5_1) LBQ_GEMM_GO(TYPE_Q2_K) LBQ_GEMM_GO(TYPE_Q3_K)
+#undef LBQ_GEMM_GO
+    default: return hipErrorInvalidValue;
+    }
+}
+
+// a gate/up pair: square tiles of 128 columns of each weight, k whole
+Plan pair_plan(int64_t n, int64_t k, int64_t m) {
+    Plan p;
+    p.mt = MT_SQ;
+    p.tiles_m = (int)((m + XBM - 1) / XBM);
+    p.tiles_n = (int)((n + XBN / 2 - 1) / (XBN / 2));
+    p.bps = (int)(k / KB);
+    p.splits = 1;
+    return p;
+}
+}  // namespace
+
+bool gemm_pair_serves(int type, int64_t n, int64_t k, int64_t m) {
+    // where the tiles keep more than half the CUs busy; the product launch (three passes
+    // over m x n values) it saves is worth more than the rounds' rounding
+    return gemm_serves(type, k) && square_ok(type, k, m) && !tuning().gemm_pair_off && 2 * square_tiles(n, m, XBN / 2) > num_cus();
+}
+
+size_t gemm_pair_workspace_bytes(int type, int64_t n, int64_t k, int64_t m) {
+    return ws_layout(type, pair_plan(n, k, m), n, k, m).total;
+}
+
+hipError_t gemm_pair(int type, const uint8_t *w_gate, const int8_t *rexp_gate, const uint8_t *w_up, const int8_t *rexp_up,
+                     int64_t n, int64_t k, int64_t row_bytes, int64_t m, float *out, void *ws, hipStream_t st) {
+    if (!ws || !rexp_gate || !rexp_up || !gemm_pair_serves(type, n, k, m)) return hipErrorInvalidValue;
+    Plan p = pair_plan(n, k, m);
+    p.w2 = w_up;
+    p.rexp2 = rexp_up;
+    const WsLayout L = ws_layout(type, p, n, k, m);
+    uint8_t *base = static_cast<uint8_t *>(ws);
+    return launch_any(type, p, w_gate, rexp_gate, n, row_bytes, reinterpret_cast<const _Float16 *>(base + L.a_off),
+                      reinterpret_cast<const int *>(base + L.e_off), nullptr, k, m, out, 0, nullptr, out, nullptr, st);
+}
+
 hipError_t gemm_main(int type, const uint8_t *w, const int8_t *rexp, int64_t n, int64_t k, int64_t row_bytes, int64_t m,
                      float *y, void *ws, uint32_t *counters, const float *x, hipStream_t st) {
     if (!ws || !rexp || !gemm_serves(type, k)) return hipErrorInvalidValue;
@@ -595,20 +667,7 @@ hipError_t gemm_main(int type, const uint8_t *w, const int8_t *rexp, int64_t n, 
                      (int64_t)p.splits * m * n * 4 < ((int64_t)1 << 31))
                         ? counters
                         : nullptr;
-    hipError_t e;
-    switch (type) {
-    case TYPE_Q4_K: e = launch_typed<TYPE_Q4_K>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q5_K: e = launch_typed<TYPE_Q5_K>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q6_K: e = launch_typed<TYPE_Q6_K>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q8_0: e = launch_typed<TYPE_Q8_0>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q4_0: e = launch_typed<TYPE_Q4_0>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q4_1: e = launch_typed<TYPE_Q4_1>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q5_0: e = launch_typed<TYPE_Q5_0>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q5_1: e = launch_typed<TYPE_Q5_1>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q2_K: e = launch_typed<TYPE_Q2_K>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    case TYPE_Q3_K: e = launch_typed<TYPE_Q3_K>(p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st); break;
-    default: return hipErrorInvalidValue;
-    }
+    const hipError_t e = launch_any(type, p, w, rexp, n, row_bytes, a, erow, ofs, k, m, out, stride, cnt, y, x, st);
     if (e != hipSuccess || p.splits == 1 || cnt) return e;
     return launch_split_sum(part, p.splits, m * n, y, st);
 }

@@ -23,7 +23,8 @@
 // Kernels by m (plan_for): k_gemm_ks, k-sliced 32- or 64-row tiles, for m <= 32
 // (Q6_K: 64); k_gemm<MT>, 32*MT-row tiles, up to 127 rows (Q6_K: 64); k_gemm_w,
 // eight-wave 128 x 256 tiles, from 128 rows (Q6_K: 65) below 256 (Q4_K: up to
-// 512); k_gemm_t, 256 x 128 tiles, above.  Each has its own description below;
+// 512); k_gemm_t, 256 x 128 tiles, above; k_gemm_x, 256 x 256 tiles, from 256 rows
+// where such tiles fill the chip, and gate/up pairs.  Each has its own description below;
 // the work split of k_gemm<MT>, on which the others build, follows.
 //
 // Work split.  A 256-thread workgroup owns BM = 32*MT rows of y and BN = 256
@@ -507,6 +508,8 @@ struct GemmGrid {
     uint32_t *cnt;              // k-sliced split: per column tile, slices done (null: k_split_sum adds them)
     float *y;                   // ... and the output the last slice of a tile writes
     const float *x;             // k-sliced, Q8_K rows: f32 x [m][k] each workgroup quantises itself
+    const uint8_t *w2;          // square tiles: the up weight of a gate/up pair (null: one weight) ...
+    const int8_t *rexp2;        // ... and its row exponents
 };
 
 // whether a weight type adds an extra k-step per super-block (odw)
@@ -1138,6 +1141,196 @@ __global__ __launch_bounds__(64 * NW, 1) void k_gemm_w(const uint8_t *__restrict
 }
 
 // ---------------------------------------------------------------------------
+// Square tiles: workgroup tile 256 x 256, eight waves (two per SIMD) as 2 x 4, each
+// 128 rows x 64 columns (4 x 2 MFMA tiles).  Both operands come from LDS: a wave
+// reads 6 KB for its 8 MFMAs of a k-step where the tall and wide kernels, whose waves
+// dequantise their own 32 columns, read 8, and every dequantised operand feeds 256
+// rows at two waves per SIMD.
+// k advances in stages of 64 (four k-steps, a quarter of a block), two buffers of 32 KB
+// each for A and B.  A: 256 operand rows of 128 B by buffer loads to LDS, chunk c
+// (h, k-step) in slot c ^ ((row >> 1) & 7).  B: wave w dequantises columns
+// 32w..32w+31 of the next stage while the current one's MFMAs run, 16 dwords (four
+// operands) a lane, stored operand-major (1 KB per k-step and 32 columns: no bank
+// conflicts either way); a block's raw bytes are loaded a block ahead.
+// One barrier a stage, before its last k-step, when every wave has read all of the
+// stage's operands, has stored its part of the next stage's B and its A loads have
+// landed: behind it the A buffer is refilled and the next stage's first operands are
+// read under the last k-step's MFMAs.
+// Pair (gate/up): columns are taken 32 of gate and the same 32 of up in turn, so a wave
+// holds both for 32 outputs and writes silu(gate) * up: the two products never reach
+// memory.
+// Bound by the matrix cores' rate beside the rest (Q4_K 14336x4096 pair, M = 4096: 1040
+// us, 0.92 PFLOP/s; without the dequantisation's VALU 880, without the A loads 930, without
+// both and the B stores 770).  Four waves of 128 x 128 a workgroup, which read a third
+// less from LDS, took 1218 us: one wave a SIMD leaves its waits uncovered.
+// us per call, tall / wide tiles -> these: Q4_K 14336x4096 M = 2048 302 -> 262, Q5_K 322 ->
+// 280, Q6_K 375 -> 341, Q8_0 8192^2 371 -> 330; gate + up + product Q4_K M = 512 178 -> 133
+// (kernels), M = 4096 1373 -> 1043.
+// ---------------------------------------------------------------------------
+constexpr int XBM = 256, XBN = 256;
+constexpr int XBUF = 32768;  // a stage of A, of B
+
+template <int TYPE, bool PAIR>
+__global__ __launch_bounds__(512) void k_gemm_x(const uint8_t *__restrict__ W, int64_t N, int64_t row_bytes,
+                                                const _Float16 *__restrict__ A, const int *__restrict__ erow, int64_t K,
+                                                int64_t M, float *__restrict__ out, GemmGrid g) {
+    using B = GB<TYPE>;
+    static_assert(!gemm_offset_step(TYPE), "no extra k-step here");
+    __shared__ __align__(1024) uint8_t As0[XBUF], As1[XBUF], Bs0[XBUF], Bs1[XBUF];
+    __shared__ int Es[XBM];
+    const int G = (int)gridDim.x, L = (int)blockIdx.x;
+    const int T = (G & 7) == 0 ? (L & 7) * (G >> 3) + (L >> 3) : L;
+    const int tm = T % g.tiles_m, tn = (T / g.tiles_m) % g.tiles_n, z = T / (g.tiles_m * g.tiles_n);
+    const int nb = (int)(K / KB);
+    const int b0 = z * g.bps, b1 = min(nb, b0 + g.bps);
+    constexpr int CN = PAIR ? XBN / 2 : XBN;  // columns of one weight
+    const int64_t m0 = (int64_t)tm * XBM, n0 = (int64_t)tn * CN;
+
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5, lr = lane & 31;
+    const int wm = wave >> 2, wn = wave & 3;
+    // the columns this wave dequantises
+    const bool up = PAIR && (wave & 1);
+    const int64_t wr = min(n0 + 32 * (PAIR ? wave >> 1 : wave) + lr, N - 1);
+    const uint8_t *wrow = (up ? g.w2 : W) + wr * row_bytes;
+    const float wsc = __builtin_amdgcn_ldexpf(1.f, -(up ? g.rexp2 : g.rexp)[wr]);
+    if (t < XBM) Es[t] = erow[min(m0 + t, M - 1)];
+
+    const uint64_t abase = reinterpret_cast<uint64_t>(A + m0 * K);
+    const uint64_t abase_s = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)abase) |
+                             ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(abase >> 32)) << 32);
+    const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void *>(abase_s), (short)0, __builtin_amdgcn_readfirstlane((int)(XBM * K * 2)), 0x00020000);
+    // staging instruction j of wave w: rows 8 (w + 8 j) + l/8, slot l%8
+    const int ach = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
+    const uint32_t voff = (uint32_t)((lane >> 3) * (int)K * 2 + 256 * (ach >> 2) + 16 * (ach & 3));
+    const int ns = 4 * (b1 - b0);
+    auto a_dma = [&](int s, int buf, int j) __attribute__((always_inline)) {  // stage s of the slice; past it, zeros
+        const int rb = wave + 8 * j;
+        const int soff = (8 * rb * (int)K + (b0 + (s >> 2)) * KB) * 2 + 64 * (s & 3);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, (__attribute__((address_space(3))) void *)((buf ? As1 : As0) + 8 * rb * 128),
+                                                 16, s < ns ? voff : 0x80000000u, soff, 0, 0);
+    };
+    int oa[4], ob = wn * 2048 + lane * 16, ow = wave * 1024 + lane * 16;
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) {
+        oa[ks] = wm * 16384 + lr * 128 + 16 * ((4 * h + ks) ^ ((lr >> 1) & 7));
+        asm volatile("" : "+v"(oa[ks]));
+    }
+    asm volatile("" : "+v"(ob), "+v"(ow));
+
+    typename B::Raw raw;
+    typename B::Prep p;
+    auto w_load = [&](int b, int q) __attribute__((always_inline)) { B::load_part(wrow + (int64_t)b * B::BYTES, h, raw, q); };
+    auto w_prep = [&](int b) __attribute__((always_inline)) { gb_prep<TYPE>(raw, h, wrow + (int64_t)b * B::BYTES, wsc, p); };
+    uint32_t bw[4];
+    // dword d of k-step s of the block in p; the operand's last dword stores it
+    auto b_form = [&](int s, int d, int buf) __attribute__((always_inline)) {
+        bw[d] = B::dw(p, s, d);
+        if (d == 3)
+            *reinterpret_cast<uint4 *>((buf ? Bs1 : Bs0) + (ow + (s & 3) * 8192)) = make_uint4(bw[0], bw[1], bw[2], bw[3]);
+    };
+    floatx16 acc[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+    uint4 op[2][6];  // operands of this k-step and the next: two B, four A
+    auto read = [&](int buf, int ks, int r, int q) __attribute__((always_inline)) {
+        if (q < 2) op[r][q] = *reinterpret_cast<const uint4 *>((buf ? Bs1 : Bs0) + (ob + ks * 8192 + q * 1024));
+        else op[r][q] = *reinterpret_cast<const uint4 *>((buf ? As1 : As0) + (oa[ks] + (q - 2) * 4096));
+    };
+
+#pragma unroll
+    for (int j = 0; j < 4; j++) a_dma(0, 0, j);
+#pragma unroll
+    for (int j = 0; j < 4; j++) a_dma(1, 1, j);
+#pragma unroll
+    for (int q = 0; q < B::NL; q++) w_load(b0, q);
+    w_prep(b0);
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) b_form(s, d, 0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 6; q++) read(0, 0, 0, q);
+
+    auto stage = [&](int b, int q4) __attribute__((always_inline)) {  // stage q4 of block b
+        const int buf = q4 & 1, bn = min(b + 1, b1 - 1);
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            if (ks == 3) {
+                __builtin_amdgcn_s_waitcnt(0);
+                __syncthreads();
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int i = u >> 1, j = u & 1, r = ks & 1;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, op[r][2 + i]),
+                                                                   __builtin_bit_cast(half8, op[r][j]), acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int q = u * 6 / 8; q < (u + 1) * 6 / 8; q++) {
+                    if (ks < 3) read(buf, ks + 1, r ^ 1, q);
+                    else read(buf ^ 1, 0, r ^ 1, q);
+                }
+                if (ks < 3) {
+                    // the next stage's B: 16 dwords over these 24 MFMAs
+                    const int slot = 8 * ks + u;
+                    if (q4 == 3 && slot == 0) w_prep(bn);
+#pragma unroll
+                    for (int e = slot * 16 / 24; e < (slot + 1) * 16 / 24; e++) b_form(4 * ((q4 + 1) & 3) + (e >> 2), e & 3, buf ^ 1);
+                } else {
+                    if (u < 4) a_dma(4 * (b - b0) + q4 + 2, buf, u);
+                    // the next block's bytes, spread over the stages' last k-steps (behind the A loads)
+                    else if (q4 < 3)
+#pragma unroll
+                        for (int e = 4 * q4 + u - 4; e < B::NL; e += 12) w_load(bn, e);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    for (int b = b0; b < b1; b++) {
+        stage(b, 0);
+        stage(b, 1);
+        stage(b, 2);
+        stage(b, 3);
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // the loads past the slice
+
+    float *y = out + (int64_t)z * g.split_stride;
+    if constexpr (PAIR) {
+        const int64_t n = n0 + 32 * wn + lr, nc = min(n, N - 1);
+        const int eg = g.rexp[nc], eu = g.rexp2[nc];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int r = 128 * wm + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
+                const float a = __builtin_amdgcn_ldexpf(acc[i][0][v], Es[r] + eg), c = __builtin_amdgcn_ldexpf(acc[i][1][v], Es[r] + eu);
+                if (m0 + r < M && n < N) __builtin_nontemporal_store(a / (1.f + expf(-a)) * c, y + (m0 + r) * N + n);
+            }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int64_t n = n0 + 64 * wn + 32 * j + lr;
+            const int en = g.rexp[min(n, N - 1)];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const int r = 128 * wm + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
+                    if (m0 + r < M && n < N)
+                        __builtin_nontemporal_store(__builtin_amdgcn_ldexpf(acc[i][j][v], Es[r] + en), y + (m0 + r) * N + n);
+                }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // K-sliced tiles for m <= 32.  A workgroup owns 128 columns (32 per wave) and a
 // slice of S consecutive blocks of k that its four waves share.  The slice's
 // activation operands (16 KB per block, operand-major) go into LDS by buffer
@@ -1475,13 +1668,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ks(const uint8_t *W, int64_t N,
 struct Plan {
     int mt, tiles_m, tiles_n, splits, bps;  // bps: blocks of k per split
     int rt = 1;                             // k-sliced kernel: 32-row tiles per workgroup
+    const uint8_t *w2 = nullptr;            // square tiles: the up weight of a gate/up pair
+    const int8_t *rexp2 = nullptr;          // and its row exponents
 };
 
 // mt = 8 selects the tall kernel (256 x 128 tiles), MT_WIDE the wide one (128 x 256),
 // MT_WIDE7 the wide one with seven waves (128 x 224)
 constexpr int MT_WIDE = 16, MT_WIDE7 = 17, MT_KS = 32;  // MT_KS: the k-sliced kernel (m <= 64)
+constexpr int MT_SQ = 64;  // the square tiles (256 x 256)
 inline int tile_rows(const Plan &p) {
-    return p.mt == MT_KS ? 32 * p.rt : p.mt == 8 ? TBM : (p.mt == MT_WIDE || p.mt == MT_WIDE7) ? WBM : 32 * p.mt;
+    return p.mt == MT_KS ? 32 * p.rt : p.mt == 8 || p.mt == MT_SQ ? TBM : (p.mt == MT_WIDE || p.mt == MT_WIDE7) ? WBM : 32 * p.mt;
 }
 // the pre-pass layout: 32-row tiles of operand-major rows, or 0 (row-major)
 inline int operand_major(const Plan &p) { return p.mt == MT_KS ? p.rt : 0; }
@@ -1489,7 +1685,7 @@ template <int TYPE>
 hipError_t launch_typed(const Plan &p, const uint8_t *w, const int8_t *rexp, int64_t n, int64_t row_bytes,
                         const _Float16 *a, const int *erow, const _Float16 *ofs, int64_t k, int64_t m, float *out,
                         int64_t split_stride, uint32_t *cnt, float *y, const float *x, hipStream_t st) {
-    const GemmGrid g{p.tiles_m, p.tiles_n, p.bps, split_stride, p.splits, rexp, ofs, cnt, y, x};
+    const GemmGrid g{p.tiles_m, p.tiles_n, p.bps, split_stride, p.splits, rexp, ofs, cnt, y, x, p.w2, p.rexp2};
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits));
     if constexpr (ks_group_exponents<TYPE>()) {
         if (x) {  // k-sliced, quantising x in the kernel (ks_fx_shape slices)
@@ -1521,6 +1717,14 @@ hipError_t launch_typed(const Plan &p, const uint8_t *w, const int8_t *rexp, int
         default: k_gemm_ks<TYPE, 4, 1><<<grid, 256, 0, st>>>(w, n, row_bytes, a, erow, k, m, out, g); break;
         }
         return hipGetLastError();
+    }
+    if (p.mt == MT_SQ) {
+        if constexpr (gemm_square(TYPE)) {
+            if (p.w2) k_gemm_x<TYPE, true><<<grid, 512, 0, st>>>(w, n, row_bytes, a, erow, k, m, out, g);
+            else k_gemm_x<TYPE, false><<<grid, 512, 0, st>>>(w, n, row_bytes, a, erow, k, m, out, g);
+            return hipGetLastError();
+        }
+        return hipErrorInvalidValue;
     }
     switch (p.mt) {
     case 8: k_gemm_t<TYPE><<<grid, 256, 0, st>>>(w, n, row_bytes, a, erow, k, m, out, g); break;

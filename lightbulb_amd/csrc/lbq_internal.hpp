@@ -35,6 +35,8 @@ constexpr bool gemm_offset_step(int t) { return t == TYPE_Q4_1 || t == TYPE_Q5_1
 constexpr bool gemm_heavy(int t) {
     return t == TYPE_Q6_K || t == TYPE_Q8_0 || t == TYPE_Q3_K || t == TYPE_Q5_0 || t == TYPE_Q5_1;
 }
+// types the square-tile kernel serves
+constexpr bool gemm_square(int t) { return has_mfma_gemm(t) && !gemm_offset_step(t); }
 // activation type of QMatMul's vec_dot for a weight type (candle GgmlType::VecDotType)
 constexpr int vec_dot_type(int t) {
     return is_kquant(t) ? TYPE_Q8_K : (t == TYPE_Q4_1 || t == TYPE_Q5_1) ? TYPE_Q8_1 : TYPE_Q8_0;
@@ -47,7 +49,7 @@ struct ActView;
 // the same result; only the kernel shape changes.  Zero / false: the measured
 // default plan.
 //   LBQ_GEMM_KS64, LBQ_GEMM_NO_KS, LBQ_GEMM_KS=<blocks>, LBQ_GEMM_NO_TALL,
-//   LBQ_GEMM_BIG=wide|tall, LBQ_GEMM_SPLITS=<n>,
+//   LBQ_GEMM_BIG=wide|tall|square, LBQ_GEMM_SPLITS=<n>, LBQ_GEMM_PAIR_OFF,
 //   LBQ_GEMM_WIDE7=0|1                              batched GEMM plan
 //   LBQ_GEMV1_NOFUSE, LBQ_GEMV1_CFG=<ppb>,<rpw>, LBQ_GEMV1_WPC=<waves per CU>,
 //   LBQ_GEMV1_WPG=<waves per workgroup>, LBQ_GEMV="rpw,it,wpc,fused",
@@ -58,7 +60,8 @@ struct ActView;
 struct Tuning {
     bool gemm_ks64 = false, gemm_no_ks = false, gemm_no_tall = false;
     int gemm_ks = 0;      // k-sliced tiles: blocks per slice (0: planned)
-    int gemm_big = 0;     // 1: wide tiles, 2: tall tiles (0: planned)
+    int gemm_big = 0;     // 1: wide tiles, 2: tall tiles, 3: square tiles (0: planned)
+    bool gemm_pair_off = false;  // gate/up pairs on the square tiles as two GEMMs and a product launch
     int gemm_splits = 0;  // split-k count (0: planned)
     int gemm_wide7 = 0;   // seven-wave wide tiles: 1 always where n allows, -1 never (0: planned)
     bool gemm_split_launch = false;  // k-sliced slices added by the separate launch, never in the kernel
@@ -208,6 +211,13 @@ hipError_t gemm_prepass(int type, int64_t k, const ActView &act, const float *x,
 // no pre-pass then), or nullptr for the operands gemm_prepass left in ws.
 hipError_t gemm_main(int type, const uint8_t *w, const int8_t *rexp, int64_t n, int64_t k, int64_t row_bytes, int64_t m,
                      float *y, void *ws, uint32_t *counters, const float *x, hipStream_t st);
+// A gate/up pair after gemm_prepass (the same operand rows as each weight's own GEMM) in
+// one launch: out = silu(x . gate) * (x . up), the two products never in memory.
+// gemm_pair_workspace_bytes at ws.
+bool gemm_pair_serves(int type, int64_t n, int64_t k, int64_t m);
+size_t gemm_pair_workspace_bytes(int type, int64_t n, int64_t k, int64_t m);
+hipError_t gemm_pair(int type, const uint8_t *w_gate, const int8_t *rexp_gate, const uint8_t *w_up, const int8_t *rexp_up,
+                     int64_t n, int64_t k, int64_t row_bytes, int64_t m, float *out, void *ws, hipStream_t st);
 // whether the GEMM for (type, n, k, m) quantises f32 x itself (the k-sliced
 // kernel with Q8_K activations, on slices whose x fits its registers)
 bool gemm_quantises_in_kernel(int type, int64_t n, int64_t k, int64_t m, const float *x);
