@@ -859,7 +859,7 @@ int group_f32(lbq_ctx *ctx, const lbq_weight *const *ws, int count, const float 
     bool all_mx = true;  // every weight on the integer matrix-core kernel: x quantised once below
     for (int i = 0; i < count; i++) all_mx = all_mx && uses_mx(ws[i], m);
     if (m > 8 && !all_mx && lbq::gemm_serves(w0->type, w0->k)) {
-        if (nm) return fail(LBQ_ERR_INVALID_ARG, "internal: the fused norm needs pre-quantised activations");
+        // (nm: every weight on the GEMM after one pre-pass, which normalises x: rmsnorm_fuses)
         // batched: one operand pre-pass (quantising x itself when it can) shared
         // by every weight's GEMM; weights on the integer matrix-core kernel share
         // one Q8_K quantisation of x and run after the GEMMs (their split partials
@@ -891,7 +891,7 @@ int group_f32(lbq_ctx *ctx, const lbq_weight *const *ws, int count, const float 
             // every GEMM weight's k-sliced kernel quantises x itself
         } else if (fused_prepass) {
             const lbq::ActView none{nullptr, nullptr, nullptr, w0->k, L.nb};
-            e = lbq::gemm_prepass(w0->type, w0->k, none, d_x, m, ctx->ws, st);
+            e = lbq::gemm_prepass(w0->type, w0->k, none, d_x, m, ctx->ws, st, nm ? nm->w : nullptr, nm ? nm->eps : 0.f);
         } else {
             e = quant_into(act_type, d_x, m, w0->k, av, st, &zl);
             quantised = true;
@@ -985,7 +985,7 @@ int gate_up_f32(lbq_ctx *ctx, const lbq_weight *w_gate, const lbq_weight *w_up, 
                                          w_gate->row_bytes, av, (int)m, d_out, st);
         return e == hipSuccess ? LBQ_OK : hip_fail(e, "gate/up launch");
     }
-    if (!nm && m > 64 && !lbq::is_dense(w_gate->type) && lbq::gemm_pair_serves(w_gate->type, w_gate->n, w_gate->k, m)) {
+    if (m > 64 && !lbq::is_dense(w_gate->type) && lbq::gemm_pair_serves(w_gate->type, w_gate->n, w_gate->k, m)) {
         // one operand pre-pass, then both weights and the product in one launch
         std::lock_guard<std::mutex> lock(ctx->mu);
         int s = ensure_buffer(&ctx->ws, &ctx->ws_bytes,
@@ -1001,7 +1001,9 @@ int gate_up_f32(lbq_ctx *ctx, const lbq_weight *w_gate, const lbq_weight *w_up, 
             av = view_of(ctx->scratch, L, w_gate->k);
             e = quant_into(act_type, d_x, m, w_gate->k, av, st);
         }
-        if (e == hipSuccess) e = lbq::gemm_prepass(w_gate->type, w_gate->k, av, fused ? d_x : nullptr, m, ctx->ws, st);
+        if (e == hipSuccess)
+            e = lbq::gemm_prepass(w_gate->type, w_gate->k, av, fused ? d_x : nullptr, m, ctx->ws, st, nm ? nm->w : nullptr,
+                                  nm ? nm->eps : 0.f);
         if (e == hipSuccess)
             e = lbq::gemm_pair(w_gate->type, w_gate->d_blocks, w_gate->d_rexp, w_up->d_blocks, w_up->d_rexp, w_gate->n,
                                w_gate->k, w_gate->row_bytes, m, d_out, ctx->ws, st);
@@ -1057,20 +1059,23 @@ int norm_into_tmp(lbq_ctx *ctx, const float *d_x, const float *d_w, float eps, i
     return e == hipSuccess ? LBQ_OK : hip_fail(e, "rmsnorm launch");
 }
 
-// Whether the RMS norm can run in the Q8_K quantisation launch (launch_rmsnorm_q8k)
-// instead of a launch of its own: Q8_K activations, k up to 64 blocks, 16-byte
-// aligned x and norm weight, and every weight on a path that reads pre-quantised
-// activations (m <= 8, or the integer matrix-core kernel) -- not the fp16 GEMM's
-// pre-pass or in-kernel quantisation, which read f32 x.
+// Whether the RMS norm can run in the launch that quantises x instead of one of its
+// own: every weight reads pre-quantised Q8_K activations (m <= 8, or the integer
+// matrix-core kernel; launch_rmsnorm_q8k: k up to 64 blocks, 16-byte aligned x and norm
+// weight), or every weight runs the fp16 GEMM after a pre-pass by rows.
 bool rmsnorm_fuses(const lbq_weight *const *ws, int count, const float *d_x, const float *d_w, int64_t m) {
     const lbq_weight *w0 = ws[0];
-    if (lbq::is_dense(w0->type) || lbq::vec_dot_type(w0->type) != lbq::TYPE_Q8_K) return false;
-    if (w0->k % 256 || w0->k / 256 > 64) return false;
-    if ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_w)) & 15u) return false;
-    if (m <= 8) return true;
-    for (int i = 0; i < count; i++)
-        if (!uses_mx(ws[i], m)) return false;
-    return true;
+    if (lbq::is_dense(w0->type)) return false;
+    bool any_mx = false, all_mx = true;
+    for (int i = 0; i < count; i++) {
+        const bool mx = uses_mx(ws[i], m);
+        any_mx = any_mx || mx;
+        all_mx = all_mx && mx;
+    }
+    if (lbq::vec_dot_type(w0->type) == lbq::TYPE_Q8_K && (m <= 8 || all_mx))
+        return w0->k % 256 == 0 && w0->k / 256 <= 64 &&
+               !((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_w)) & 15u);
+    return !any_mx && lbq::gemm_prepass_fuses_norm(w0->type, w0->k, m, d_x, d_w);
 }
 }  // namespace
 

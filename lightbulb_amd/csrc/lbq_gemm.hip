@@ -87,15 +87,43 @@ __global__ __launch_bounds__(T) void k_act_f16(ActView act, int64_t M, _Float16 
     }
 }
 
+// 16 consecutive values at a 16-byte aligned address
+__device__ __forceinline__ void load16(const float *p, float v[16]) {
+    const float4 *s = reinterpret_cast<const float4 *>(p);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float4 f = s[i];
+        v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
+    }
+}
+
+// sqrt(sum / K + eps) of the workgroup's T threads' shares of a sum of squares
+template <int T>
+__device__ __forceinline__ float row_rms(float ss, int t, int64_t K, float eps) {
+    __shared__ float red[T / 64];
+    ss = row_sum_f32(ss);
+    ss = __int_as_float(rl(__float_as_uint(ss), 0)) + __int_as_float(rl(__float_as_uint(ss), 16)) +
+         __int_as_float(rl(__float_as_uint(ss), 32)) + __int_as_float(rl(__float_as_uint(ss), 48));
+    if ((t & 63) == 0) red[t >> 6] = ss;
+    __syncthreads();
+    float sum = red[0];
+#pragma unroll
+    for (int w = 1; w < T / 64; w++) sum += red[w];
+    return sqrtf(sum / (float)K + eps);
+}
+
 // The same operand rows straight from f32 x (k <= 16384): the workgroup
 // quantises its row to Q8_K in registers (q8k_lane16, as the standalone
 // quantiser), shares the block scales through LDS for the row exponent, and
 // converts with the same arithmetic as k_act_f16 -- one launch instead of two,
 // bit-identical operands.  P: passes of T / 16 blocks, the fewest covering the
 // row (every load of a pass is issued, so no more passes than the row needs).
-template <int T, int P>
-__global__ __launch_bounds__(T) void k_quant_f16(const float *__restrict__ x, int64_t K, _Float16 *__restrict__ A,
-                                                 int *__restrict__ erow, int opmajor) {
+// NORM: candle's RmsNorm (f32, weight nw) of the row first, so that the normalised row
+// never reaches memory (k_rmsnorm and this took 14.3 + 5.1 us at 512x4096, 45 + 19 us at
+// 4096x4096; together 6.2 and 28).
+template <int T, int P, bool NORM>
+__global__ __launch_bounds__(T) void k_quant_f16(const float *__restrict__ x, const float *__restrict__ nw, float eps,
+                                                 int64_t K, _Float16 *__restrict__ A, int *__restrict__ erow, int opmajor) {
     constexpr int BPP = T / 16, MAXP = P;  // passes of BPP blocks, 64 blocks at most
     static_assert(BPP * P <= 64 && P >= 1, "at most 64 blocks per row");
     __shared__ float wmax[T / 64];
@@ -113,6 +141,23 @@ __global__ __launch_bounds__(T) void k_quant_f16(const float *__restrict__ x, in
             const float4 f = src[i];
             v[j][4 * i] = f.x; v[j][4 * i + 1] = f.y; v[j][4 * i + 2] = f.z; v[j][4 * i + 3] = f.w;
         }
+    }
+    if constexpr (NORM) {
+        float al[MAXP][16];
+#pragma unroll
+        for (int j = 0; j < MAXP; j++)
+            load16(nw + (int64_t)min(BPP * j + (t >> 4), nbx - 1) * KB + 16 * sub, al[j]);
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < MAXP; j++)
+            if (BPP * j + (t >> 4) < nbx)  // clamped duplicates do not count
+#pragma unroll
+                for (int i = 0; i < 16; i++) ss += v[j][i] * v[j][i];
+        const float rms = row_rms<T>(ss, t, K, eps);
+#pragma unroll
+        for (int j = 0; j < MAXP; j++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[j][i] = v[j][i] / rms * al[j][i];
     }
     uint4 codes[MAXP];
     float dj[MAXP];
@@ -163,11 +208,15 @@ __global__ __launch_bounds__(T) void k_quant_f16(const float *__restrict__ x, in
 // k_act_f16's arithmetic -- bit-identical operands, one launch.
 // With ofs (Q4_1 / Q5_1 weights: candle's BlockQ8_1::from_float codes are these
 // Q8_0 codes), also the extra k-step's operands of k_act_f16, from the block sum
-// s = f16(f16(sum of codes) * d) the reference stores.
-template <int T>
-__global__ __launch_bounds__(T) void k_quant_f16_q80(const float *__restrict__ x, int64_t K, _Float16 *__restrict__ A,
-                                                     int *__restrict__ erow, int opmajor, _Float16 *__restrict__ ofs) {
-    constexpr int BPP = T / 2, MAXP = 512 / BPP;  // passes of BPP blocks, 512 blocks at most
+// s = f16(f16(sum of codes) * d) the reference stores.  P: passes of T / 2 blocks, the
+// fewest of 1, 2 and 4 covering the row (333 x 4096: 5.4 us with four, 5.1 with one).
+// NORM as k_quant_f16.
+template <int T, int P, bool NORM>
+__global__ __launch_bounds__(T) void k_quant_f16_q80(const float *__restrict__ x, const float *__restrict__ nw, float eps,
+                                                     int64_t K, _Float16 *__restrict__ A, int *__restrict__ erow, int opmajor,
+                                                     _Float16 *__restrict__ ofs) {
+    constexpr int BPP = T / 2, MAXP = P;  // 512 blocks at most
+    static_assert(BPP * P <= 512 && P >= 1, "at most 512 blocks per row");
     __shared__ float wmax[T / 64];
     const int64_t m = blockIdx.x;
     const int t = threadIdx.x, sub = t & 1;
@@ -183,6 +232,23 @@ __global__ __launch_bounds__(T) void k_quant_f16_q80(const float *__restrict__ x
             const float4 f = src[i];
             v[j][4 * i] = f.x; v[j][4 * i + 1] = f.y; v[j][4 * i + 2] = f.z; v[j][4 * i + 3] = f.w;
         }
+    }
+    if constexpr (NORM) {
+        float al[MAXP][16];
+#pragma unroll
+        for (int j = 0; j < MAXP; j++)
+            load16(nw + (int64_t)min(BPP * j + (t >> 1), nbx - 1) * 32 + 16 * sub, al[j]);
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < MAXP; j++)
+            if (BPP * j + (t >> 1) < nbx)
+#pragma unroll
+                for (int i = 0; i < 16; i++) ss += v[j][i] * v[j][i];
+        const float rms = row_rms<T>(ss, t, K, eps);
+#pragma unroll
+        for (int j = 0; j < MAXP; j++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[j][i] = v[j][i] / rms * al[j][i];
     }
     uint32_t codes[MAXP][4];
     float dj[MAXP], sj[MAXP];
@@ -539,8 +605,16 @@ bool gemm_prepass_fuses_quant(int type, int64_t k, const float *x) {
     return x && gemm_serves(type, k) && k / KB <= 64 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
 }
 
-hipError_t gemm_prepass(int type, int64_t k, const ActView &act, const float *x, int64_t m, void *ws, hipStream_t st) {
+bool gemm_prepass_fuses_norm(int type, int64_t k, int64_t m, const float *x, const float *norm_w) {
+    // (the k-sliced layout's pre-pass works by groups of blocks, not by rows)
+    return norm_w && m > 8 && gemm_prepass_fuses_quant(type, k, x) && (reinterpret_cast<uintptr_t>(norm_w) & 15u) == 0 &&
+           !operand_major(plan_for(type, 1, k, m));
+}
+
+hipError_t gemm_prepass(int type, int64_t k, const ActView &act, const float *x, int64_t m, void *ws, hipStream_t st,
+                        const float *norm_w, float eps) {
     if (!ws || !gemm_serves(type, k)) return hipErrorInvalidValue;
+    if (norm_w && !gemm_prepass_fuses_norm(type, k, m, x, norm_w)) return hipErrorInvalidValue;
     const Plan p = plan_for(type, 1, k, m);  // the operand rows do not depend on n
     const WsLayout L = ws_layout(type, p, 1, k, m);
     uint8_t *base = static_cast<uint8_t *>(ws);
@@ -564,18 +638,36 @@ hipError_t gemm_prepass(int type, int64_t k, const ActView &act, const float *x,
     if (x) {
         if (!gemm_prepass_fuses_quant(type, k, x)) return hipErrorInvalidValue;
         if (vec_dot_type(type) != TYPE_Q8_K) {  // Q8_0 codes (the Q8_1 codes are the same)
-            if (wide_wg) k_quant_f16_q80<1024><<<(unsigned)m, 1024, 0, st>>>(x, k, a, erow, om, ofs);
-            else k_quant_f16_q80<256><<<(unsigned)m, 256, 0, st>>>(x, k, a, erow, om, ofs);
+            const int nbx = (int)(k / 32);
+            auto go = [&](auto kern, int T) { kern<<<(unsigned)m, T, 0, st>>>(x, norm_w, eps, k, a, erow, om, ofs); };
+            if (wide_wg) {
+                if (norm_w) go(k_quant_f16_q80<1024, 1, true>, 1024);
+                else go(k_quant_f16_q80<1024, 1, false>, 1024);
+            } else if (norm_w) {
+                if (nbx <= 128) go(k_quant_f16_q80<256, 1, true>, 256);
+                else if (nbx <= 256) go(k_quant_f16_q80<256, 2, true>, 256);
+                else go(k_quant_f16_q80<256, 4, true>, 256);
+            } else {
+                if (nbx <= 128) go(k_quant_f16_q80<256, 1, false>, 256);
+                else if (nbx <= 256) go(k_quant_f16_q80<256, 2, false>, 256);
+                else go(k_quant_f16_q80<256, 4, false>, 256);
+            }
         } else {
             const int nbx = (int)(k / KB);
+            auto go = [&](auto kern, int T) { kern<<<(unsigned)m, T, 0, st>>>(x, norm_w, eps, k, a, erow, om); };
             if (wide_wg) {
-                k_quant_f16<1024, 1><<<(unsigned)m, 1024, 0, st>>>(x, k, a, erow, om);
+                if (norm_w) go(k_quant_f16<1024, 1, true>, 1024);
+                else go(k_quant_f16<1024, 1, false>, 1024);
+            } else if (norm_w) {
+                if (nbx <= 16) go(k_quant_f16<256, 1, true>, 256);
+                else if (nbx <= 32) go(k_quant_f16<256, 2, true>, 256);
+                else if (nbx <= 48) go(k_quant_f16<256, 3, true>, 256);
+                else go(k_quant_f16<256, 4, true>, 256);
             } else {
-                auto go = [&](auto kern) { kern<<<(unsigned)m, 256, 0, st>>>(x, k, a, erow, om); };
-                if (nbx <= 16) go(k_quant_f16<256, 1>);
-                else if (nbx <= 32) go(k_quant_f16<256, 2>);
-                else if (nbx <= 48) go(k_quant_f16<256, 3>);
-                else go(k_quant_f16<256, 4>);
+                if (nbx <= 16) go(k_quant_f16<256, 1, false>, 256);
+                else if (nbx <= 32) go(k_quant_f16<256, 2, false>, 256);
+                else if (nbx <= 48) go(k_quant_f16<256, 3, false>, 256);
+                else go(k_quant_f16<256, 4, false>, 256);
             }
         }
     } else if (vec_dot_type(type) != TYPE_Q8_K) {  // Q8_0 / Q8_1 activations

@@ -202,7 +202,11 @@ hipError_t launch_silu_mul(const float *g, const float *u, int64_t count, float 
 // for (the operand rows do not depend on n).
 size_t gemm_workspace_bytes(int type, int64_t n, int64_t k, int64_t m);
 bool gemm_prepass_fuses_quant(int type, int64_t k, const float *x);
-hipError_t gemm_prepass(int type, int64_t k, const ActView &act, const float *x, int64_t m, void *ws, hipStream_t st);
+// whether gemm_prepass takes an RMS norm's weight too (norm_w, eps): x's rows are then
+// normalised (candle's RmsNorm) on the way
+bool gemm_prepass_fuses_norm(int type, int64_t k, int64_t m, const float *x, const float *norm_w);
+hipError_t gemm_prepass(int type, int64_t k, const ActView &act, const float *x, int64_t m, void *ws, hipStream_t st,
+                        const float *norm_w = nullptr, float eps = 0.f);
 // rexp: the weight's per-row operand exponents (launch_row_exponents).
 // counters: KS_COUNTERS zeroed words the k-sliced kernel uses to add its own
 // slices (the last workgroup of a column tile sums them and puts the word back
