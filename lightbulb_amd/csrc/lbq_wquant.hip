@@ -20,10 +20,17 @@ __device__ __forceinline__ int nearest_int(float fval) {
 
 __device__ __forceinline__ uint32_t f2h_bits(float f) { return __half_as_ushort(__float2half_rn(f)); }
 
-// ggml make_qkx2_quants(n = 32, weights, use_mad = false)
+// ggml make_qkx2_quants(n = 32, weights, use_mad = false).
+//
+// The search's loop is VALU bound (Q4_K 4096^2 217 -> 180 us, Q5_K and Q6_K alike; 24 instructions an element and
+// step with codes as integers, 17 as floats): for |v| < 2^22, v + 1.5 2^23 - 1.5 2^23 is
+// nearest_int(v) as a float, exactly, so rounding and clamping a code cost an add, a
+// subtraction and a median, and no conversions.  `finite`: no x of the wave is infinite
+// or NaN; a step whose iscale * (x - min) could leave that range in some lane (a
+// fitted min next to max) takes the integer codes.
 template <int NMAX>
 __device__ float make_qkx2_32(const float *x, const float *weights, uint8_t *L, float *the_min, float rmin,
-                              float rdelta, int nstep) {
+                              float rdelta, int nstep, bool finite) {
     float min = x[0], max = x[0];
     float sum_w = weights[0];
     float sum_x = sum_w * x[0];
@@ -44,28 +51,41 @@ __device__ float make_qkx2_32(const float *x, const float *weights, uint8_t *L, 
     }
     float iscale = (float)NMAX / (max - min);
     float scale = 1.f / iscale;
+    const float lo0 = min, hi0 = max;
+    // codes of all 32 for a scale; the lanes here are the wave's that have a search
+    auto codes = [&](float isc, float *l) __attribute__((always_inline)) {
+        const float spread = fmaxf(fabsf(hi0 - min), fabsf(lo0 - min));
+        if (finite && !__any(!(fabsf(isc) * spread < 4e6f))) {
+#pragma unroll
+            for (int i = 0; i < 32; ++i)
+                l[i] = __builtin_amdgcn_fmed3f((isc * (x[i] - min) + 12582912.f) - 12582912.f, 0.f, (float)NMAX);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 32; ++i) {
+                const int q = nearest_int(isc * (x[i] - min));
+                l[i] = (float)(q < 0 ? 0 : q > NMAX ? NMAX : q);
+            }
+        }
+    };
     float best_mad = 0;
+    float Lf[32], Laux[32];
+    codes(iscale, Lf);
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
-        const int l = nearest_int(iscale * (x[i] - min));
-        L[i] = (uint8_t)(l < 0 ? 0 : l > NMAX ? NMAX : l);
-        float diff = scale * (float)L[i] + min - x[i];
+        float diff = scale * Lf[i] + min - x[i];
         diff = diff * diff;
         best_mad += weights[i] * diff;
     }
     for (int is = 0; is <= nstep; ++is) {
         iscale = (rmin + rdelta * (float)is + (float)NMAX) / (max - min);
         float sum_l = 0, sum_l2 = 0, sum_xl = 0;
-        uint8_t Laux[32];
+        codes(iscale, Laux);
 #pragma unroll
         for (int i = 0; i < 32; ++i) {
-            int l = nearest_int(iscale * (x[i] - min));
-            l = l < 0 ? 0 : l > NMAX ? NMAX : l;
-            Laux[i] = (uint8_t)l;
-            const float w = weights[i];
-            sum_l += w * (float)l;
-            sum_l2 += w * (float)l * (float)l;
-            sum_xl += w * (float)l * x[i];
+            const float wl = weights[i] * Laux[i];
+            sum_l += wl;
+            sum_l2 += wl * Laux[i];
+            sum_xl += wl * x[i];
         }
         const float D = sum_w * sum_l2 - sum_l * sum_l;
         if (D > 0) {
@@ -78,19 +98,21 @@ __device__ float make_qkx2_32(const float *x, const float *weights, uint8_t *L, 
             float mad = 0;
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
-                float diff = this_scale * (float)Laux[i] + this_min - x[i];
+                float diff = this_scale * Laux[i] + this_min - x[i];
                 diff = diff * diff;
                 mad += weights[i] * diff;
             }
             if (mad < best_mad) {
 #pragma unroll
-                for (int i = 0; i < 32; ++i) L[i] = Laux[i];
+                for (int i = 0; i < 32; ++i) Lf[i] = Laux[i];
                 best_mad = mad;
                 scale = this_scale;
                 min = this_min;
             }
         }
     }
+#pragma unroll
+    for (int i = 0; i < 32; ++i) L[i] = (uint8_t)Lf[i];
     *the_min = -min;
     return scale;
 }
@@ -98,7 +120,7 @@ __device__ float make_qkx2_32(const float *x, const float *weights, uint8_t *L, 
 // Q4_K (NMAX 15) / Q5_K (NMAX 31): 8 lanes per super-block, lane j owns sub-block j.
 template <int NMAX>
 __global__ __launch_bounds__(256) void k_quant_w_k45(const float *__restrict__ w, int64_t nblocks,
-                                                     uint8_t *__restrict__ out) {
+                                                     uint8_t *__restrict__ out, bool vec) {
     constexpr int TS = NMAX == 15 ? 144 : 176;
     __shared__ uint8_t Ls[32][QK_K];
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -107,9 +129,22 @@ __global__ __launch_bounds__(256) void k_quant_w_k45(const float *__restrict__ w
     const bool ok = blk < nblocks;
     float x[32], weights[32];
     uint8_t L[32];
+    // (lanes past the last block work on the first one and store nothing)
     const float *src = w + (ok ? blk : 0) * QK_K + 32 * j;
+    if (vec) {
 #pragma unroll
-    for (int l = 0; l < 32; ++l) x[l] = ok ? src[l] : 0.f;
+        for (int l = 0; l < 8; ++l) {
+            const float4 f = reinterpret_cast<const float4 *>(src)[l];
+            x[4 * l] = f.x; x[4 * l + 1] = f.y; x[4 * l + 2] = f.z; x[4 * l + 3] = f.w;
+        }
+    } else {
+#pragma unroll
+        for (int l = 0; l < 32; ++l) x[l] = src[l];
+    }
+    bool finite = true;
+#pragma unroll
+    for (int l = 0; l < 32; ++l) finite = finite && fabsf(x[l]) <= 3.4028234664e38f;
+    finite = __all(finite);
     float sum_x2 = 0;
 #pragma unroll
     for (int l = 0; l < 32; ++l) sum_x2 += x[l] * x[l];
@@ -117,8 +152,8 @@ __global__ __launch_bounds__(256) void k_quant_w_k45(const float *__restrict__ w
 #pragma unroll
     for (int l = 0; l < 32; ++l) weights[l] = av_x + fabsf(x[l]);
     float mn;
-    const float sc = NMAX == 15 ? make_qkx2_32<15>(x, weights, L, &mn, -1.f, 0.1f, 20)
-                                : make_qkx2_32<31>(x, weights, L, &mn, -0.5f, 0.1f, 15);
+    const float sc = NMAX == 15 ? make_qkx2_32<15>(x, weights, L, &mn, -1.f, 0.1f, 20, finite)
+                                : make_qkx2_32<31>(x, weights, L, &mn, -0.5f, 0.1f, 15, finite);
     // max over the 8 sub-blocks (ggml: strict > from 0)
     float max_scale = sc > 0.f ? sc : 0.f, max_min = mn > 0.f ? mn : 0.f;
 #pragma unroll
@@ -188,6 +223,7 @@ __global__ __launch_bounds__(256) void k_quant_w_k45(const float *__restrict__ w
 }
 
 // ggml make_qx_quants(n = 16, nmax = 32, rmse_type = 1, qw = NULL)
+template <bool FLOATS>
 __device__ float make_qx_16(const float *x, uint8_t *L) {
     constexpr int nmax = 32;
     float max = 0, amax = 0;
@@ -204,16 +240,24 @@ __device__ float make_qx_16(const float *x, uint8_t *L) {
         for (int i = 0; i < 16; ++i) L[i] = 0;
         return 0.f;
     }
+    // codes as floats (as make_qkx2_32): |iscale * x| is at most nmax + 0.9 where every x
+    // is finite and max at least 1e-15
+    auto code = [&](float v) __attribute__((always_inline)) -> float {
+        if constexpr (FLOATS) return __builtin_amdgcn_fmed3f((v + 12582912.f) - 12582912.f, -(float)nmax, (float)(nmax - 1));
+        const int l = nearest_int(v);
+        return (float)(l < -nmax ? -nmax : l > nmax - 1 ? nmax - 1 : l);
+    };
     float iscale = -(float)nmax / max;
     float sumlx = 0, suml2 = 0;
+    float Lf[16], wx[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        int l = nearest_int(iscale * x[i]);
-        l = l < -nmax ? -nmax : l > nmax - 1 ? nmax - 1 : l;
-        L[i] = (uint8_t)(l + nmax);
+        const float l = code(iscale * x[i]);
+        Lf[i] = l;
         const float w = x[i] * x[i];
-        sumlx += w * x[i] * (float)l;
-        suml2 += w * (float)l * (float)l;
+        wx[i] = w * x[i];
+        sumlx += wx[i] * l;
+        suml2 += w * l * l;
     }
     float scale = suml2 != 0.f ? sumlx / suml2 : 0.0f;
     float best = scale * sumlx;
@@ -221,31 +265,30 @@ __device__ float make_qx_16(const float *x, uint8_t *L) {
         if (is == 0) continue;
         iscale = -((float)nmax + 0.1f * (float)is) / max;
         sumlx = suml2 = 0;
+        float Laux[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            int l = nearest_int(iscale * x[i]);
-            l = l < -nmax ? -nmax : l > nmax - 1 ? nmax - 1 : l;
+            const float l = code(iscale * x[i]);
+            Laux[i] = l;
             const float w = x[i] * x[i];
-            sumlx += w * x[i] * (float)l;
-            suml2 += w * (float)l * (float)l;
+            sumlx += wx[i] * l;
+            suml2 += w * l * l;
         }
         if (suml2 > 0 && sumlx * sumlx > best * suml2) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                int l = nearest_int(iscale * x[i]);
-                l = l < -nmax ? -nmax : l > nmax - 1 ? nmax - 1 : l;
-                L[i] = (uint8_t)(nmax + l);
-            }
+            for (int i = 0; i < 16; ++i) Lf[i] = Laux[i];
             scale = sumlx / suml2;
             best = scale * sumlx;
         }
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) L[i] = (uint8_t)((int)Lf[i] + nmax);
     return scale;
 }
 
 // Q6_K: 16 lanes per super-block, lane t owns values 16t..16t+15.
 __global__ __launch_bounds__(256) void k_quant_w_q6k(const float *__restrict__ w, int64_t nblocks,
-                                                     uint8_t *__restrict__ out) {
+                                                     uint8_t *__restrict__ out, bool vec) {
     __shared__ uint8_t Ls[16][QK_K];
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t blk = t >> 4;
@@ -254,9 +297,21 @@ __global__ __launch_bounds__(256) void k_quant_w_q6k(const float *__restrict__ w
     float x[16];
     uint8_t L[16];
     const float *src = w + (ok ? blk : 0) * QK_K + 16 * ib;
+    // (lanes past the last block work on the first one and store nothing)
+    if (vec) {
 #pragma unroll
-    for (int l = 0; l < 16; ++l) x[l] = ok ? src[l] : 0.f;
-    const float scale = make_qx_16(x, L);
+        for (int l = 0; l < 4; ++l) {
+            const float4 f = reinterpret_cast<const float4 *>(src)[l];
+            x[4 * l] = f.x; x[4 * l + 1] = f.y; x[4 * l + 2] = f.z; x[4 * l + 3] = f.w;
+        }
+    } else {
+#pragma unroll
+        for (int l = 0; l < 16; ++l) x[l] = src[l];
+    }
+    bool finite = true;
+#pragma unroll
+    for (int l = 0; l < 16; ++l) finite = finite && fabsf(x[l]) <= 3.4028234664e38f;
+    const float scale = __all(finite) ? make_qx_16<true>(x, L) : make_qx_16<false>(x, L);
     // first sub-block of largest |scale| (ggml: strict > from 0)
     float ba = (scale == scale) ? fabsf(scale) : -1.f, bs = scale;
     int bi = ib;
@@ -396,21 +451,22 @@ __global__ __launch_bounds__(256) void k_quant_w_legacy(const float *__restrict_
 }
 
 hipError_t launch_quant_weights(int type, const float *w, int64_t nelem, uint8_t *out, hipStream_t st) {
+    const bool vec = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
     switch (type) {
     case TYPE_Q8_0: return launch_quant_act(TYPE_Q8_0, w, 1, nelem, nullptr, nullptr, nullptr, nullptr, out, st);
     case TYPE_Q4_K: {
         const int64_t nb = nelem / QK_K;
-        k_quant_w_k45<15><<<dim3((unsigned)((nb * 8 + 255) / 256)), 256, 0, st>>>(w, nb, out);
+        k_quant_w_k45<15><<<dim3((unsigned)((nb * 8 + 255) / 256)), 256, 0, st>>>(w, nb, out, vec);
         break;
     }
     case TYPE_Q5_K: {
         const int64_t nb = nelem / QK_K;
-        k_quant_w_k45<31><<<dim3((unsigned)((nb * 8 + 255) / 256)), 256, 0, st>>>(w, nb, out);
+        k_quant_w_k45<31><<<dim3((unsigned)((nb * 8 + 255) / 256)), 256, 0, st>>>(w, nb, out, vec);
         break;
     }
     case TYPE_Q6_K: {
         const int64_t nb = nelem / QK_K;
-        k_quant_w_q6k<<<dim3((unsigned)((nb * 16 + 255) / 256)), 256, 0, st>>>(w, nb, out);
+        k_quant_w_q6k<<<dim3((unsigned)((nb * 16 + 255) / 256)), 256, 0, st>>>(w, nb, out, vec);
         break;
     }
     case TYPE_Q4_0: case TYPE_Q4_1: case TYPE_Q5_0: case TYPE_Q5_1: {
