@@ -264,6 +264,9 @@ int lbq_dequantize_blocks_f32(uint32_t ggml_type, const void *d_blocks, int64_t 
  * k must be a multiple of 16; d_out 16-byte aligned. */
 int lbq_embedding_f32(lbq_ctx *ctx, const lbq_weight *w, const int32_t *d_ids, int64_t count, float *d_out,
                       void *stream);
+/* The same for int64 ids (8-byte aligned), as a tensor library holds them. */
+int lbq_embedding_i64_f32(lbq_ctx *ctx, const lbq_weight *w, const int64_t *d_ids, int64_t count, float *d_out,
+                          void *stream);
 
 /* Quantise activations x[m][k] to GGUF blocks of `act_type` (LBQ_TYPE_Q8_K:
  * 292-byte blocks; LBQ_TYPE_Q8_0: 34-byte blocks; LBQ_TYPE_Q8_1: 36-byte

@@ -1255,22 +1255,33 @@ int lbq_dequantize_blocks_f32(uint32_t type, const void *d_blocks, int64_t nelem
     return LBQ_OK;
 }
 
-int lbq_embedding_f32(lbq_ctx *ctx, const lbq_weight *w, const int32_t *d_ids, int64_t count, float *d_out,
-                      void *stream) {
+namespace {
+int embedding(lbq_ctx *ctx, const lbq_weight *w, const void *d_ids, bool i64, int64_t count, float *d_out, void *stream) {
     if (!ctx || !w) return fail(LBQ_ERR_INVALID_ARG, "null argument to lbq_embedding_f32");
     if (count < 0) return fail(LBQ_ERR_INVALID_ARG, "count = %lld is negative", (long long)count);
     if (w->k % 16) return fail(LBQ_ERR_SHAPE, "k = %lld is not a multiple of 16", (long long)w->k);
     if (count == 0) return LBQ_OK;
     if (!d_ids || !d_out) return fail(LBQ_ERR_INVALID_ARG, "null ids or output pointer");
-    if ((reinterpret_cast<uintptr_t>(d_ids) & 3u) || (reinterpret_cast<uintptr_t>(d_out) & 15u))
-        return fail(LBQ_ERR_INVALID_ARG, "ids must be 4-byte and the output 16-byte aligned");
+    if ((reinterpret_cast<uintptr_t>(d_ids) & (i64 ? 7u : 3u)) || (reinterpret_cast<uintptr_t>(d_out) & 15u))
+        return fail(LBQ_ERR_INVALID_ARG, "ids must be %d-byte and the output 16-byte aligned", i64 ? 8 : 4);
     if (count > ((int64_t)1 << 40) / w->k) return fail(LBQ_ERR_LIMIT, "count = %lld exceeds the supported maximum", (long long)count);
     DeviceGuard g(ctx->device);
     if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
     lbq::TuningScope tsc(&ctx->tune);
-    hipError_t e = lbq::launch_embedding(w->type, w->d_blocks, w->n, w->k, w->row_bytes, d_ids, count, d_out,
+    hipError_t e = lbq::launch_embedding(w->type, w->d_blocks, w->n, w->k, w->row_bytes, d_ids, i64, count, d_out,
                                          static_cast<hipStream_t>(stream));
     return e == hipSuccess ? LBQ_OK : hip_fail(e, "embedding launch");
+}
+}  // namespace
+
+int lbq_embedding_f32(lbq_ctx *ctx, const lbq_weight *w, const int32_t *d_ids, int64_t count, float *d_out,
+                      void *stream) {
+    return embedding(ctx, w, d_ids, false, count, d_out, stream);
+}
+
+int lbq_embedding_i64_f32(lbq_ctx *ctx, const lbq_weight *w, const int64_t *d_ids, int64_t count, float *d_out,
+                          void *stream) {
+    return embedding(ctx, w, d_ids, true, count, d_out, stream);
 }
 
 int lbq_quantize_act(uint32_t act_type, const float *d_x, int64_t m, int64_t k, void *d_out_blocks, void *stream) {

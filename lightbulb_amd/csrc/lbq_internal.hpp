@@ -132,7 +132,8 @@ hipError_t launch_dequant(int type, const uint8_t *blocks, int64_t nelem, float 
 
 // y[i][:] = the dequantised row ids[i] of an [n][k] weight (rows row_bytes apart),
 // i < count; an id outside [0, n) gives a row of NaN.  k is a multiple of 16.
-hipError_t launch_embedding(int type, const uint8_t *w, int64_t n, int64_t k, int64_t row_bytes, const int32_t *ids,
+// ids: int64 or int32
+hipError_t launch_embedding(int type, const uint8_t *w, int64_t n, int64_t k, int64_t row_bytes, const void *ids, bool i64,
                             int64_t count, float *y, hipStream_t st);
 
 // y[m][n] += nothing: y is overwritten.  Weight rows are row_bytes apart.

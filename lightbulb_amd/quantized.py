@@ -467,10 +467,12 @@ class QEmbedding:
 
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
         dev = self._qmatmul.qtensor().data.device
-        flat = ids.reshape(-1).to(device=dev, dtype=torch.int32).contiguous()
+        # int64 ids as they are, without a launch to narrow them
+        i64 = ids.dtype == torch.int64
+        flat = ids.reshape(-1).to(device=dev, dtype=torch.int64 if i64 else torch.int32).contiguous()
         out = torch.empty(flat.numel(), self.hidden_size, dtype=torch.float32, device=dev)
-        _lib.check(_lib.lib().lbq_embedding_f32(context(dev), self._qmatmul._handle, flat.data_ptr(), flat.numel(),
-                                                out.data_ptr(), _stream(dev)))
+        lookup = _lib.lib().lbq_embedding_i64_f32 if i64 else _lib.lib().lbq_embedding_f32
+        _lib.check(lookup(context(dev), self._qmatmul._handle, flat.data_ptr(), flat.numel(), out.data_ptr(), _stream(dev)))
         return out.reshape(*ids.shape, self.hidden_size)
 
     __call__ = forward
