@@ -142,8 +142,16 @@ def context(device="cuda") -> int:
         return _ctxs[idx]
 
 
-def _stream(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(torch.device(device)).cuda_stream)
+#: the current stream's handle by device index, without building a Stream object (0.06
+#: against 2.0 us: a quarter of a decode projection's call, Q4_K 1024x4096 m = 1 7.8 -> 5.9 us)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(device) -> int:
+    dev = device if isinstance(device, torch.device) else torch.device(device)
+    if _raw_stream is None or dev.index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(dev.index)
 
 
 # ---------------------------------------------------------------------------
@@ -233,21 +241,21 @@ class QMatMul:
 
     def forward(self, xs: torch.Tensor) -> torch.Tensor:
         n, k = self._qt.shape()
+        shape, dev = xs.shape, xs.device
         if xs.dtype != torch.float32:
             raise ValueError(f"the lhs for quantized matmul must be f32, got {xs.dtype}")
-        if xs.dim() < 2:
-            raise ValueError(f"input tensor has only one dimension {tuple(xs.shape)}")
-        if xs.shape[-1] != k:
-            raise ValueError(f"input tensor {tuple(xs.shape)} incompatible with {(n, k)}")
+        if len(shape) < 2:
+            raise ValueError(f"input tensor has only one dimension {tuple(shape)}")
+        if shape[-1] != k:
+            raise ValueError(f"input tensor {tuple(shape)} incompatible with {(n, k)}")
         if not xs.is_contiguous():
-            raise ValueError(f"input tensor is not contiguous {tuple(xs.shape)}")
-        if xs.device != self._qt.data.device:
-            raise ValueError(f"input on {xs.device}, weights on {self._qt.data.device}")
+            raise ValueError(f"input tensor is not contiguous {tuple(shape)}")
+        if dev != self._qt.data.device:
+            raise ValueError(f"input on {dev}, weights on {self._qt.data.device}")
         m = xs.numel() // k
-        y = torch.empty(*xs.shape[:-1], n, dtype=torch.float32, device=xs.device)
+        y = torch.empty((*shape[:-1], n), dtype=torch.float32, device=dev)
         if m:
-            _lib.check(_lib.lib().lbq_qmatmul_f32(self._ctx, self._handle, xs.data_ptr(), m, y.data_ptr(),
-                                                  _stream(xs.device)))
+            _lib.check(_lib.lib().lbq_qmatmul_f32(self._ctx, self._handle, xs.data_ptr(), m, y.data_ptr(), _stream(dev)))
         return y
 
     __call__ = forward
@@ -472,7 +480,7 @@ class QEmbedding:
         flat = ids.reshape(-1).to(device=dev, dtype=torch.int64 if i64 else torch.int32).contiguous()
         out = torch.empty(flat.numel(), self.hidden_size, dtype=torch.float32, device=dev)
         lookup = _lib.lib().lbq_embedding_i64_f32 if i64 else _lib.lib().lbq_embedding_f32
-        _lib.check(lookup(context(dev), self._qmatmul._handle, flat.data_ptr(), flat.numel(), out.data_ptr(), _stream(dev)))
+        _lib.check(lookup(self._qmatmul._ctx, self._qmatmul._handle, flat.data_ptr(), flat.numel(), out.data_ptr(), _stream(dev)))
         return out.reshape(*ids.shape, self.hidden_size)
 
     __call__ = forward
