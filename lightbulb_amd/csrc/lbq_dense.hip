@@ -10,11 +10,12 @@
 //           the next unit's 16-byte loads in flight, x staged in LDS, f32 FMA
 //           against up to 8 activation rows, DPP row sums -- HBM-bound like the
 //           quantised decode GEMV;
-//   m > 8   k_dense_mm (F16 / BF16): x as two fp16 or three bf16 operands that add
-//           up to it, on the 16-bit matrix cores with f32 accumulation;
-//           k_dense_gemm (F32 weights, and calls without a workspace): 64 x 128
+//   m > 8   k_dense_mm (F16 / BF16), k_dense_mm32 (F32): x, and an F32 weight, as two
+//           fp16 or three bf16 operands that add up to it, on the 16-bit matrix
+//           cores with f32 accumulation;
+//           k_dense_gemm (calls without a workspace): 64 x 128
 //           output tiles on v_mfma_f32_32x32x2_f32, operands staged through LDS.
-// Every product is formed at f32 precision or better and summed in f32; only the
+// Every product is formed at f32 precision and summed in f32; only the
 // summation order differs from candle's, so results agree to f32 rounding (~1e-6
 // relative on a row).
 #include <algorithm>
@@ -331,10 +332,15 @@ __device__ __forceinline__ floatx16 dense_mfma(uint4 a, uint4 b, floatx16 c) {
 
 __device__ __forceinline__ bool dense_finite(float v) { return fabsf(v) <= 3.4028234664e38f; }  // false for NaN
 
-template <bool BF>
+template <bool BF, bool W32 = false>
 __device__ __attribute__((noinline)) float dense_dot(const float *x, const uint8_t *w, int64_t K) {
     float s = 0.f;
-    for (int64_t i = 0; i < K; i++) s = fmaf(w16<BF>(reinterpret_cast<const unsigned short *>(w)[i]), x[i], s);
+    for (int64_t i = 0; i < K; i++) {
+        float v;
+        if constexpr (W32) v = reinterpret_cast<const float *>(w)[i];
+        else v = w16<BF>(reinterpret_cast<const unsigned short *>(w)[i]);
+        s = fmaf(v, x[i], s);
+    }
     return s;
 }
 
@@ -549,8 +555,193 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
         }
 }
 
-// y[m][n] = 2^e_m * (sum over the slices, in order); blockIdx.y: row m
-template <bool BF>
+// ---------------------------------------------------------------------------
+// m > 8 with F32 weights: x as the three bf16 pieces of k_dense_pieces<true> (their sum
+// is x), and each weight as three bf16 pieces that a wave forms in registers from the
+// f32 value in LDS: hi = bf16(w), mid = bf16(w - hi), lo = w - hi - mid, rounded to
+// nearest, again exact.  Six of the nine products, all exact in the accumulator:
+// hi hi, hi mid, mid hi, mid mid, hi lo, lo hi.  The three left out are at most 2^-23
+// of |x w| together and of either sign.  As k_dense_mm otherwise (tiles, two LDS buffers
+// filled by loads to LDS, one barrier a stage), with stages of 32 values of k: a
+// weight row is 128 B of a stage, its 16-byte chunk c in slot c ^ ((r >> 1) & 7); a
+// piece's row is 64 B, two rows a line, chunk c of row r in slot
+// (c ^ ((r >> 2) & 3)) + 4 (r & 1), so operand reads meet no bank twice.
+// The split costs about 5.5 vector instructions a weight: under the MFMAs of TM tiles
+// (192 TM clocks against 176), so waves take two row tiles where m has them.
+// Bound by the matrix cores from M = 200 (1.0-1.3 PFLOP/s of operand products), by the
+// weights' bytes and the launches below.  Against k_dense_gemm, us per call and relative
+// error against 64 bits:
+//   4096^2       M = 9 / 64 / 512  232 / 243 / 246 -> 19.5 / 30.3 / 105, 1.1e-6 -> 2.7e-7 / 2.7e-7 / 7.1e-7
+//   1024 x 4096  M = 32            234 -> 15.5
+//   8192^2       M = 512 / 2048    773 / 3021 -> 359 / 1309, 1.6e-6 -> 1.4e-6
+//   512^2        M = 9 / 128       31.7 / 35.1 -> 12.2 / 17.2
+// ---------------------------------------------------------------------------
+constexpr int DK32 = 32;  // values of k per stage
+
+typedef __bf16 dbf2 __attribute__((ext_vector_type(2)));
+typedef float dfl2 __attribute__((ext_vector_type(2)));
+
+// two values' bf16 (nearest), value 0 in the low half; v keeps what is left
+__device__ __forceinline__ uint32_t dense_split2(float &v0, float &v1) {
+    const dfl2 f = {v0, v1};
+    const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, dbf2));
+    v0 -= __uint_as_float(b << 16);
+    v1 -= __uint_as_float(b & 0xffff0000u);
+    return b;
+}
+
+template <int WM, int WN, int TM, int TN>
+__global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__restrict__ W, int64_t N, int64_t K,
+                                                             const unsigned short *__restrict__ A,
+                                                             const float *__restrict__ x, int64_t M,
+                                                             float *__restrict__ out, DenseGrid g) {
+    constexpr int NW = WM * WN, BM = 32 * WM * TM, BN = 32 * WN * TN;
+    constexpr int RA = 3 * BM / 16, RB = BN / 8;  // staging instructions (1 KB): all pieces, the weights
+    static_assert(RB % NW == 0 && NW % 2 == 0 && (BM / 16) % 2 == 0, "whole staging instructions per wave");
+    constexpr int RAW = (RA + NW - 1) / NW;  // per wave, the last ones of them without a piece
+    __shared__ __align__(1024) uint8_t As0[1024 * RAW * NW], As1[1024 * RAW * NW];
+    __shared__ __align__(1024) uint8_t Bs0[BN * 128], Bs1[BN * 128];
+    // tiles that share weight rows on one XCD
+    const int G = (int)gridDim.x, L = (int)blockIdx.x;
+    const int T = (G & 7) == 0 ? (L & 7) * (G >> 3) + (L >> 3) : L;
+    const int tm = T % g.tiles_m, tn = (T / g.tiles_m) % g.tiles_n, z = T / (g.tiles_m * g.tiles_n);
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+    const int s0 = z * g.sps, ns = min(g.sps, (int)(g.Kp / DK32) - s0);  // ns >= 1
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5, lr = lane & 31;
+    const int wm = wave / WN, wn = wave % WN;
+
+    // the piece that this wave's instruction j = 0, 1, 2 loads from
+    const int64_t ps = g.rows * g.Kp;
+    const unsigned short *Am = A + m0 * g.Kp;
+    const __amdgpu_buffer_rsrc_t a0 = dense_rsrc(Am + wave / (BM / 16) * ps, BM * g.Kp * 2);
+    const __amdgpu_buffer_rsrc_t a1 = dense_rsrc(Am + (wave + NW) / (BM / 16) * ps, BM * g.Kp * 2);
+    const __amdgpu_buffer_rsrc_t a2 = dense_rsrc(Am + (wave + 2 * NW) / (BM / 16) * ps, BM * g.Kp * 2);
+    const __amdgpu_buffer_rsrc_t br = dense_rsrc(W + n0 * K * 4, (N - n0 < BN ? N - n0 : BN) * K * 4);
+    // pieces: lane l of an instruction fills line l/8 of 8, slot l%8: row 2 (l/8) + slot/4 of 16
+    const uint32_t va = (uint32_t)((2 * (lane >> 3) + ((lane >> 2) & 1)) * (int)g.Kp * 2 + 16 * ((lane & 3) ^ (lane >> 4)));
+    // weights: row l/8, slot l%8 of 8 rows whose number / 8 has the wave's parity
+    const int ch = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
+    const uint32_t vb = (uint32_t)((lane >> 3) * (int)K * 4 + 16 * ch);
+    auto stage_in = [&](int s, int buf) __attribute__((always_inline)) {
+        const int k0 = (s0 + s) * DK32;
+        const uint32_t v0 = s < ns ? va : 0x80000000u;
+#pragma unroll
+        for (int j = 0; j < RAW; j++) {
+            const int q = wave + NW * j;  // instruction q: piece q / (BM / 16), its rows 16 (q % (BM / 16)) on
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                j == 0 ? a0 : j == 1 ? a1 : a2, (__attribute__((address_space(3))) void *)((buf ? As1 : As0) + 1024 * q), 16,
+                RA % NW == 0 || q < RA ? v0 : 0x80000000u, (16 * (q % (BM / 16)) * (int)g.Kp + k0) * 2, 0, 0);
+        }
+        const uint32_t v1 = s < ns && k0 + 4 * ch < (int)K ? vb : 0x80000000u;  // past K: zero
+#pragma unroll
+        for (int j = 0; j < RB / NW; j++) {
+            const int rb = wave + NW * j;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                br, (__attribute__((address_space(3))) void *)((buf ? Bs1 : Bs0) + 1024 * rb), 16, v1,
+                (8 * rb * (int)K + k0) * 4, 0, 0);
+        }
+    };
+    int oa[2], ob[4];  // byte offsets of a lane's operands: pieces of k-step ks; weight chunks
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+        oa[ks] = wm * TM * 2048 + (lr >> 1) * 128 + 16 * (((2 * ks + h) ^ ((lr >> 2) & 3)) + 4 * (lr & 1));
+        asm volatile("" : "+v"(oa[ks]));
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            ob[2 * ks + i] = wn * TN * 4096 + lr * 128 + 16 * ((4 * ks + 2 * h + i) ^ ((lr >> 1) & 7));
+            asm volatile("" : "+v"(ob[2 * ks + i]));
+        }
+    }
+
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+    // operands of this k-step and the next: x pieces, weight pieces; the next one's weights
+    constexpr int NA = 3 * TM, NB = 2 * TN, NM = 6 * TM * TN;
+    uint4 xa[2][NA], wb[2][TN][3], raw[NB];
+    auto read = [&](int buf, int ks, int r, int q) __attribute__((always_inline)) {
+        if (q < NB) raw[q] = *reinterpret_cast<const uint4 *>((buf ? Bs1 : Bs0) + (ob[2 * ks + (q & 1)] + (q >> 1) * 4096));
+        else
+            xa[r][q - NB] = *reinterpret_cast<const uint4 *>((buf ? As1 : As0) +
+                                                             (oa[ks] + (q - NB) / TM * (BM * 64) + (q - NB) % TM * 2048));
+    };
+    // pair c (two weights) of raw -> wb[r]
+    auto split = [&](int r, int c) __attribute__((always_inline)) {
+        const int j = c >> 2, e = c & 3;
+        const uint4 v = raw[2 * j + (e >> 1)];
+        float v0 = __uint_as_float(e & 1 ? v.z : v.x), v1 = __uint_as_float(e & 1 ? v.w : v.y);
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            const uint32_t b = dense_split2(v0, v1);
+            if (e == 0) wb[r][j][p].x = b;
+            else if (e == 1) wb[r][j][p].y = b;
+            else if (e == 2) wb[r][j][p].z = b;
+            else wb[r][j][p].w = b;
+        }
+    };
+    // the MFMAs of the k-step in xa[r], wb[r], each followed by its share of the next
+    // one's reads (first half) or splits (second half)
+    auto step = [&](int r, int buf, int ks) __attribute__((always_inline)) {
+        constexpr int H = NM / 2, PR[6] = {0, 0, 1, 1, 0, 2}, PW[6] = {0, 1, 0, 1, 2, 0};
+#pragma unroll
+        for (int u = 0; u < NM; u++) {
+            const int j = u % TN, i = u / TN % TM, p = u / TN / TM;
+            acc[i][j] = dense_mfma<true>(xa[r][PR[p] * TM + i], wb[r][j][PW[p]], acc[i][j]);
+            if (u < H) {
+#pragma unroll
+                for (int q = u * (NA + NB) / H; q < (u + 1) * (NA + NB) / H; q++) read(buf, ks, r ^ 1, q);
+            } else {
+#pragma unroll
+                for (int c = (u - H) * 4 * TN / (NM - H); c < (u - H + 1) * 4 * TN / (NM - H); c++) split(r ^ 1, c);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    stage_in(0, 0);
+    stage_in(1, 1);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NA + NB; q++) read(0, 0, 0, q);
+#pragma unroll
+    for (int c = 0; c < 4 * TN; c++) split(0, c);
+    auto stage = [&](int s, int buf) __attribute__((always_inline)) {
+        step(0, buf, 1);
+        __builtin_amdgcn_s_waitcnt(0);  // this wave's operands, and its loads of stage s + 1
+        __syncthreads();
+        stage_in(s + 2, buf);
+        __builtin_amdgcn_sched_barrier(0);
+        step(1, buf ^ 1, 0);
+    };
+    for (int s = 0; s < ns; s += 2) {  // an odd count ends with a stage of zeros
+        stage(s, 0);
+        stage(s + 1, 1);
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // the loads past the slice
+    // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
+    float *y = out + (int64_t)z * g.split_stride;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int64_t n = n0 + 32 * (wn * TN + j) + lr;
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int64_t m = m0 + 32 * (wm * TM + i) + 8 * (v >> 2) + 4 * h + (v & 3);
+                if (m >= M || n >= N) continue;
+                float r = acc[i][j][v];
+                if (g.split_stride == 0 && !dense_finite(r)) r = dense_dot<true, true>(x + m * K, W + n * K * 4, K);
+                y[m * N + n] = r;
+            }
+        }
+}
+
+// y[m][n] = 2^e_m * (sum over the slices, in order); blockIdx.y: row m.  BF: no exponent
+template <bool BF, bool W32 = false>
 __global__ __launch_bounds__(256) void k_dense_sum(const float *__restrict__ part, int S, int64_t M, int64_t N,
                                                    const int *__restrict__ erow, const float *__restrict__ x,
                                                    const uint8_t *__restrict__ W, int64_t K, float *__restrict__ y) {
@@ -578,7 +769,7 @@ __global__ __launch_bounds__(256) void k_dense_sum(const float *__restrict__ par
     for (int i = 0; i < 4; i++) {
         if (n + i >= N) break;
         float r = BF ? s[i] : __builtin_amdgcn_ldexpf(s[i], e);
-        if (!dense_finite(r)) r = dense_dot<BF>(x + m * K, W + (n + i) * K * 2, K);
+        if (!dense_finite(r)) r = dense_dot<BF, W32>(x + m * K, W + (n + i) * K * (W32 ? 4 : 2), K);
         y[m * N + n + i] = r;
     }
 }
@@ -589,24 +780,25 @@ struct DensePlan {
     DenseGrid g;
     size_t a_off, e_off, part_off, total;
 };
-// Tile by m (32, 64, 128 rows; 128 x 256 for F16 where such tiles fill the chip by
-// themselves), then k split until the resident workgroups (LDS: three of the 32-row
-// tiles a CU, two of the 64-row, one of the 128-row) are there, at least four
-// stages a slice.
+// Tile by m (32, 64, 128 rows; 128 x 256 for F16 and F32 where such tiles fill the chip
+// by themselves), then k split until the resident workgroups (LDS: three of the 32-row
+// tiles a CU, two of the 64-row, one of the 128-row) are there, at least 256 values of
+// k a slice.
 DensePlan dense_plan(int type, int64_t n, int64_t k, int64_t m) {
     DensePlan p;
-    const int P = type == TYPE_BF16 ? 3 : 2;
+    const int P = type == TYPE_F16 ? 2 : 3;
+    const bool w32 = type == TYPE_F32;
     p.bm = m <= 32 ? 32 : m <= 64 ? 64 : 128;
     p.bn = 128;
     const int64_t cus = num_cus();
-    if (p.bm == 128 && P == 2 && ((m + 127) / 128) * ((n + 255) / 256) * 4 >= 3 * cus) p.bn = 256;
+    if (p.bm == 128 && (P == 2 || w32) && ((m + 127) / 128) * ((n + 255) / 256) * 4 >= 3 * cus) p.bn = 256;
     p.g.tiles_m = (int)((m + p.bm - 1) / p.bm);
     p.g.tiles_n = (int)((n + p.bn - 1) / p.bn);
     p.g.rows = (int64_t)p.g.tiles_m * p.bm;
     p.g.Kp = (k + DK - 1) / DK * DK;
-    const int64_t ns = p.g.Kp / DK, tiles = (int64_t)p.g.tiles_m * p.g.tiles_n;
+    const int64_t ns = p.g.Kp / (w32 ? DK32 : DK), tiles = (int64_t)p.g.tiles_m * p.g.tiles_n;
     const int64_t slots = cus * (p.bm == 32 ? 3 : p.bm == 64 ? 2 : 1);
-    const int64_t s = std::max<int64_t>(1, std::min(slots / tiles, ns / 4));
+    const int64_t s = std::max<int64_t>(1, std::min(slots / tiles, ns / (w32 ? 8 : 4)));
     p.g.sps = (int)((ns + s - 1) / s);
     p.g.splits = (int)((ns + p.g.sps - 1) / p.g.sps);
     p.g.split_stride = p.g.splits > 1 ? m * n : 0;
@@ -620,8 +812,8 @@ DensePlan dense_plan(int type, int64_t n, int64_t k, int64_t m) {
 }  // namespace
 
 size_t dense_workspace_bytes(int type, int64_t n, int64_t k, int64_t m) {
-    // the pieces' buffer resources: 128 rows of k within 2^31 bytes
-    if ((type != TYPE_F16 && type != TYPE_BF16) || m <= 8 || k % 8 || k > (1 << 22) || m > 65535) return 0;
+    // the buffer resources: 128 rows of pieces, 256 of f32 weights within 2^31 bytes
+    if (m <= 8 || k % 8 || k > (type == TYPE_F32 ? 1 << 20 : 1 << 22) || m > 65535) return 0;
     return dense_plan(type, n, k, m).total;
 }
 
@@ -642,6 +834,23 @@ static hipError_t dense_pieces(int type, const uint8_t *w, int64_t n, int64_t k,
     if (p.g.splits > 1)
         k_dense_sum<BF><<<dim3((unsigned)((n + 1023) / 1024), (unsigned)m), 256, 0, st>>>(out, p.g.splits, m, n, e, x, w,
                                                                                         k, y);
+    return hipGetLastError();
+}
+
+static hipError_t dense_pieces32(const uint8_t *w, int64_t n, int64_t k, const float *x, int64_t m, float *y, uint8_t *ws,
+                                 hipStream_t st) {
+    const DensePlan p = dense_plan(TYPE_F32, n, k, m);
+    unsigned short *a = reinterpret_cast<unsigned short *>(ws + p.a_off);
+    float *out = p.g.splits > 1 ? reinterpret_cast<float *>(ws + p.part_off) : y;
+    k_dense_pieces<true><<<(unsigned)m, 256, 0, st>>>(x, k, p.g.Kp, p.g.rows, a, nullptr);
+    const unsigned grid = (unsigned)(p.g.tiles_m * p.g.tiles_n * p.g.splits);
+    if (p.bm == 32) k_dense_mm32<1, 4, 1, 1><<<grid, 256, 0, st>>>(w, n, k, a, x, m, out, p.g);
+    else if (p.bm == 64) k_dense_mm32<2, 4, 1, 1><<<grid, 512, 0, st>>>(w, n, k, a, x, m, out, p.g);
+    else if (p.bn == 128) k_dense_mm32<2, 4, 2, 1><<<grid, 512, 0, st>>>(w, n, k, a, x, m, out, p.g);
+    else k_dense_mm32<2, 4, 2, 2><<<grid, 512, 0, st>>>(w, n, k, a, x, m, out, p.g);
+    if (p.g.splits > 1)
+        k_dense_sum<true, true><<<dim3((unsigned)((n + 1023) / 1024), (unsigned)m), 256, 0, st>>>(out, p.g.splits, m, n,
+                                                                                                nullptr, x, w, k, y);
     return hipGetLastError();
 }
 
@@ -672,6 +881,8 @@ static hipError_t dense_typed(const uint8_t *w, int64_t n, int64_t k, const floa
 hipError_t launch_dense(int type, const uint8_t *w, int64_t n, int64_t k, const float *x, int64_t m, float *y,
                         void *ws, hipStream_t st) {
     if (k % 8 || m > 65535LL * DBM) return hipErrorInvalidValue;
+    if (ws && dense_workspace_bytes(type, n, k, m) && type == TYPE_F32)
+        return dense_pieces32(w, n, k, x, m, y, static_cast<uint8_t *>(ws), st);
     if (ws && dense_workspace_bytes(type, n, k, m))
         return type == TYPE_BF16 ? dense_pieces<true>(type, w, n, k, x, m, y, static_cast<uint8_t *>(ws), st)
                                  : dense_pieces<false>(type, w, n, k, x, m, y, static_cast<uint8_t *>(ws), st);

@@ -1,7 +1,8 @@
-"""Dense F16 / BF16 weights at m > 8: x as 16-bit operands that add up to it, on the
-matrix cores, against a float64 product.
+"""Dense F16 / BF16 / F32 weights at m > 8: x (and an F32 weight) as 16-bit operands that
+add up to it, on the matrix cores, against a float64 product.
 
-Bound: every product is exact in the f32 accumulator, so a row's relative L2 error is
+Bound: every product is exact in the f32 accumulator (of an F32 weight's, what is left
+out is below 2^-23 of it), so a row's relative L2 error is
 that of adding P k/16 partial sums one after the other, each rounded to half an ulp
 (2^-24) of the running sum: 2^-24 sqrt(P k / 16) for errors of independent sign, taken
 twice, and never below f32's own rounding of a handful of steps.
@@ -15,19 +16,19 @@ import torch
 from test_gpu_parity import to_dev
 
 pytestmark = pytest.mark.gpu
-F16, BF16 = 1, 30
+F32, F16, BF16 = 0, 1, 30
 
 
 def _weight(t, n, k, rng, dev, w=None):
     from lightbulb_amd.quantized import GgmlDType, QMatMul, QTensor
     w = torch.from_numpy((rng.standard_normal((n, k)) * 0.05).astype(np.float32) if w is None else w)
-    w = w.to(torch.float16 if t == F16 else torch.bfloat16)
+    w = w.to({F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[t])
     qm = QMatMul.from_qtensor(QTensor(w.reshape(-1).view(torch.uint8).to(dev), GgmlDType(t), (n, k)))
     return qm, w.to(torch.float64).numpy()
 
 
 def _bound(t, k):
-    return 2.0 ** -23 * max(4.0, ((3 if t == BF16 else 2) * k / 16) ** 0.5)
+    return 2.0 ** -23 * max(4.0, ({F32: 6, F16: 2, BF16: 3}[t] * k / 16) ** 0.5)
 
 
 def _assert_rows(y, ref, bound):
@@ -35,7 +36,7 @@ def _assert_rows(y, ref, bound):
     assert err.max() <= bound, (err.max(), bound)
 
 
-@pytest.mark.parametrize("t", [F16, BF16])
+@pytest.mark.parametrize("t", [F16, BF16, F32])
 # each row tile's edges (32, 64, 128 rows), column tiles of 128 and 256, k that is no
 # multiple of a stage (64) or of two, one stage, slices of k and none
 @pytest.mark.parametrize("m,n,k", [(9, 1, 8), (32, 130, 520), (33, 300, 4096), (64, 127, 72), (65, 257, 1000),
@@ -48,7 +49,7 @@ def test_dense_mm_shapes(lbq, dev, t, m, n, k):
     _assert_rows(qm.forward(to_dev(x, dev)).cpu().numpy(), x.astype(np.float64) @ w.T, _bound(t, k))
 
 
-@pytest.mark.parametrize("t", [F16, BF16])
+@pytest.mark.parametrize("t", [F16, BF16, F32])
 def test_dense_mm_range_and_alignment(lbq, dev, t):
     # rows of very different size, subnormal rows, zero rows; x only 4-byte aligned
     rng = np.random.default_rng(7)
@@ -64,7 +65,7 @@ def test_dense_mm_range_and_alignment(lbq, dev, t):
     assert not y[3].any()
 
 
-@pytest.mark.parametrize("t", [F16, BF16])
+@pytest.mark.parametrize("t", [F16, BF16, F32])
 @pytest.mark.parametrize("m,n,k", [(20, 140, 64), (20, 140, 2048)])  # unsplit, and slices of k
 def test_dense_mm_nonfinite(lbq, dev, t, m, n, k):
     # an infinity gives the infinities and NaN of the f32 product, nowhere else
@@ -89,18 +90,19 @@ def test_dense_mm_nonfinite(lbq, dev, t, m, n, k):
             assert np.linalg.norm(y[r][c] - ref[r][c]) <= _bound(t, k) * np.linalg.norm(ref[r][c])
 
 
-def test_dense_mm_streams_growth_and_capture(lbq, dev):
+@pytest.mark.parametrize("t", [F16, F32])
+def test_dense_mm_streams_growth_and_capture(lbq, dev, t):
     # the operand buffer: two streams in turn, a larger call while a captured graph
     # uses the smaller buffer, and replays between eager calls
     rng = np.random.default_rng(13)
-    qm, w = _weight(F16, 512, 1024, rng, dev)
-    big, wb = _weight(F16, 1024, 8192, rng, dev)
+    qm, w = _weight(t, 512, 1024, rng, dev)
+    big, wb = _weight(t, 1024, 8192, rng, dev)
     x = rng.standard_normal((48, 1024)).astype(np.float32)
     xb = rng.standard_normal((600, 8192)).astype(np.float32)
     xd, xbd = to_dev(x, dev), to_dev(xb, dev)
     want, wantb = qm.forward(xd).cpu().numpy(), big.forward(xbd).cpu().numpy()
-    _assert_rows(want, x.astype(np.float64) @ w.T, _bound(F16, 1024))
-    _assert_rows(wantb, xb.astype(np.float64) @ wb.T, _bound(F16, 8192))
+    _assert_rows(want, x.astype(np.float64) @ w.T, _bound(t, 1024))
+    _assert_rows(wantb, xb.astype(np.float64) @ wb.T, _bound(t, 8192))
     s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
     ys = []
     torch.cuda.synchronize()
@@ -113,7 +115,7 @@ def test_dense_mm_streams_growth_and_capture(lbq, dev):
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         yg = qm.forward(xd)
-    huge, wh = _weight(F16, 256, 16384, rng, dev)
+    huge, wh = _weight(t, 256, 16384, rng, dev)
     xh = to_dev(rng.standard_normal((2000, 16384)).astype(np.float32), dev)
     for _ in range(3):
         huge.forward(xh)
@@ -123,12 +125,13 @@ def test_dense_mm_streams_growth_and_capture(lbq, dev):
         assert np.array_equal(yg.cpu().numpy(), want)
 
 
-def test_dense_mm_noalloc_beyond_scratch(lbq, dev):
+@pytest.mark.parametrize("t", [F16, F32])
+def test_dense_mm_noalloc_beyond_scratch(lbq, dev, t):
     # operands beyond the fixed scratch: the f32 matrix cores, as accurate
     from lightbulb_amd.quantized import context
     rng = np.random.default_rng(17)
     n, k, m = 64, 16384, 1100
-    qm, w = _weight(F16, n, k, rng, dev)
+    qm, w = _weight(t, n, k, rng, dev)
     x = rng.standard_normal((m, k)).astype(np.float32)
     xd, y = to_dev(x, dev), torch.empty(m, n, device=dev)
     st = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
