@@ -530,6 +530,45 @@ constexpr int gemm_occupancy() {
 template <int TYPE, int MT>
 constexpr bool gemm_deep() { return TYPE == TYPE_Q4_K && MT == 1; }
 
+// Stores of one 32 x 32 MFMA tile: lane holds column n (its own), rows 8(v/4) + 4h + v%4
+// of the tile whose first row is y and of which `left` rows exist; val(v) is element v.
+// Nontemporal: a tile is written once, at the end, by every workgroup at about the same
+// time (Q4_K 14336x4096 M = 512 83.1 -> 80.5 us), and split partials too (cached, they
+// cost the split GEMMs at M = 100 about 1 us more).  Through a buffer resource over
+// eight rows at a time, so that its range check drops rows past M and columns past N:
+// three instructions a store instead of 21 with a 64-bit address and a mask formed for
+// each element, which one wave a SIMD had nothing to hide behind (Q8_0 4096^2 M = 333
+// 42.5 -> 38.8 us; Q4_K gate/up/down 4096 -> 14336, M = 512 / 4096 234 / 1551 -> 228 /
+// 1508; the wide tiles' split partials are bound by memory instead: 39.1 -> 38.6 at
+// Q5_K 4096x14336, M = 100).
+constexpr int64_t STORE_MAX_N = int64_t(1) << 26;  // eight rows below 2^31 bytes
+template <typename F>
+__device__ __forceinline__ void store_tile(float *y, int64_t left, int64_t N, int64_t n, int h, F val) {
+    if (N < STORE_MAX_N) {
+        uint32_t vo[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) vo[e] = n < N ? ((uint32_t)(4 * h + e) * (uint32_t)N + (uint32_t)n) * 4u : 0x80000000u;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint64_t a = reinterpret_cast<uint64_t>(y + 8 * q * N);
+            const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
+                               ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32);
+            const int rows = left >= 8 * q + 8 ? 8 : left > 8 * q ? (int)(left - 8 * q) : 0;
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                reinterpret_cast<void *>(u), (short)0, __builtin_amdgcn_readfirstlane(rows * (int)N * 4), 0x00020000);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val(4 * q + e)), rs, vo[e], 0, 2 /* nt */);
+        }
+    } else {
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int r = 8 * (v >> 2) + 4 * h + (v & 3);
+            if (r < left && n < N) __builtin_nontemporal_store(val(v), y + r * N + n);
+        }
+    }
+}
+
 // Pipeline.  The MFMAs of a block run as 16 k-steps of 2*MT MFMAs; each MFMA sits
 // in its own scheduling region (sched_barrier) together with a share of the
 // other work, so that work issues in the MFMA shadow instead of as a bubble
@@ -557,7 +596,7 @@ __global__ __launch_bounds__(256, (gemm_occupancy<TYPE, MT>())) void k_gemm(cons
     constexpr int PER = 8 / NG;                // B-operand dwords built per region
     constexpr int NPR = (8 + NG - 2) / (NG - 1 > 0 ? NG - 1 : 1);  // step 15: dwords per region after the scales
     __shared__ __align__(16) _Float16 As[2][BM][ALD];
-    __shared__ int Es[BM];
+    __shared__ __align__(16) int Es[BM];
 
     // tile of this workgroup: consecutive workgroup ids go to different XCDs, so
     // renumber them such that each XCD receives a contiguous run of tiles; tiles
@@ -717,23 +756,13 @@ __global__ __launch_bounds__(256, (gemm_occupancy<TYPE, MT>())) void k_gemm(cons
     }
     if (b < b1) block(b, 0);
 
-    // D layout of a 32x32 MFMA tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
+    for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
-            const int64_t m = m0 + r;
-            const int e = Es[r];
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int64_t n = n0 + 64 * wave + 32 * j + lr;
-                // nontemporal, as in the wide and tall tiles (Q4_K 14336x4096 M = 48 / 64
-                // 30.1 / 32.1 -> 29.5 / 31.2 us, split partials included)
-                if (m < M && n < N) __builtin_nontemporal_store(__builtin_amdgcn_ldexpf(acc[i][j][v], e + en[j]), y + m * N + n);
-            }
-        }
-    }
+        for (int j = 0; j < 2; j++)
+            store_tile(y + (m0 + 32 * i) * N, M - m0 - 32 * i, N, n0 + 64 * wave + 32 * j + lr, h, [&](int v) __attribute__((always_inline)) {
+                return __builtin_amdgcn_ldexpf(acc[i][j][v], Es[32 * i + 8 * (v >> 2) + 4 * h + (v & 3)] + en[j]);
+            });
 }
 
 // ---------------------------------------------------------------------------
@@ -774,7 +803,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_t(const uint8_t *__restrict__ W
     // places waits for the direct-to-LDS loads
     __shared__ __align__(1024) uint8_t As0[TBM * TROW];
     __shared__ __align__(1024) uint8_t As1[TBM * TROW];
-    __shared__ int Es[TBM];
+    __shared__ __align__(16) int Es[TBM];
 
     const int G = (int)gridDim.x, L = (int)blockIdx.x;
     const int T = (G & 7) == 0 ? (L & 7) * (G >> 3) + (L >> 3) : L;
@@ -937,18 +966,10 @@ __global__ __launch_bounds__(256, 1) void k_gemm_t(const uint8_t *__restrict__ W
     }
 
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
-            const int64_t m = m0 + r;
-            const int64_t n = n0 + 32 * wave + lr;
-            // nontemporal: the output tile is written once, at the end, by every
-            // workgroup at about the same time (Q4_K 14336x4096 M = 512 83.1 -> 80.5 us,
-            // M = 2048 308.6 -> 302.3 us; Q6_K M = 512 108.5 -> 105.6 us)
-            if (m < M && n < N) __builtin_nontemporal_store(__builtin_amdgcn_ldexpf(acc[i][v], Es[r] + en), y + m * N + n);
-        }
-    }
+    for (int i = 0; i < 8; i++)
+        store_tile(y + (m0 + 32 * i) * N, M - m0 - 32 * i, N, n0 + 32 * wave + lr, h, [&](int v) __attribute__((always_inline)) {
+            return __builtin_amdgcn_ldexpf(acc[i][v], Es[32 * i + 8 * (v >> 2) + 4 * h + (v & 3)] + en);
+        });
 }
 
 // ---------------------------------------------------------------------------
@@ -982,7 +1003,7 @@ __global__ __launch_bounds__(64 * NW, 1) void k_gemm_w(const uint8_t *__restrict
     using B = GB<TYPE>;
     __shared__ __align__(1024) uint8_t As0[WBM * TROW];
     __shared__ __align__(1024) uint8_t As1[WBM * TROW];
-    __shared__ int Es[WBM];
+    __shared__ __align__(16) int Es[WBM];
 
     const int G = (int)gridDim.x, L = (int)blockIdx.x;
     const int T = (G & 7) == 0 ? (L & 7) * (G >> 3) + (L >> 3) : L;
@@ -1126,18 +1147,10 @@ __global__ __launch_bounds__(64 * NW, 1) void k_gemm_w(const uint8_t *__restrict
     }
 
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
-            const int64_t m = m0 + r;
-            const int64_t n = n0 + 32 * wave + lr;
-            // nontemporal: the output tile is written once, at the end, by every
-            // workgroup at about the same time (Q4_K 14336x4096 M = 512 83.1 -> 80.5 us,
-            // M = 2048 308.6 -> 302.3 us; Q6_K M = 512 108.5 -> 105.6 us)
-            if (m < M && n < N) __builtin_nontemporal_store(__builtin_amdgcn_ldexpf(acc[i][v], Es[r] + en), y + m * N + n);
-        }
-    }
+    for (int i = 0; i < 4; i++)
+        store_tile(y + (m0 + 32 * i) * N, M - m0 - 32 * i, N, n0 + 32 * wave + lr, h, [&](int v) __attribute__((always_inline)) {
+            return __builtin_amdgcn_ldexpf(acc[i][v], Es[32 * i + 8 * (v >> 2) + 4 * h + (v & 3)] + en);
+        });
 }
 
 // ---------------------------------------------------------------------------
@@ -1177,7 +1190,7 @@ __global__ __launch_bounds__(512) void k_gemm_x(const uint8_t *__restrict__ W, i
     using B = GB<TYPE>;
     static_assert(!gemm_offset_step(TYPE), "no extra k-step here");
     __shared__ __align__(1024) uint8_t As0[XBUF], As1[XBUF], Bs0[XBUF], Bs1[XBUF];
-    __shared__ int Es[XBM];
+    __shared__ __align__(16) int Es[XBM];
     const int G = (int)gridDim.x, L = (int)blockIdx.x;
     const int T = (G & 7) == 0 ? (L & 7) * (G >> 3) + (L >> 3) : L;
     const int tm = T % g.tiles_m, tn = (T / g.tiles_m) % g.tiles_n, z = T / (g.tiles_m * g.tiles_n);
@@ -1306,26 +1319,26 @@ __global__ __launch_bounds__(512) void k_gemm_x(const uint8_t *__restrict__ W, i
         const int64_t n = n0 + 32 * wn + lr, nc = min(n, N - 1);
         const int eg = g.rexp[nc], eu = g.rexp2[nc];
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int r = 128 * wm + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
-                const float a = __builtin_amdgcn_ldexpf(acc[i][0][v], Es[r] + eg), c = __builtin_amdgcn_ldexpf(acc[i][1][v], Es[r] + eu);
-                if (m0 + r < M && n < N) __builtin_nontemporal_store(a / (1.f + expf(-a)) * c, y + (m0 + r) * N + n);
-            }
+        for (int i = 0; i < 4; i++) {
+            const int r0 = 128 * wm + 32 * i;
+            store_tile(y + (m0 + r0) * N, M - m0 - r0, N, n, h, [&](int v) __attribute__((always_inline)) {
+                const int e = Es[r0 + 8 * (v >> 2) + 4 * h + (v & 3)];
+                const float a = __builtin_amdgcn_ldexpf(acc[i][0][v], e + eg), c = __builtin_amdgcn_ldexpf(acc[i][1][v], e + eu);
+                return a / (1.f + expf(-a)) * c;
+            });
+        }
     } else {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int64_t n = n0 + 64 * wn + 32 * j + lr;
             const int en = g.rexp[min(n, N - 1)];
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int r = 128 * wm + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
-                    if (m0 + r < M && n < N)
-                        __builtin_nontemporal_store(__builtin_amdgcn_ldexpf(acc[i][j][v], Es[r] + en), y + (m0 + r) * N + n);
-                }
+            for (int i = 0; i < 4; i++) {
+                const int r0 = 128 * wm + 32 * i;
+                store_tile(y + (m0 + r0) * N, M - m0 - r0, N, n, h, [&](int v) __attribute__((always_inline)) {
+                    return __builtin_amdgcn_ldexpf(acc[i][j][v], Es[r0 + 8 * (v >> 2) + 4 * h + (v & 3)] + en);
+                });
+            }
         }
     }
 }
