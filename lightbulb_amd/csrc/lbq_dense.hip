@@ -344,6 +344,29 @@ __device__ __attribute__((noinline)) float dense_dot(const float *x, const uint8
     return s;
 }
 
+// One 32 x 32 tile from row mt on (store_tile).  last: these are results, not partial
+// sums, and one that is not finite is formed again; 0 * r summed over the lane's sixteen
+// is a NaN if any of them is.  For the 128 x 256 tiles, with 64 stores a lane (F16 8192^2
+// M = 2048 511 -> 499 us, 14336x4096 M = 512 124 -> 119); the smaller tiles' few stores
+// gain nothing by it (1000^3 23.7 -> 24.5).
+template <bool BF, bool W32>
+__device__ __forceinline__ void dense_store(floatx16 &acc, float *y, int64_t mt, int64_t M, int64_t N, int64_t n, int h,
+                                            bool last, const float *x, const uint8_t *W, int64_t K) {
+    if (last) {
+        float z = 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; v++) z = fmaf(acc[v], 0.f, z);
+        if (z != 0.f) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int64_t m = mt + 8 * (v >> 2) + 4 * h + (v & 3);
+                if (m < M && n < N && !dense_finite(acc[v])) acc[v] = dense_dot<BF, W32>(x + m * K, W + n * K * (W32 ? 4 : 2), K);
+            }
+        }
+    }
+    store_tile(y + mt * N, M - mt, N, n, h, [&](int v) __attribute__((always_inline)) { return acc[v]; });
+}
+
 // x [M][K] -> pieces [P][rows][Kp] (Kp = K up to a multiple of DK, zero filled) and,
 // for F16, the row exponents; one workgroup per row of x.
 template <bool BF>
@@ -534,8 +557,30 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
         stage(s + 1, 1);
     }
     __builtin_amdgcn_s_waitcnt(0);  // the loads past the slice
-    // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
     float *y = out + (int64_t)z * g.split_stride;
+    if constexpr (TM * TN >= 4) {
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            const int64_t mt = m0 + 32 * (wm * TM + i);
+            int e[16];
+            if constexpr (!BF) {
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const int64_t m = mt + 8 * (v >> 2) + 4 * h + (v & 3);
+                    e[v] = g.split_stride == 0 ? erow[m < M ? m : M - 1] : 0;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                if constexpr (!BF)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) acc[i][j][v] = __builtin_amdgcn_ldexpf(acc[i][j][v], e[v]);
+                dense_store<BF, false>(acc[i][j], y, mt, M, N, n0 + 32 * (wn * TN + j) + lr, h, g.split_stride == 0, x, W, K);
+            }
+        }
+        return;
+    }
+    // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -722,8 +767,17 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
         stage(s + 1, 1);
     }
     __builtin_amdgcn_s_waitcnt(0);  // the loads past the slice
-    // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
     float *y = out + (int64_t)z * g.split_stride;
+    if constexpr (TM * TN >= 4) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                dense_store<true, true>(acc[i][j], y, m0 + 32 * (wm * TM + i), M, N, n0 + 32 * (wn * TN + j) + lr, h,
+                                        g.split_stride == 0, x, W, K);
+        return;
+    }
+    // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll

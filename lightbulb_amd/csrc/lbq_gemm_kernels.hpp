@@ -535,45 +535,6 @@ constexpr int gemm_occupancy() {
 template <int TYPE, int MT>
 constexpr bool gemm_deep() { return TYPE == TYPE_Q4_K && MT == 1; }
 
-// Stores of one 32 x 32 MFMA tile: lane holds column n (its own), rows 8(v/4) + 4h + v%4
-// of the tile whose first row is y and of which `left` rows exist; val(v) is element v.
-// Nontemporal: a tile is written once, at the end, by every workgroup at about the same
-// time (Q4_K 14336x4096 M = 512 83.1 -> 80.5 us), and split partials too (cached, they
-// cost the split GEMMs at M = 100 about 1 us more).  Through a buffer resource over
-// eight rows at a time, so that its range check drops rows past M and columns past N:
-// three instructions a store instead of 21 with a 64-bit address and a mask formed for
-// each element, which one wave a SIMD had nothing to hide behind (Q8_0 4096^2 M = 333
-// 42.5 -> 38.8 us; Q4_K gate/up/down 4096 -> 14336, M = 512 / 4096 234 / 1551 -> 228 /
-// 1508; the wide tiles' split partials are bound by memory instead: 39.1 -> 38.6 at
-// Q5_K 4096x14336, M = 100).
-constexpr int64_t STORE_MAX_N = int64_t(1) << 26;  // eight rows below 2^31 bytes
-template <typename F>
-__device__ __forceinline__ void store_tile(float *y, int64_t left, int64_t N, int64_t n, int h, F val) {
-    if (N < STORE_MAX_N) {
-        uint32_t vo[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) vo[e] = n < N ? ((uint32_t)(4 * h + e) * (uint32_t)N + (uint32_t)n) * 4u : 0x80000000u;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint64_t a = reinterpret_cast<uint64_t>(y + 8 * q * N);
-            const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
-                               ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32);
-            const int rows = left >= 8 * q + 8 ? 8 : left > 8 * q ? (int)(left - 8 * q) : 0;
-            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                reinterpret_cast<void *>(u), (short)0, __builtin_amdgcn_readfirstlane(rows * (int)N * 4), 0x00020000);
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val(4 * q + e)), rs, vo[e], 0, 2 /* nt */);
-        }
-    } else {
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int r = 8 * (v >> 2) + 4 * h + (v & 3);
-            if (r < left && n < N) __builtin_nontemporal_store(val(v), y + r * N + n);
-        }
-    }
-}
-
 // Pipeline.  The MFMAs of a block run as 16 k-steps of 2*MT MFMAs; each MFMA sits
 // in its own scheduling region (sched_barrier) together with a share of the
 // other work, so that work issues in the MFMA shadow instead of as a bubble

@@ -91,6 +91,24 @@ def test_dense_mm_nonfinite(lbq, dev, t, m, n, k):
 
 
 @pytest.mark.parametrize("t", [F16, F32])
+def test_dense_mm_nonfinite_large_tiles(lbq, dev, t):
+    # 128 x 256 tiles, the last row tile short: a lane's sixteen results are tested together
+    rng = np.random.default_rng(19)
+    m, n, k = 1430, 4096, 72
+    w = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1, 5], x[700, 9], x[1429, 60] = np.inf, np.nan, -np.inf
+    w[7, 20], w[9, 5], w[4095, 30] = np.inf, 0.0, np.nan
+    qm, w = _weight(t, n, k, rng, dev, w)
+    y = qm.forward(to_dev(x, dev)).cpu().numpy()
+    ref = (torch.from_numpy(x).double() @ torch.from_numpy(w).double().T).numpy()
+    fin = np.isfinite(ref)
+    assert np.array_equal(np.isnan(ref), np.isnan(y))
+    assert np.array_equal(ref[~fin & ~np.isnan(ref)], y[~fin & ~np.isnan(ref)])
+    _assert_rows(np.where(fin, y, 0)[fin.any(1)], np.where(fin, ref, 0)[fin.any(1)], _bound(t, k))
+
+
+@pytest.mark.parametrize("t", [F16, F32])
 def test_dense_mm_streams_growth_and_capture(lbq, dev, t):
     # the operand buffer: two streams in turn, a larger call while a captured graph
     # uses the smaller buffer, and replays between eager calls
