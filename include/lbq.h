@@ -160,8 +160,8 @@ int lbq_weight_info(const lbq_weight *w, uint32_t *ggml_type, int64_t *n, int64_
  * adds when y is plain device memory (hipMalloc; checked once per allocation),
  * else through partial sums in the workspace; either way y = a + b for the two
  * halves, the same bits for finite normal-range halves.  Dense F32/F16/BF16
- * weights are candle's dense variant: no quantisation, an f32 matmul (F16 / BF16
- * at m > 8: x as 16-bit operands that add up to it, in the context's scratch;
+ * weights are candle's dense variant: no quantisation, an f32 matmul (at
+ * m > 8 x, and an F32 weight, as 16-bit operands that add up to it, x's in the context's scratch;
  * under a graph capture that would have to grow that scratch, the f32 matrix
  * cores).  m == 0 is a no-op. */
 int lbq_qmatmul_f32(lbq_ctx *ctx, const lbq_weight *w, const float *d_x, int64_t m, float *d_y, void *stream);

@@ -42,7 +42,7 @@ struct lbq_ctx {
     size_t ws_bytes;
     uint8_t *tmp;         // gate and up outputs when their product is not fused
     size_t tmp_bytes;
-    // dense F16 / BF16 at m > 8: operand pieces and split-k partials.  Outgrown buffers
+    // dense weights at m > 8: operand pieces and split-k partials.  Outgrown buffers
     // stay until the context goes (their sizes double, so they add up to less than the
     // current one): a captured graph may still use them.
     uint8_t *dense_ws;
