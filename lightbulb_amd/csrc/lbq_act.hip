@@ -443,50 +443,39 @@ hipError_t launch_embedding(int type, const uint8_t *w, int64_t n, int64_t k, in
 // candle's RmsNorm (f32): y = x / sqrt(sum(x^2) / k + eps) * w, one workgroup per row
 __global__ __launch_bounds__(256) void k_rmsnorm(const float *__restrict__ x, const float *__restrict__ w, float eps,
                                                  int64_t k, float *__restrict__ y) {
-    __shared__ float red[4];
     const int64_t m = blockIdx.x;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int t = threadIdx.x;
     const float *xr = x + m * k;
-    float ss = 0.f;
-    for (int64_t i = t; i < k; i += 256) ss += xr[i] * xr[i];
-    ss = row_sum_f32(ss);
-    ss = __int_as_float(rl(__float_as_uint(ss), 0)) + __int_as_float(rl(__float_as_uint(ss), 16)) +
-         __int_as_float(rl(__float_as_uint(ss), 32)) + __int_as_float(rl(__float_as_uint(ss), 48));
-    if (lane == 0) red[wave] = ss;
-    __syncthreads();
-    const float rms = sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+    const float rms = row_rms(xr, t, k, eps);
     for (int64_t i = t; i < k; i += 256) y[m * k + i] = xr[i] / rms * w[i];
 }
 
-// The same for 16-byte aligned rows of k % 4 == 0 up to 1024 P values: the row and the
-// weight in registers, loaded once, 16 bytes at a time (32x4096 6.4 -> 3.2 us against
-// four-byte loads of the row twice).
+// The same for rows up to 256 P values: the row and the weight in registers, loaded once,
+// every load in flight before the first is used (no branch around a load), in the order of
+// k_rmsnorm's sum (the same bits).  Bound by one pass's latency, by memory from about a
+// thousand rows: k_rmsnorm's two passes of one load a step -> this, 512x4096 11.0 -> 5.9
+// us, 4096x4096 32.2 -> 21.3.  16-byte loads with sums of four neighbours took 5.6 and 20.7
+// but gave another last bit.
 template <int P>
-__global__ __launch_bounds__(256) void k_rmsnorm_v(const float *__restrict__ x, const float *__restrict__ w, float eps,
+__global__ __launch_bounds__(256) void k_rmsnorm_r(const float *__restrict__ x, const float *__restrict__ w, float eps,
                                                    int64_t k, float *__restrict__ y) {
-    __shared__ float red[4];
     const int64_t m = blockIdx.x;
-    const int t = threadIdx.x, k4 = (int)(k / 4);
-    const float4 *xr = reinterpret_cast<const float4 *>(x + m * k), *wr = reinterpret_cast<const float4 *>(w);
-    float4 v[P], g[P];
+    const int t = threadIdx.x;
+    const float *xr = x + m * k;
+    const int last = (int)k - 1;
+    float v[P], g[P];
 #pragma unroll
-    for (int j = 0; j < P; j++) v[j] = t + 256 * j < k4 ? xr[t + 256 * j] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j = 0; j < P; j++) v[j] = xr[min(t + 256 * j, last)];
 #pragma unroll
-    for (int j = 0; j < P; j++) g[j] = t + 256 * j < k4 ? wr[t + 256 * j] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j = 0; j < P; j++) g[j] = w[min(t + 256 * j, last)];
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < P; j++) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
-    ss = row_sum_f32(ss);
-    ss = __int_as_float(rl(__float_as_uint(ss), 0)) + __int_as_float(rl(__float_as_uint(ss), 16)) +
-         __int_as_float(rl(__float_as_uint(ss), 32)) + __int_as_float(rl(__float_as_uint(ss), 48));
-    if ((t & 63) == 0) red[t >> 6] = ss;
-    __syncthreads();
-    const float rms = sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
-    float4 *yr = reinterpret_cast<float4 *>(y + m * k);
+    for (int j = 0; j < P; j++) ss = t + 256 * j <= last ? fmaf(v[j], v[j], ss) : ss;
+    const float rms = rms_of_256(ss, t, k, eps);
+    float *yr = y + m * k;
 #pragma unroll
     for (int j = 0; j < P; j++)
-        if (t + 256 * j < k4)
-            yr[t + 256 * j] = make_float4(v[j].x / rms * g[j].x, v[j].y / rms * g[j].y, v[j].z / rms * g[j].z, v[j].w / rms * g[j].w);
+        if (t + 256 * j <= last) yr[t + 256 * j] = v[j] / rms * g[j];
 }
 
 // candle's RmsNorm (f32) of each row and the Q8_K quantisation of the result in
@@ -575,12 +564,11 @@ hipError_t launch_rmsnorm_q8k(const float *x, const float *w, float eps, int64_t
 
 hipError_t launch_rmsnorm(const float *x, const float *w, float eps, int64_t m, int64_t k, float *y, hipStream_t st) {
     if (m <= 0) return hipSuccess;
-    const uintptr_t all = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y);
-    if (k % 4 == 0 && k <= 16384 && !(all & 15u)) {
-        if (k <= 2048) k_rmsnorm_v<2><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
-        else if (k <= 4096) k_rmsnorm_v<4><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
-        else if (k <= 8192) k_rmsnorm_v<8><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
-        else k_rmsnorm_v<16><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
+    if (k <= 16384) {
+        if (k <= 2048) k_rmsnorm_r<8><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
+        else if (k <= 4096) k_rmsnorm_r<16><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
+        else if (k <= 8192) k_rmsnorm_r<32><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
+        else k_rmsnorm_r<64><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
         return hipGetLastError();
     }
     k_rmsnorm<<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);

@@ -65,6 +65,36 @@ __device__ __forceinline__ int quad_sum_i32(int v) {
 }
 __device__ __forceinline__ uint32_t rl(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lane); }
 
+// sqrt(sum(x^2) / k + eps) of a row, the same value in every thread of a workgroup of at
+// least 256, all of which call it.  One order of summation wherever a row's norm is
+// formed -- thread t of 256 adds the squares of x[t], x[t + 256], ... in turn, then the
+// threads' sums are added by lanes, rows of 16 and waves -- so that a norm inside another
+// kernel gives k_rmsnorm's bits: another last bit of the RMS moves the codes that lie at a
+// tie (4e-4 of an MLP's output).
+// rms_of_256: from the first 256 threads' sums; row_rms: from the row, eight loads at a time.
+__device__ __forceinline__ float rms_of_256(float ss, int t, int64_t k, float eps) {
+    __shared__ float red[4];
+    if (t < 256) {  // wave-uniform
+        ss = row_sum_f32(ss);
+        ss = __int_as_float(rl(__float_as_uint(ss), 0)) + __int_as_float(rl(__float_as_uint(ss), 16)) +
+             __int_as_float(rl(__float_as_uint(ss), 32)) + __int_as_float(rl(__float_as_uint(ss), 48));
+        if ((t & 63) == 0) red[t >> 6] = ss;
+    }
+    __syncthreads();
+    return sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+}
+__device__ __forceinline__ float row_rms(const float *xr, int t, int64_t k, float eps) {
+    float ss = 0.f;
+    for (int64_t i = t; t < 256 && i < k; i += 2048) {
+        float u[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) u[j] = xr[i + 256 * j < k ? i + 256 * j : k - 1];  // (no branch: all in flight)
+#pragma unroll
+        for (int j = 0; j < 8; j++) ss = i + 256 * j < k ? fmaf(u[j], u[j], ss) : ss;
+    }
+    return rms_of_256(ss, t, k, eps);
+}
+
 // Q8_K quantisation of one 256-value block by 16 aligned lanes, 16 consecutive
 // values per lane (lane sub = lane % 16 holds values 16 sub .. 16 sub + 15).
 // Candle's BlockQ8K::from_float: the first value of largest |x| (NaN never

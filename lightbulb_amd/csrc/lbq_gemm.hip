@@ -97,21 +97,6 @@ __device__ __forceinline__ void load16(const float *p, float v[16]) {
     }
 }
 
-// sqrt(sum / K + eps) of the workgroup's T threads' shares of a sum of squares
-template <int T>
-__device__ __forceinline__ float row_rms(float ss, int t, int64_t K, float eps) {
-    __shared__ float red[T / 64];
-    ss = row_sum_f32(ss);
-    ss = __int_as_float(rl(__float_as_uint(ss), 0)) + __int_as_float(rl(__float_as_uint(ss), 16)) +
-         __int_as_float(rl(__float_as_uint(ss), 32)) + __int_as_float(rl(__float_as_uint(ss), 48));
-    if ((t & 63) == 0) red[t >> 6] = ss;
-    __syncthreads();
-    float sum = red[0];
-#pragma unroll
-    for (int w = 1; w < T / 64; w++) sum += red[w];
-    return sqrtf(sum / (float)K + eps);
-}
-
 // The same operand rows straight from f32 x (k <= 16384): the workgroup
 // quantises its row to Q8_K in registers (q8k_lane16, as the standalone
 // quantiser), shares the block scales through LDS for the row exponent, and
@@ -119,8 +104,10 @@ __device__ __forceinline__ float row_rms(float ss, int t, int64_t K, float eps) 
 // bit-identical operands.  P: passes of T / 16 blocks, the fewest covering the
 // row (every load of a pass is issued, so no more passes than the row needs).
 // NORM: candle's RmsNorm (f32, weight nw) of the row first, so that the normalised row
-// never reaches memory (k_rmsnorm and this took 14.3 + 5.1 us at 512x4096, 45 + 19 us at
-// 4096x4096; together 6.2 and 28).
+// never reaches memory: k_rmsnorm and this took 11.0 + 4.8 us at 512x4096, 32.2 + 16.6 at
+// 4096x4096; together 7.2 and 24.5.  The sum of squares is k_rmsnorm's to the bit: its
+// threads take values 256 apart, here from a copy of the row in LDS (0.7 us at 512
+// rows beside the sum of a thread's own 16; from memory again 1.3).
 template <int T, int P, bool NORM>
 __global__ __launch_bounds__(T) void k_quant_f16(const float *__restrict__ x, const float *__restrict__ nw, float eps,
                                                  int64_t K, _Float16 *__restrict__ A, int *__restrict__ erow, int opmajor) {
@@ -143,17 +130,18 @@ __global__ __launch_bounds__(T) void k_quant_f16(const float *__restrict__ x, co
         }
     }
     if constexpr (NORM) {
+        __shared__ float4 row[T * P * 4];  // x in order: k_rmsnorm's sum takes it 256 values apart
         float al[MAXP][16];
 #pragma unroll
         for (int j = 0; j < MAXP; j++)
             load16(nw + (int64_t)min(BPP * j + (t >> 4), nbx - 1) * KB + 16 * sub, al[j]);
-        float ss = 0.f;
 #pragma unroll
         for (int j = 0; j < MAXP; j++)
-            if (BPP * j + (t >> 4) < nbx)  // clamped duplicates do not count
 #pragma unroll
-                for (int i = 0; i < 16; i++) ss += v[j][i] * v[j][i];
-        const float rms = row_rms<T>(ss, t, K, eps);
+            for (int i = 0; i < 4; i++)
+                row[4 * (T * j + t) + i] = make_float4(v[j][4 * i], v[j][4 * i + 1], v[j][4 * i + 2], v[j][4 * i + 3]);
+        __syncthreads();
+        const float rms = row_rms(reinterpret_cast<const float *>(row), t, K, eps);
 #pragma unroll
         for (int j = 0; j < MAXP; j++)
 #pragma unroll
@@ -234,17 +222,18 @@ __global__ __launch_bounds__(T) void k_quant_f16_q80(const float *__restrict__ x
         }
     }
     if constexpr (NORM) {
+        __shared__ float4 row[T * P * 4];  // x in order: k_rmsnorm's sum takes it 256 values apart
         float al[MAXP][16];
 #pragma unroll
         for (int j = 0; j < MAXP; j++)
             load16(nw + (int64_t)min(BPP * j + (t >> 1), nbx - 1) * 32 + 16 * sub, al[j]);
-        float ss = 0.f;
 #pragma unroll
         for (int j = 0; j < MAXP; j++)
-            if (BPP * j + (t >> 1) < nbx)
 #pragma unroll
-                for (int i = 0; i < 16; i++) ss += v[j][i] * v[j][i];
-        const float rms = row_rms<T>(ss, t, K, eps);
+            for (int i = 0; i < 4; i++)
+                row[4 * (T * j + t) + i] = make_float4(v[j][4 * i], v[j][4 * i + 1], v[j][4 * i + 2], v[j][4 * i + 3]);
+        __syncthreads();
+        const float rms = row_rms(reinterpret_cast<const float *>(row), t, K, eps);
 #pragma unroll
         for (int j = 0; j < MAXP; j++)
 #pragma unroll
