@@ -10,9 +10,9 @@
 //           the next unit's 16-byte loads in flight, x staged in LDS, f32 FMA
 //           against up to 8 activation rows, DPP row sums -- HBM-bound like the
 //           quantised decode GEMV;
-//   m > 8   k_dense_mm (F16 / BF16), k_dense_mm32 (F32): x, and an F32 weight, as two
-//           fp16 or three bf16 operands that add up to it, on the 16-bit matrix
-//           cores with f32 accumulation;
+//   m > 8   k_dense_mm (F16 / BF16), k_dense_mm32 (F32): x as three bf16 operands that add
+//           up to it, an F16 weight as two and an F32 weight as three, on the 16-bit
+//           matrix cores with f32 accumulation;
 //           k_dense_gemm (calls without a workspace): 64 x 128
 //           output tiles on v_mfma_f32_32x32x2_f32, operands staged through LDS.
 // Every product is formed at f32 precision and summed in f32; only the
@@ -283,27 +283,25 @@ __global__ __launch_bounds__(256) void k_dense_gemm(const uint8_t *__restrict__ 
 
 
 // ---------------------------------------------------------------------------
-// m > 8 with F16 / BF16 weights: the weights are fp16 / bf16 MFMA operands as they
-// lie in memory, and x enters as P operands of the same type that add up to it:
-//   F16   P = 2: x * 2^-e = hi + lo, e the row's exponent (largest finite |x| in
-//         [2^14, 2^15) after it), hi and lo rounded to nearest: 22 bits and the
-//         rounding sign of x (lo is exact to 2^-25, so what a value loses below
-//         that is 2^-39 of the row's largest);
-//   BF16  P = 3: x = hi + mid + lo by truncation, 3 x 8 bits: exact, no exponent.
-// Every product is exact in the f32 accumulator of v_mfma_f32_32x32x16_{f16,bf16},
-// so only the f32 summation rounds.  P MFMAs of 16 k-values replace eight
-// v_mfma_f32_32x32x2_f32, at 16 times their rate.  Bound by the matrix cores and
-// their clock from M = 512 (0.9-1.1 PFLOP/s of operand products), by the launches
-// below.  Against k_dense_gemm, us per call and relative error against 64 bits:
-//   F16 4096^2    M = 9 / 64 / 512   237 / 241 / 244 -> 15.6 / 21.1 / 47.7, 1.1e-6 -> 4.1e-7
-//   F16 8192^2    M = 2048           3003 -> 503,  1.6e-6 -> 8.2e-7
-//   BF16 4096^2   M = 32 / 512       239 / 246 -> 17.1 / 57.2, 1.1e-6 -> 5.0e-7
-//   BF16 8192^2   M = 2048           3003 -> 955,  1.6e-6 -> 1.0e-6
-//   F16 512^2     M = 9              32.2 -> 14.0, 4e-7 -> 1.6e-7
+// m > 8 with F16 / BF16 weights.  x enters as three bf16 operands (k_dense_pieces) whose
+// sum is x; a BF16 weight is an operand as it lies in memory, and an F16 weight, 11 bits,
+// is the sum of two bf16 values that a wave forms in registers (dense_split2).  All
+// products, three or six of them, are taken, and each is exact in the f32 accumulator
+// of v_mfma_f32_32x32x16_bf16, so only the f32 summation rounds: an output is as good as
+// an f32 product's whatever the range of its row.  (Two fp16 operands for x at one
+// exponent a row took a third of the MFMAs, but lose what lies 2^-17 and more below the
+// row's largest |x|, which may well meet a zero weight.)
+// Bound by the matrix cores from M = 512 (1.0-1.5 PFLOP/s of operand products), by the
+// launches below.  Against k_dense_gemm, us per call and relative error against 64 bits:
+//   F16 4096^2    M = 9 / 64 / 512   236 / 240 / 243 -> 16.6 / 26.7 / 90.9, 1.2e-6 -> 1.2e-7 / 1.2e-7 / 2.7e-7
+//   F16 8192^2    M = 2048           2976 -> 1110, 1.6e-6 -> 5.7e-7
+//   BF16 4096^2   M = 32 / 512       238 / 245 -> 17.3 / 58.7, 1.2e-6 -> 1.2e-7 / 2.7e-7
+//   BF16 8192^2   M = 2048           2980 -> 622,  1.6e-6 -> 5.7e-7
+//   F16 512^2     M = 9              32.1 -> 12.1, 4.1e-7 -> 9.5e-8
 //
 // Tiles.  A workgroup of WM x WN waves owns BM = 32 WM TM rows of x and
 // BN = 32 WN TN weight rows; a wave its TM x TN tiles of 32 x 32.  k advances in
-// stages of 64: the P x BM x 64 pieces and the BN x 64 weights go into LDS by
+// stages of 64: the 3 x BM x 64 pieces and the BN x 64 weights go into LDS by
 // buffer loads to LDS (16 B a lane, 8 rows of 128 B an instruction), two buffers;
 // row r's 16-byte chunk c sits in slot c ^ ((r >> 1) & 7), so the 32 rows of an
 // operand read spread over the banks.  One barrier a stage, before its last k-step:
@@ -315,19 +313,25 @@ __global__ __launch_bounds__(256) void k_dense_gemm(const uint8_t *__restrict__ 
 // slice order.
 //
 // A result that is not finite is formed again from x and W by f32 FMAs in k order
-// (dense_dot): an infinity in x or W would otherwise meet the zero lo pieces.
+// (dense_dot): an infinity in x or W would otherwise meet the zero pieces.
 // ---------------------------------------------------------------------------
 constexpr int DK = 64;  // values of k per stage
 
-typedef _Float16 dhalf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 dbf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 dbf2 __attribute__((ext_vector_type(2)));
+typedef float dfl2 __attribute__((ext_vector_type(2)));
 
-template <bool BF>
 __device__ __forceinline__ floatx16 dense_mfma(uint4 a, uint4 b, floatx16 c) {
-    if constexpr (BF)
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(dbf8, a), __builtin_bit_cast(dbf8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(dhalf8, a), __builtin_bit_cast(dhalf8, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(dbf8, a), __builtin_bit_cast(dbf8, b), c, 0, 0, 0);
+}
+
+// two values' bf16 (nearest), value 0 in the low half; v keeps what is left
+__device__ __forceinline__ uint32_t dense_split2(float &v0, float &v1) {
+    const dfl2 f = {v0, v1};
+    const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, dbf2));
+    v0 -= __uint_as_float(b << 16);
+    v1 -= __uint_as_float(b & 0xffff0000u);
+    return b;
 }
 
 __device__ __forceinline__ bool dense_finite(float v) { return fabsf(v) <= 3.4028234664e38f; }  // false for NaN
@@ -367,59 +371,30 @@ __device__ __forceinline__ void dense_store(floatx16 &acc, float *y, int64_t mt,
     store_tile(y + mt * N, M - mt, N, n, h, [&](int v) __attribute__((always_inline)) { return acc[v]; });
 }
 
-// x [M][K] -> pieces [P][rows][Kp] (Kp = K up to a multiple of DK, zero filled) and,
-// for F16, the row exponents; one workgroup per row of x.
-template <bool BF>
+// x [M][K] -> pieces [3][rows][Kp] (Kp = K up to a multiple of DK, zero filled); one
+// workgroup per row of x
 __global__ __launch_bounds__(256) void k_dense_pieces(const float *__restrict__ x, int64_t K, int64_t Kp, int64_t rows,
-                                                      unsigned short *__restrict__ A, int *__restrict__ erow) {
+                                                      unsigned short *__restrict__ A) {
     const int64_t m = blockIdx.x;
-    const int t = threadIdx.x;
     const bool xv = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
     const float *xr = x + m * K;
-    int e = 0;
-    if constexpr (!BF) {
-        __shared__ float wmax[4];
-        float mx = 0.f;
-        for (int64_t c = 8 * t; c < K; c += 2048) {
-            float v[8];
-            load_x8(xr + c, xv, v);
-#pragma unroll
-            for (int i = 0; i < 8; i++) mx = fmaxf(mx, dense_finite(v[i]) ? fabsf(v[i]) : 0.f);
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-        if ((t & 63) == 0) wmax[t >> 6] = mx;
-        __syncthreads();
-        mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-        e = mx > 0.f ? __builtin_amdgcn_frexp_expf(mx) - 15 : 0;
-        if (t == 0) erow[m] = e;
-    }
     unsigned short *a = A + m * Kp;
     const int64_t ps = rows * Kp;
-    for (int64_t c = 8 * t; c < Kp; c += 2048) {
+    for (int64_t c = 8 * threadIdx.x; c < Kp; c += 2048) {
         float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         if (c < K) load_x8(xr + c, xv, v);
         uint32_t pc[3][4];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             uint32_t b[3];
-            if constexpr (BF) {
-                const uint32_t u0 = __float_as_uint(v[i]);
-                const bool fin = dense_finite(v[i]);
-                // a NaN keeps a mantissa bit in the upper half
-                b[0] = (u0 >> 16) | (v[i] != v[i] ? 0x40u : 0u);
-                const float r1 = v[i] - __uint_as_float(u0 & 0xffff0000u);
-                const uint32_t u1 = fin ? __float_as_uint(r1) : 0u;
-                b[1] = u1 >> 16;
-                b[2] = fin ? __float_as_uint(r1 - __uint_as_float(u1 & 0xffff0000u)) >> 16 : 0u;
-            } else {
-                const float s = __builtin_amdgcn_ldexpf(v[i], -e);
-                const _Float16 hi = (_Float16)s;
-                const _Float16 lo = (_Float16)(dense_finite(s) ? s - (float)hi : 0.f);
-                b[0] = __builtin_bit_cast(unsigned short, hi);
-                b[1] = __builtin_bit_cast(unsigned short, lo);
-                b[2] = 0u;
-            }
+            const uint32_t u0 = __float_as_uint(v[i]);
+            const bool fin = dense_finite(v[i]);
+            // a NaN keeps a mantissa bit in the upper half
+            b[0] = (u0 >> 16) | (v[i] != v[i] ? 0x40u : 0u);
+            const float r1 = v[i] - __uint_as_float(u0 & 0xffff0000u);
+            const uint32_t u1 = fin ? __float_as_uint(r1) : 0u;
+            b[1] = u1 >> 16;
+            b[2] = fin ? __float_as_uint(r1 - __uint_as_float(u1 & 0xffff0000u)) >> 16 : 0u;
 #pragma unroll
             for (int p = 0; p < 3; p++) {
                 if (i & 1) pc[p][i >> 1] |= b[p] << 16;
@@ -427,7 +402,7 @@ __global__ __launch_bounds__(256) void k_dense_pieces(const float *__restrict__ 
             }
         }
 #pragma unroll
-        for (int p = 0; p < (BF ? 3 : 2); p++)
+        for (int p = 0; p < 3; p++)
             *reinterpret_cast<uint4 *>(a + p * ps + c) = make_uint4(pc[p][0], pc[p][1], pc[p][2], pc[p][3]);
     }
 }
@@ -447,11 +422,11 @@ struct DenseGrid {
     int64_t split_stride;               // partials apart (0: out is y)
 };
 
-template <bool BF, int P, int WM, int WN, int TM, int TN>
+template <bool BF, int WM, int WN, int TM, int TN>
 __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__restrict__ W, int64_t N, int64_t K,
-                                                           const unsigned short *__restrict__ A,
-                                                           const int *__restrict__ erow, const float *__restrict__ x,
+                                                           const unsigned short *__restrict__ A, const float *__restrict__ x,
                                                            int64_t M, float *__restrict__ out, DenseGrid g) {
+    constexpr int P = 3;
     constexpr int NW = WM * WN, BM = 32 * WM * TM, BN = 32 * WN * TN;
     constexpr int RA = BM / 8 / NW, RB = BN / 8 / NW;  // staging instructions per wave: RA per piece, RB
     static_assert(RA * 8 * NW == BM && RB * 8 * NW == BN && NW % 2 == 0, "whole staging instructions per wave");
@@ -468,7 +443,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
 
     const __amdgpu_buffer_rsrc_t a0 = dense_rsrc(A + m0 * g.Kp, BM * g.Kp * 2);
     const __amdgpu_buffer_rsrc_t a1 = dense_rsrc(A + (g.rows + m0) * g.Kp, BM * g.Kp * 2);
-    const __amdgpu_buffer_rsrc_t a2 = dense_rsrc(A + ((P - 1) * g.rows + m0) * g.Kp, BM * g.Kp * 2);
+    const __amdgpu_buffer_rsrc_t a2 = dense_rsrc(A + (2 * g.rows + m0) * g.Kp, BM * g.Kp * 2);
     const __amdgpu_buffer_rsrc_t br = dense_rsrc(W + n0 * K * 2, (N - n0 < BN ? N - n0 : BN) * K * 2);
     // lane l of an instruction fills row l/8, slot l%8 of its 8 rows; the rows' number
     // / 8 has the wave's parity (NW is even)
@@ -510,30 +485,49 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
         asm volatile("" : "+v"(oa[ks]), "+v"(ob[ks]));
     }
 
-    floatx16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-    // operands of this k-step and the next; operand q of a k-step: its TN B, then its P TM A
-    constexpr int NO = TN + P * TM, NM = P * TM * TN;  // operands, MFMAs per k-step
-    uint4 op[2][NO];
+    // sums of the first pieces' products, and of the others, which are 2^-7 of them and
+    // less: a rounding at the size of the result an MFMA step instead of three to eight
+    floatx16 acc[TM][TN] = {}, low[TM][TN] = {};
+    // operands of this k-step and the next: a weight's (BF) or its two pieces', x's pieces;
+    // the next one's F16 weights
+    constexpr int Q = BF ? 1 : 2, NA = P * TM, NM = P * Q * TM * TN;
+    uint4 xa[2][NA], wb[2][TN][Q], raw[TN];
     auto read = [&](int buf, int ks, int r, int q) __attribute__((always_inline)) {
-        if (q < TN) op[r][q] = *reinterpret_cast<const uint4 *>((buf ? Bs1 : Bs0) + (ob[ks] + q * 4096));
+        if (q < TN) (BF ? wb[r][q][0] : raw[q]) = *reinterpret_cast<const uint4 *>((buf ? Bs1 : Bs0) + (ob[ks] + q * 4096));
         else
-            op[r][q] = *reinterpret_cast<const uint4 *>((buf ? As1 : As0) +
-                                                        (oa[ks] + (q - TN) / TM * (BM * 128) + (q - TN) % TM * 4096));
+            xa[r][q - TN] = *reinterpret_cast<const uint4 *>((buf ? As1 : As0) +
+                                                             (oa[ks] + (q - TN) / TM * (BM * 128) + (q - TN) % TM * 4096));
     };
-    // the MFMAs of the k-step in op[r], each followed by its share of the next one's reads
+    // pair c (two F16 weights) of raw -> wb[r]
+    auto split = [&](int r, int c) __attribute__((always_inline)) {
+        const int j = c >> 2, e = c & 3;
+        const uint32_t u = e == 0 ? raw[j].x : e == 1 ? raw[j].y : e == 2 ? raw[j].z : raw[j].w;
+        float v0 = w16<false>(u & 0xffffu), v1 = w16<false>(u >> 16);
+#pragma unroll
+        for (int p = 0; p < Q; p++) {
+            const uint32_t b = dense_split2(v0, v1);
+            if (e == 0) wb[r][j][p].x = b;
+            else if (e == 1) wb[r][j][p].y = b;
+            else if (e == 2) wb[r][j][p].z = b;
+            else wb[r][j][p].w = b;
+        }
+    };
+    // the MFMAs of the k-step in xa[r], wb[r], each followed by its share of the next one's
+    // reads and, F16, after half of them of its splits
     auto step = [&](int r, int buf, int ks) __attribute__((always_inline)) {
+        constexpr int H = BF ? NM : NM / 2, NR = TN + NA;
 #pragma unroll
         for (int u = 0; u < NM; u++) {
             const int j = u % TN, i = u / TN % TM, p = u / TN / TM;
-            acc[i][j] = dense_mfma<BF>(op[r][TN + p * TM + i], op[r][j], acc[i][j]);
+            floatx16 &to = p ? low[i][j] : acc[i][j];
+            to = dense_mfma(xa[r][p / Q * TM + i], wb[r][j][p % Q], to);
+            if (u < H) {
 #pragma unroll
-            for (int q = u * NO / NM; q < (u + 1) * NO / NM; q++) read(buf, ks, r ^ 1, q);
+                for (int q = u * NR / H; q < (u + 1) * NR / H; q++) read(buf, ks, r ^ 1, q);
+            } else {
+#pragma unroll
+                for (int c = (u - H) * 4 * TN / (NM - H + BF); c < (u - H + 1) * 4 * TN / (NM - H + BF); c++) split(r ^ 1, c);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -542,7 +536,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NO; q++) read(0, 0, 0, q);
+    for (int q = 0; q < TN + NA; q++) read(0, 0, 0, q);
+    if constexpr (!BF)
+#pragma unroll
+        for (int c = 0; c < 4 * TN; c++) split(0, c);
     auto stage = [&](int s, int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int ks = 0; ks < 3; ks++) step(ks & 1, buf, ks + 1);
@@ -557,27 +554,18 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
         stage(s + 1, 1);
     }
     __builtin_amdgcn_s_waitcnt(0);  // the loads past the slice
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] += low[i][j];
     float *y = out + (int64_t)z * g.split_stride;
     if constexpr (TM * TN >= 4) {
 #pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int64_t mt = m0 + 32 * (wm * TM + i);
-            int e[16];
-            if constexpr (!BF) {
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int64_t m = mt + 8 * (v >> 2) + 4 * h + (v & 3);
-                    e[v] = g.split_stride == 0 ? erow[m < M ? m : M - 1] : 0;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                if constexpr (!BF)
-#pragma unroll
-                    for (int v = 0; v < 16; v++) acc[i][j][v] = __builtin_amdgcn_ldexpf(acc[i][j][v], e[v]);
-                dense_store<BF, false>(acc[i][j], y, mt, M, N, n0 + 32 * (wn * TN + j) + lr, h, g.split_stride == 0, x, W, K);
-            }
-        }
+            for (int j = 0; j < TN; j++)
+                dense_store<BF, false>(acc[i][j], y, m0 + 32 * (wm * TM + i), M, N, n0 + 32 * (wn * TN + j) + lr, h,
+                                       g.split_stride == 0, x, W, K);
         return;
     }
     // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
@@ -591,17 +579,14 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
                 const int64_t m = m0 + 32 * (wm * TM + i) + 8 * (v >> 2) + 4 * h + (v & 3);
                 if (m >= M || n >= N) continue;
                 float r = acc[i][j][v];
-                if (g.split_stride == 0) {
-                    if constexpr (!BF) r = __builtin_amdgcn_ldexpf(r, erow[m]);
-                    if (!dense_finite(r)) r = dense_dot<BF>(x + m * K, W + n * K * 2, K);
-                }
+                if (g.split_stride == 0 && !dense_finite(r)) r = dense_dot<BF>(x + m * K, W + n * K * 2, K);
                 y[m * N + n] = r;
             }
         }
 }
 
 // ---------------------------------------------------------------------------
-// m > 8 with F32 weights: x as the three bf16 pieces of k_dense_pieces<true> (their sum
+// m > 8 with F32 weights: x as the three bf16 pieces of k_dense_pieces (their sum
 // is x), and each weight as three bf16 pieces that a wave forms in registers from the
 // f32 value in LDS: hi = bf16(w), mid = bf16(w - hi), lo = w - hi - mid, rounded to
 // nearest, again exact.  Six of the nine products, all exact in the accumulator:
@@ -616,24 +601,12 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
 // Bound by the matrix cores from M = 200 (1.0-1.3 PFLOP/s of operand products), by the
 // weights' bytes and the launches below.  Against k_dense_gemm, us per call and relative
 // error against 64 bits:
-//   4096^2       M = 9 / 64 / 512  232 / 243 / 246 -> 19.5 / 30.3 / 105, 1.1e-6 -> 2.7e-7 / 2.7e-7 / 7.1e-7
-//   1024 x 4096  M = 32            234 -> 15.5
-//   8192^2       M = 512 / 2048    773 / 3021 -> 359 / 1309, 1.6e-6 -> 1.4e-6
-//   512^2        M = 9 / 128       31.7 / 35.1 -> 12.2 / 17.2
+//   4096^2       M = 9 / 64 / 512  231 / 242 / 244 -> 19.7 / 27.0 / 99.7, 1.2e-6 -> 1.2e-7 / 1.2e-7 / 2.7e-7
+//   1024 x 4096  M = 32            234 -> 15.0
+//   8192^2       M = 2048          3016 -> 1280, 1.6e-6 -> 5.7e-7
+//   512^2        M = 9 / 128       31.8 / 35.1 -> 12.3 / 17.4
 // ---------------------------------------------------------------------------
 constexpr int DK32 = 32;  // values of k per stage
-
-typedef __bf16 dbf2 __attribute__((ext_vector_type(2)));
-typedef float dfl2 __attribute__((ext_vector_type(2)));
-
-// two values' bf16 (nearest), value 0 in the low half; v keeps what is left
-__device__ __forceinline__ uint32_t dense_split2(float &v0, float &v1) {
-    const dfl2 f = {v0, v1};
-    const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, dbf2));
-    v0 -= __uint_as_float(b << 16);
-    v1 -= __uint_as_float(b & 0xffff0000u);
-    return b;
-}
 
 template <int WM, int WN, int TM, int TN>
 __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__restrict__ W, int64_t N, int64_t K,
@@ -698,13 +671,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
         }
     }
 
-    floatx16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+    // sums of the first pieces' products, and of the others, which are 2^-7 of them and
+    // less: a rounding at the size of the result an MFMA step instead of three to eight
+    floatx16 acc[TM][TN] = {}, low[TM][TN] = {};
     // operands of this k-step and the next: x pieces, weight pieces; the next one's weights
     constexpr int NA = 3 * TM, NB = 2 * TN, NM = 6 * TM * TN;
     uint4 xa[2][NA], wb[2][TN][3], raw[NB];
@@ -735,7 +704,8 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
 #pragma unroll
         for (int u = 0; u < NM; u++) {
             const int j = u % TN, i = u / TN % TM, p = u / TN / TM;
-            acc[i][j] = dense_mfma<true>(xa[r][PR[p] * TM + i], wb[r][j][PW[p]], acc[i][j]);
+            floatx16 &to = p ? low[i][j] : acc[i][j];
+            to = dense_mfma(xa[r][PR[p] * TM + i], wb[r][j][PW[p]], to);
             if (u < H) {
 #pragma unroll
                 for (int q = u * (NA + NB) / H; q < (u + 1) * (NA + NB) / H; q++) read(buf, ks, r ^ 1, q);
@@ -767,6 +737,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
         stage(s + 1, 1);
     }
     __builtin_amdgcn_s_waitcnt(0);  // the loads past the slice
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] += low[i][j];
     float *y = out + (int64_t)z * g.split_stride;
     if constexpr (TM * TN >= 4) {
 #pragma unroll
@@ -794,13 +768,12 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
         }
 }
 
-// y[m][n] = 2^e_m * (sum over the slices, in order); blockIdx.y: row m.  BF: no exponent
+// y[m][n] = sum over the slices, in order; blockIdx.y: row m
 template <bool BF, bool W32 = false>
 __global__ __launch_bounds__(256) void k_dense_sum(const float *__restrict__ part, int S, int64_t M, int64_t N,
-                                                   const int *__restrict__ erow, const float *__restrict__ x,
-                                                   const uint8_t *__restrict__ W, int64_t K, float *__restrict__ y) {
+                                                   const float *__restrict__ x, const uint8_t *__restrict__ W, int64_t K,
+                                                   float *__restrict__ y) {
     const int64_t m = blockIdx.y, st = M * N;
-    const int e = BF ? 0 : erow[m];
     const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (n >= N) return;
     const float *p = part + m * N + n;
@@ -822,7 +795,7 @@ __global__ __launch_bounds__(256) void k_dense_sum(const float *__restrict__ par
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         if (n + i >= N) break;
-        float r = BF ? s[i] : __builtin_amdgcn_ldexpf(s[i], e);
+        float r = s[i];
         if (!dense_finite(r)) r = dense_dot<BF, W32>(x + m * K, W + (n + i) * K * (W32 ? 4 : 2), K);
         y[m * N + n + i] = r;
     }
@@ -832,20 +805,19 @@ namespace {
 struct DensePlan {
     int bm, bn;
     DenseGrid g;
-    size_t a_off, e_off, part_off, total;
+    size_t a_off, part_off, total;
 };
-// Tile by m (32, 64, 128 rows; 128 x 256 for F16 and F32 where such tiles fill the chip
-// by themselves), then k split until the resident workgroups (LDS: three of the 32-row
-// tiles a CU, two of the 64-row, one of the 128-row) are there, at least 256 values of
-// k a slice.
+// Tile by m (32, 64, 128 rows; 128 x 256 where such tiles fill the chip by themselves:
+// BF16 8192^2 M = 2048 945 -> 622 us, 14336x4096 M = 512 158 -> 143), then k split until the
+// resident workgroups (three of the 32-row tiles a CU, two of the 64-row, one of the
+// 128-row) are there, at least 256 values of k a slice.
 DensePlan dense_plan(int type, int64_t n, int64_t k, int64_t m) {
     DensePlan p;
-    const int P = type == TYPE_F16 ? 2 : 3;
     const bool w32 = type == TYPE_F32;
     p.bm = m <= 32 ? 32 : m <= 64 ? 64 : 128;
     p.bn = 128;
     const int64_t cus = num_cus();
-    if (p.bm == 128 && (P == 2 || w32) && ((m + 127) / 128) * ((n + 255) / 256) * 4 >= 3 * cus) p.bn = 256;
+    if (p.bm == 128 && ((m + 127) / 128) * ((n + 255) / 256) * 4 >= 3 * cus) p.bn = 256;
     p.g.tiles_m = (int)((m + p.bm - 1) / p.bm);
     p.g.tiles_n = (int)((n + p.bn - 1) / p.bn);
     p.g.rows = (int64_t)p.g.tiles_m * p.bm;
@@ -858,8 +830,7 @@ DensePlan dense_plan(int type, int64_t n, int64_t k, int64_t m) {
     p.g.split_stride = p.g.splits > 1 ? m * n : 0;
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     p.a_off = 0;
-    p.e_off = up((size_t)P * (size_t)p.g.rows * (size_t)p.g.Kp * 2);
-    p.part_off = p.e_off + up((size_t)m * 4);
+    p.part_off = up((size_t)3 * (size_t)p.g.rows * (size_t)p.g.Kp * 2);
     p.total = p.part_off + (p.g.splits > 1 ? up((size_t)p.g.splits * (size_t)(m * n) * 4) : 0);
     return p;
 }
@@ -871,40 +842,34 @@ size_t dense_workspace_bytes(int type, int64_t n, int64_t k, int64_t m) {
     return dense_plan(type, n, k, m).total;
 }
 
-template <bool BF>
 static hipError_t dense_pieces(int type, const uint8_t *w, int64_t n, int64_t k, const float *x, int64_t m, float *y,
                                uint8_t *ws, hipStream_t st) {
     const DensePlan p = dense_plan(type, n, k, m);
     unsigned short *a = reinterpret_cast<unsigned short *>(ws + p.a_off);
-    int *e = reinterpret_cast<int *>(ws + p.e_off);
     float *out = p.g.splits > 1 ? reinterpret_cast<float *>(ws + p.part_off) : y;
-    k_dense_pieces<BF><<<(unsigned)m, 256, 0, st>>>(x, k, p.g.Kp, p.g.rows, a, e);
+    k_dense_pieces<<<(unsigned)m, 256, 0, st>>>(x, k, p.g.Kp, p.g.rows, a);
     const unsigned grid = (unsigned)(p.g.tiles_m * p.g.tiles_n * p.g.splits);
-    constexpr int P = BF ? 3 : 2;
-    if (p.bm == 32) k_dense_mm<BF, P, 1, 4, 1, 1><<<grid, 256, 0, st>>>(w, n, k, a, e, x, m, out, p.g);
-    else if (p.bm == 64) k_dense_mm<BF, P, 2, 4, 1, 1><<<grid, 512, 0, st>>>(w, n, k, a, e, x, m, out, p.g);
-    else if (p.bn == 128) k_dense_mm<BF, P, 4, 2, 1, 2><<<grid, 512, 0, st>>>(w, n, k, a, e, x, m, out, p.g);
-    else if constexpr (!BF) k_dense_mm<BF, P, 2, 4, 2, 2><<<grid, 512, 0, st>>>(w, n, k, a, e, x, m, out, p.g);
-    if (p.g.splits > 1)
-        k_dense_sum<BF><<<dim3((unsigned)((n + 1023) / 1024), (unsigned)m), 256, 0, st>>>(out, p.g.splits, m, n, e, x, w,
-                                                                                        k, y);
-    return hipGetLastError();
-}
-
-static hipError_t dense_pieces32(const uint8_t *w, int64_t n, int64_t k, const float *x, int64_t m, float *y, uint8_t *ws,
-                                 hipStream_t st) {
-    const DensePlan p = dense_plan(TYPE_F32, n, k, m);
-    unsigned short *a = reinterpret_cast<unsigned short *>(ws + p.a_off);
-    float *out = p.g.splits > 1 ? reinterpret_cast<float *>(ws + p.part_off) : y;
-    k_dense_pieces<true><<<(unsigned)m, 256, 0, st>>>(x, k, p.g.Kp, p.g.rows, a, nullptr);
-    const unsigned grid = (unsigned)(p.g.tiles_m * p.g.tiles_n * p.g.splits);
-    if (p.bm == 32) k_dense_mm32<1, 4, 1, 1><<<grid, 256, 0, st>>>(w, n, k, a, x, m, out, p.g);
-    else if (p.bm == 64) k_dense_mm32<2, 4, 1, 1><<<grid, 512, 0, st>>>(w, n, k, a, x, m, out, p.g);
-    else if (p.bn == 128) k_dense_mm32<2, 4, 2, 1><<<grid, 512, 0, st>>>(w, n, k, a, x, m, out, p.g);
-    else k_dense_mm32<2, 4, 2, 2><<<grid, 512, 0, st>>>(w, n, k, a, x, m, out, p.g);
-    if (p.g.splits > 1)
-        k_dense_sum<true, true><<<dim3((unsigned)((n + 1023) / 1024), (unsigned)m), 256, 0, st>>>(out, p.g.splits, m, n,
-                                                                                                nullptr, x, w, k, y);
+    auto go = [&](auto kern, int threads) { kern<<<grid, threads, 0, st>>>(w, n, k, a, x, m, out, p.g); };
+    const dim3 sg((unsigned)((n + 1023) / 1024), (unsigned)m);
+    if (type == TYPE_F32) {
+        if (p.bm == 32) go(k_dense_mm32<1, 4, 1, 1>, 256);
+        else if (p.bm == 64) go(k_dense_mm32<2, 4, 1, 1>, 512);
+        else if (p.bn == 128) go(k_dense_mm32<2, 4, 2, 1>, 512);
+        else go(k_dense_mm32<2, 4, 2, 2>, 512);
+        if (p.g.splits > 1) k_dense_sum<true, true><<<sg, 256, 0, st>>>(out, p.g.splits, m, n, x, w, k, y);
+    } else if (type == TYPE_F16) {
+        if (p.bm == 32) go(k_dense_mm<false, 1, 4, 1, 1>, 256);
+        else if (p.bm == 64) go(k_dense_mm<false, 2, 4, 1, 1>, 512);
+        else if (p.bn == 128) go(k_dense_mm<false, 2, 4, 2, 1>, 512);
+        else go(k_dense_mm<false, 2, 4, 2, 2>, 512);
+        if (p.g.splits > 1) k_dense_sum<false><<<sg, 256, 0, st>>>(out, p.g.splits, m, n, x, w, k, y);
+    } else {
+        if (p.bm == 32) go(k_dense_mm<true, 1, 4, 1, 1>, 256);
+        else if (p.bm == 64) go(k_dense_mm<true, 2, 4, 1, 1>, 512);
+        else if (p.bn == 128) go(k_dense_mm<true, 4, 2, 1, 2>, 512);
+        else go(k_dense_mm<true, 2, 4, 2, 2>, 512);
+        if (p.g.splits > 1) k_dense_sum<true><<<sg, 256, 0, st>>>(out, p.g.splits, m, n, x, w, k, y);
+    }
     return hipGetLastError();
 }
 
@@ -935,11 +900,8 @@ static hipError_t dense_typed(const uint8_t *w, int64_t n, int64_t k, const floa
 hipError_t launch_dense(int type, const uint8_t *w, int64_t n, int64_t k, const float *x, int64_t m, float *y,
                         void *ws, hipStream_t st) {
     if (k % 8 || m > 65535LL * DBM) return hipErrorInvalidValue;
-    if (ws && dense_workspace_bytes(type, n, k, m) && type == TYPE_F32)
-        return dense_pieces32(w, n, k, x, m, y, static_cast<uint8_t *>(ws), st);
     if (ws && dense_workspace_bytes(type, n, k, m))
-        return type == TYPE_BF16 ? dense_pieces<true>(type, w, n, k, x, m, y, static_cast<uint8_t *>(ws), st)
-                                 : dense_pieces<false>(type, w, n, k, x, m, y, static_cast<uint8_t *>(ws), st);
+        return dense_pieces(type, w, n, k, x, m, y, static_cast<uint8_t *>(ws), st);
     if (type == TYPE_F16) return dense_typed<true>(w, n, k, x, m, y, st);
     if (type == TYPE_F32) return dense_typed<false>(w, n, k, x, m, y, st);
     if (type == TYPE_BF16) return dense_typed<true, true>(w, n, k, x, m, y, st);

@@ -156,3 +156,29 @@ def test_dense_mm_noalloc_beyond_scratch(lbq, dev, t):
     assert lbq.lbq_qmatmul_f32_noalloc(context(dev), qm._handle, xd.data_ptr(), m, y.data_ptr(), st) == 0
     # k/2 sums of two products, one after the other
     _assert_rows(y.cpu().numpy(), x.astype(np.float64) @ w.T, 2.0 ** -23 * (k / 2) ** 0.5)
+
+
+def _assert_outputs(y, x, w, k):
+    """Each output by itself, against the sum of its own products' sizes: eight sums an MFMA
+    of 16 k-values at most, errors of independent sign, taken twice (as _bound)."""
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    err, size = np.abs(y - x @ w.T), np.abs(x) @ np.abs(w).T
+    bound = 2.0 ** -23 * max(4.0, (8 * k / 16) ** 0.5)
+    assert (err <= bound * size).all(), (err / size).max() / bound
+
+
+@pytest.mark.parametrize("t", [F16, BF16, F32])
+@pytest.mark.parametrize("m,n,k", [(9, 130, 256), (64, 127, 2048), (300, 300, 512), (700, 8200, 200)])
+@pytest.mark.parametrize("big", [1e6, 1e9, 1e20, 1e30])
+def test_dense_mm_range_within_rows(lbq, dev, t, m, n, k, big):
+    # one large value a row whose weights are zero: the row's other products are the result
+    rng = np.random.default_rng(m + n + k)
+    w = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    w[:, [3, k // 2]] = 0
+    qm, w = _weight(t, n, k, rng, dev, w)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[:, 3] = big * np.where(np.arange(m) % 2, 1, -1)
+    x[::3, 3], x[::3, k // 2] = 0, big
+    y = qm.forward(to_dev(x, dev)).cpu().numpy()
+    x[:, [3, k // 2]] = 0
+    _assert_outputs(y, x, w, k)
