@@ -589,22 +589,22 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
 // m > 8 with F32 weights: x as the three bf16 pieces of k_dense_pieces (their sum
 // is x), and each weight as three bf16 pieces that a wave forms in registers from the
 // f32 value in LDS: hi = bf16(w), mid = bf16(w - hi), lo = w - hi - mid, rounded to
-// nearest, again exact.  Six of the nine products, all exact in the accumulator:
-// hi hi, hi mid, mid hi, mid mid, hi lo, lo hi.  The three left out are at most 2^-23
-// of |x w| together and of either sign.  As k_dense_mm otherwise (tiles, two LDS buffers
+// nearest, again exact.  Eight of the nine products, all exact in the accumulator; the
+// ninth, lo lo, is below 2^-32 of |x w| (|lo| < 2^-15 |x|, <= 2^-17 |w|), a 256th of the
+// rounding of one f32 product.  As k_dense_mm otherwise (tiles, two LDS buffers
 // filled by loads to LDS, one barrier a stage), with stages of 32 values of k: a
 // weight row is 128 B of a stage, its 16-byte chunk c in slot c ^ ((r >> 1) & 7); a
 // piece's row is 64 B, two rows a line, chunk c of row r in slot
 // (c ^ ((r >> 2) & 3)) + 4 (r & 1), so operand reads meet no bank twice.
 // The split costs about 5.5 vector instructions a weight: under the MFMAs of TM tiles
-// (192 TM clocks against 176), so waves take two row tiles where m has them.
-// Bound by the matrix cores from M = 200 (1.0-1.3 PFLOP/s of operand products), by the
+// (256 TM clocks against 176), so waves take two row tiles where m has them.
+// Bound by the matrix cores from M = 200 (1.0-1.4 PFLOP/s of operand products), by the
 // weights' bytes and the launches below.  Against k_dense_gemm, us per call and relative
 // error against 64 bits:
-//   4096^2       M = 9 / 64 / 512  231 / 242 / 244 -> 19.7 / 27.0 / 99.7, 1.2e-6 -> 1.2e-7 / 1.2e-7 / 2.7e-7
-//   1024 x 4096  M = 32            234 -> 15.0
-//   8192^2       M = 2048          3016 -> 1280, 1.6e-6 -> 5.7e-7
-//   512^2        M = 9 / 128       31.8 / 35.1 -> 12.3 / 17.4
+//   4096^2       M = 9 / 64 / 512  231 / 242 / 244 -> 20.2 / 29.7 / 119, 1.2e-6 -> 1.2e-7 / 1.2e-7 / 2.7e-7
+//   1024 x 4096  M = 32            234 -> 15.6
+//   8192^2       M = 2048          3016 -> 1561, 1.6e-6 -> 5.7e-7
+//   512^2        M = 9 / 128       31.8 / 35.1 -> 12.4 / 19.0
 // ---------------------------------------------------------------------------
 constexpr int DK32 = 32;  // values of k per stage
 
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
     // less: a rounding at the size of the result an MFMA step instead of three to eight
     floatx16 acc[TM][TN] = {}, low[TM][TN] = {};
     // operands of this k-step and the next: x pieces, weight pieces; the next one's weights
-    constexpr int NA = 3 * TM, NB = 2 * TN, NM = 6 * TM * TN;
+    constexpr int NA = 3 * TM, NB = 2 * TN, NM = 8 * TM * TN;
     uint4 xa[2][NA], wb[2][TN][3], raw[NB];
     auto read = [&](int buf, int ks, int r, int q) __attribute__((always_inline)) {
         if (q < NB) raw[q] = *reinterpret_cast<const uint4 *>((buf ? Bs1 : Bs0) + (ob[2 * ks + (q & 1)] + (q >> 1) * 4096));
@@ -700,7 +700,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
     // the MFMAs of the k-step in xa[r], wb[r], each followed by its share of the next
     // one's reads (first half) or splits (second half)
     auto step = [&](int r, int buf, int ks) __attribute__((always_inline)) {
-        constexpr int H = NM / 2, PR[6] = {0, 0, 1, 1, 0, 2}, PW[6] = {0, 1, 0, 1, 2, 0};
+        constexpr int H = NM / 2, PR[8] = {0, 0, 1, 1, 0, 2, 1, 2}, PW[8] = {0, 1, 0, 1, 2, 0, 2, 1};
 #pragma unroll
         for (int u = 0; u < NM; u++) {
             const int j = u % TN, i = u / TN % TM, p = u / TN / TM;

@@ -182,3 +182,19 @@ def test_dense_mm_range_within_rows(lbq, dev, t, m, n, k, big):
     y = qm.forward(to_dev(x, dev)).cpu().numpy()
     x[:, [3, k // 2]] = 0
     _assert_outputs(y, x, w, k)
+
+
+def test_dense_mm_f32_products(lbq, dev):
+    # one product an output: within a rounding or two of the f32 product (half an ulp, 2^-24,
+    # for the first pieces' sum and again for its sum with the others; what is left out is
+    # 2^-32), values whose pieces are as large as they get
+    rng = np.random.default_rng(23)
+    m, n, k = 300, 300, 8
+    bits = lambda s: (0x3f800000 | 0xff7f | (rng.integers(0, 128, s) << 16)).astype(np.uint32).view(np.float32)
+    x, w = np.zeros((m, k), np.float32), np.zeros((n, k), np.float32)
+    x[:, 5], w[:, 5] = bits(m), bits(n)
+    w[:, 6] = rng.standard_normal(n)  # meets zeros
+    qm, wd = _weight(F32, n, k, rng, dev, w)
+    ref = x.astype(np.float64) @ wd.T
+    y = qm.forward(to_dev(x, dev)).cpu().numpy()
+    assert np.abs(y / ref - 1).max() <= 2.1 * 2.0 ** -24
