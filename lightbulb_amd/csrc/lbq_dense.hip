@@ -291,13 +291,17 @@ __global__ __launch_bounds__(256) void k_dense_gemm(const uint8_t *__restrict__ 
 // an f32 product's whatever the range of its row.  (Two fp16 operands for x at one
 // exponent a row took a third of the MFMAs, but lose what lies 2^-17 and more below the
 // row's largest |x|, which may well meet a zero weight.)
+// Range.  x, and an F32 weight, is taken times 2^24 (DENSE_UP), results times 2^-24 for
+// each: the last bit of the smallest f32, 2^-149, is then a normal bf16, so that nothing
+// is too small for its operands to add up to it.  What is too large for the factor
+// (2^104, results 2^80 with F32 weights) gives an infinity and is formed again (below).
 // Bound by the matrix cores from M = 512 (1.0-1.5 PFLOP/s of operand products), by the
 // launches below.  Against k_dense_gemm, us per call and relative error against 64 bits:
-//   F16 4096^2    M = 9 / 64 / 512   236 / 240 / 243 -> 16.6 / 26.7 / 90.9, 1.2e-6 -> 1.2e-7 / 1.2e-7 / 2.7e-7
-//   F16 8192^2    M = 2048           2976 -> 1110, 1.6e-6 -> 5.7e-7
-//   BF16 4096^2   M = 32 / 512       238 / 245 -> 17.3 / 58.7, 1.2e-6 -> 1.2e-7 / 2.7e-7
-//   BF16 8192^2   M = 2048           2980 -> 622,  1.6e-6 -> 5.7e-7
-//   F16 512^2     M = 9              32.1 -> 12.1, 4.1e-7 -> 9.5e-8
+//   F16 4096^2    M = 9 / 64 / 512   236 / 240 / 243 -> 16.2 / 25.9 / 91.9, 1.2e-6 -> 1.2e-7 / 1.2e-7 / 2.7e-7
+//   F16 8192^2    M = 2048           2976 -> 1144, 1.6e-6 -> 5.7e-7
+//   BF16 4096^2   M = 32 / 512       238 / 245 -> 17.1 / 58.1, 1.2e-6 -> 1.2e-7 / 2.7e-7
+//   BF16 8192^2   M = 2048           2980 -> 654,  1.6e-6 -> 5.7e-7
+//   F16 512^2     M = 9              32.1 -> 12.6, 4.1e-7 -> 9.1e-8
 //
 // Tiles.  A workgroup of WM x WN waves owns BM = 32 WM TM rows of x and
 // BN = 32 WN TN weight rows; a wave its TM x TN tiles of 32 x 32.  k advances in
@@ -316,6 +320,9 @@ __global__ __launch_bounds__(256) void k_dense_gemm(const uint8_t *__restrict__ 
 // (dense_dot): an infinity in x or W would otherwise meet the zero pieces.
 // ---------------------------------------------------------------------------
 constexpr int DK = 64;  // values of k per stage
+constexpr float DENSE_UP = 0x1p24f;
+template <bool W32>
+constexpr float dense_down() { return W32 ? 0x1p-48f : 0x1p-24f; }
 
 typedef __bf16 dbf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 dbf2 __attribute__((ext_vector_type(2)));
@@ -357,6 +364,7 @@ template <bool BF, bool W32>
 __device__ __forceinline__ void dense_store(floatx16 &acc, float *y, int64_t mt, int64_t M, int64_t N, int64_t n, int h,
                                             bool last, const float *x, const uint8_t *W, int64_t K) {
     if (last) {
+        acc *= dense_down<W32>();
         float z = 0.f;
 #pragma unroll
         for (int v = 0; v < 16; v++) z = fmaf(acc[v], 0.f, z);
@@ -371,8 +379,8 @@ __device__ __forceinline__ void dense_store(floatx16 &acc, float *y, int64_t mt,
     store_tile(y + mt * N, M - mt, N, n, h, [&](int v) __attribute__((always_inline)) { return acc[v]; });
 }
 
-// x [M][K] -> pieces [3][rows][Kp] (Kp = K up to a multiple of DK, zero filled); one
-// workgroup per row of x
+// x [M][K] -> pieces [3][rows][Kp] of 2^24 x (Kp = K up to a multiple of DK, zero filled);
+// one workgroup per row of x
 __global__ __launch_bounds__(256) void k_dense_pieces(const float *__restrict__ x, int64_t K, int64_t Kp, int64_t rows,
                                                       unsigned short *__restrict__ A) {
     const int64_t m = blockIdx.x;
@@ -387,6 +395,7 @@ __global__ __launch_bounds__(256) void k_dense_pieces(const float *__restrict__ 
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             uint32_t b[3];
+            v[i] *= DENSE_UP;
             const uint32_t u0 = __float_as_uint(v[i]);
             const bool fin = dense_finite(v[i]);
             // a NaN keeps a mantissa bit in the upper half
@@ -579,7 +588,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
                 const int64_t m = m0 + 32 * (wm * TM + i) + 8 * (v >> 2) + 4 * h + (v & 3);
                 if (m >= M || n >= N) continue;
                 float r = acc[i][j][v];
-                if (g.split_stride == 0 && !dense_finite(r)) r = dense_dot<BF>(x + m * K, W + n * K * 2, K);
+                if (g.split_stride == 0) {
+                    r *= dense_down<false>();
+                    if (!dense_finite(r)) r = dense_dot<BF>(x + m * K, W + n * K * 2, K);
+                }
                 y[m * N + n] = r;
             }
         }
@@ -596,15 +608,15 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
 // weight row is 128 B of a stage, its 16-byte chunk c in slot c ^ ((r >> 1) & 7); a
 // piece's row is 64 B, two rows a line, chunk c of row r in slot
 // (c ^ ((r >> 2) & 3)) + 4 (r & 1), so operand reads meet no bank twice.
-// The split costs about 5.5 vector instructions a weight: under the MFMAs of TM tiles
-// (256 TM clocks against 176), so waves take two row tiles where m has them.
+// The split costs about 6.5 vector instructions a weight: under the MFMAs of TM tiles
+// (256 TM clocks against 208), so waves take two row tiles where m has them.
 // Bound by the matrix cores from M = 200 (1.0-1.4 PFLOP/s of operand products), by the
 // weights' bytes and the launches below.  Against k_dense_gemm, us per call and relative
 // error against 64 bits:
-//   4096^2       M = 9 / 64 / 512  231 / 242 / 244 -> 20.2 / 29.7 / 119, 1.2e-6 -> 1.2e-7 / 1.2e-7 / 2.7e-7
-//   1024 x 4096  M = 32            234 -> 15.6
-//   8192^2       M = 2048          3016 -> 1561, 1.6e-6 -> 5.7e-7
-//   512^2        M = 9 / 128       31.8 / 35.1 -> 12.4 / 19.0
+//   4096^2       M = 9 / 64 / 512  231 / 242 / 244 -> 20.3 / 29.7 / 121, 1.2e-6 -> 1.2e-7 / 1.2e-7 / 2.7e-7
+//   1024 x 4096  M = 32            234 -> 15.4
+//   8192^2       M = 2048          3016 -> 1650, 1.6e-6 -> 5.7e-7
+//   512^2        M = 9 / 128       31.8 / 35.1 -> 12.5 / 18.9
 // ---------------------------------------------------------------------------
 constexpr int DK32 = 32;  // values of k per stage
 
@@ -687,7 +699,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
     auto split = [&](int r, int c) __attribute__((always_inline)) {
         const int j = c >> 2, e = c & 3;
         const uint4 v = raw[2 * j + (e >> 1)];
-        float v0 = __uint_as_float(e & 1 ? v.z : v.x), v1 = __uint_as_float(e & 1 ? v.w : v.y);
+        float v0 = __uint_as_float(e & 1 ? v.z : v.x) * DENSE_UP, v1 = __uint_as_float(e & 1 ? v.w : v.y) * DENSE_UP;
 #pragma unroll
         for (int p = 0; p < 3; p++) {
             const uint32_t b = dense_split2(v0, v1);
@@ -762,7 +774,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
                 const int64_t m = m0 + 32 * (wm * TM + i) + 8 * (v >> 2) + 4 * h + (v & 3);
                 if (m >= M || n >= N) continue;
                 float r = acc[i][j][v];
-                if (g.split_stride == 0 && !dense_finite(r)) r = dense_dot<true, true>(x + m * K, W + n * K * 4, K);
+                if (g.split_stride == 0) {
+                    r *= dense_down<true>();
+                    if (!dense_finite(r)) r = dense_dot<true, true>(x + m * K, W + n * K * 4, K);
+                }
                 y[m * N + n] = r;
             }
         }
@@ -795,7 +810,7 @@ __global__ __launch_bounds__(256) void k_dense_sum(const float *__restrict__ par
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         if (n + i >= N) break;
-        float r = s[i];
+        float r = s[i] * dense_down<W32>();
         if (!dense_finite(r)) r = dense_dot<BF, W32>(x + m * K, W + (n + i) * K * (W32 ? 4 : 2), K);
         y[m * N + n + i] = r;
     }

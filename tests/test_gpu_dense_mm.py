@@ -198,3 +198,22 @@ def test_dense_mm_f32_products(lbq, dev):
     ref = x.astype(np.float64) @ wd.T
     y = qm.forward(to_dev(x, dev)).cpu().numpy()
     assert np.abs(y / ref - 1).max() <= 2.1 * 2.0 ** -24
+
+
+_SIZES = [(1e-36, 1.0), (1e-36, 1e4), (1e-42, 1e4), (1e-36, 1e20), (1e20, 1e-36), (1e30, 1e-42), (1e30, 1.0), (1e36, 1e-3)]
+
+
+@pytest.mark.parametrize("m,n,k", [(9, 130, 256), (64, 127, 2048), (300, 300, 512), (700, 8200, 200)])
+@pytest.mark.parametrize("t,xs,ws", [(t, xs, ws) for t in (F16, BF16, F32) for xs, ws in _SIZES
+                                     if t == F32 or ws in (1.0, 1e4) or (t == BF16 and ws >= 1e-3)])
+def test_dense_mm_small_and_large_values(lbq, dev, t, m, n, k, xs, ws):
+    # down to f32's last bit and up to its largest, on either side
+    rng = np.random.default_rng(m + k)
+    qm, w = _weight(t, n, k, rng, dev, (rng.standard_normal((n, k)) * ws).astype(np.float32))
+    x = (rng.standard_normal((m, k)) * xs).astype(np.float32)
+    y = qm.forward(to_dev(x, dev)).cpu().numpy()
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    size = np.abs(x) @ np.abs(w).T
+    # a result below the normal range has f32's fixed spacing there, 2^-149
+    bound = np.maximum(2.0 ** -23 * max(4.0, (8 * k / 16) ** 0.5) * size, 2.0 ** -149)
+    assert (np.abs(y - x @ w.T) <= bound).all()
