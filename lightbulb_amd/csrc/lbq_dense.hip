@@ -316,8 +316,10 @@ __global__ __launch_bounds__(256) void k_dense_gemm(const uint8_t *__restrict__ 
 // Few tiles: k is split over workgroups whose partial sums k_dense_sum adds in
 // slice order.
 //
-// A result that is not finite is formed again from x and W by f32 FMAs in k order
-// (dense_dot): an infinity in x or W would otherwise meet the zero pieces.
+// A result that is not finite is formed again from x and W on the f32 matrix cores
+// (dense_tile): an infinity in x or W would otherwise meet the zero pieces.  A wave does
+// that once for a 32 x 32 tile, so that a batch of nothing but NaN costs one such pass
+// (F16 4096^2 M = 512 0.33 ms, k_dense_gemm 0.26), and a finite result keeps its bits whatever stands beside it.
 // ---------------------------------------------------------------------------
 constexpr int DK = 64;  // values of k per stage
 constexpr float DENSE_UP = 0x1p24f;
@@ -343,40 +345,61 @@ __device__ __forceinline__ uint32_t dense_split2(float &v0, float &v1) {
 
 __device__ __forceinline__ bool dense_finite(float v) { return fabsf(v) <= 3.4028234664e38f; }  // false for NaN
 
-template <bool BF, bool W32 = false>
-__device__ __attribute__((noinline)) float dense_dot(const float *x, const uint8_t *w, int64_t K) {
-    float s = 0.f;
-    for (int64_t i = 0; i < K; i++) {
-        float v;
-        if constexpr (W32) v = reinterpret_cast<const float *>(w)[i];
-        else v = w16<BF>(reinterpret_cast<const unsigned short *>(w)[i]);
-        s = fmaf(v, x[i], s);
-    }
-    return s;
-}
-
-// One 32 x 32 tile from row mt on (store_tile).  last: these are results, not partial
-// sums, and one that is not finite is formed again; 0 * r summed over the lane's sixteen
-// is a NaN if any of them is.  For the 128 x 256 tiles, with 64 stores a lane (F16 8192^2
-// M = 2048 511 -> 499 us, 14336x4096 M = 512 124 -> 119); the smaller tiles' few stores
-// gain nothing by it (1000^3 23.7 -> 24.5).
+// The f32 products of x rows mt .. mt + 31 and this lane's weight row n (l % 32 of the
+// tile), in the layout of the accumulators; the whole wave calls it.  A lane takes four
+// values of k at a time, its half h those from 8 i + 4 h.
 template <bool BF, bool W32>
-__device__ __forceinline__ void dense_store(floatx16 &acc, float *y, int64_t mt, int64_t M, int64_t N, int64_t n, int h,
-                                            bool last, const float *x, const uint8_t *W, int64_t K) {
-    if (last) {
-        acc *= dense_down<W32>();
-        float z = 0.f;
+__device__ __attribute__((noinline)) floatx16 dense_tile(const float *x, const uint8_t *W, int64_t K, int64_t M, int64_t N,
+                                                         int64_t mt, int64_t n) {
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int64_t m = mt + (lane & 31);
+    const uintptr_t xr = reinterpret_cast<uintptr_t>(x + (m < M ? m : M - 1) * K + 4 * h);
+    const uint8_t *wr = W + ((n < N ? n : N - 1) * K + 4 * h) * (W32 ? 4 : 2);
+    floatx16 acc = {};
+    for (int64_t k0 = 0; k0 < K; k0 += 32) {  // four loads of each in flight
+        float a[4][4], w[4][4];
 #pragma unroll
-        for (int v = 0; v < 16; v++) z = fmaf(acc[v], 0.f, z);
-        if (z != 0.f) {
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int64_t m = mt + 8 * (v >> 2) + 4 * h + (v & 3);
-                if (m < M && n < N && !dense_finite(acc[v])) acc[v] = dense_dot<BF, W32>(x + m * K, W + n * K * (W32 ? 4 : 2), K);
+        for (int u = 0; u < 4; u++) {
+            const int64_t k = k0 + 8 * u < K ? k0 + 8 * u : 0;
+            const u32x4a4 v = gld16(reinterpret_cast<gbytes_c>(xr + 4 * k));
+            a[u][0] = __uint_as_float(v.x); a[u][1] = __uint_as_float(v.y);
+            a[u][2] = __uint_as_float(v.z); a[u][3] = __uint_as_float(v.w);
+            if constexpr (W32) {
+                const float4 b = *reinterpret_cast<const float4 *>(wr + 4 * k);
+                w[u][0] = b.x; w[u][1] = b.y; w[u][2] = b.z; w[u][3] = b.w;
+            } else {
+                const uint2 b = *reinterpret_cast<const uint2 *>(wr + 2 * k);
+                w[u][0] = w16<BF>(b.x & 0xffffu); w[u][1] = w16<BF>(b.x >> 16);
+                w[u][2] = w16<BF>(b.y & 0xffffu); w[u][3] = w16<BF>(b.y >> 16);
             }
         }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (k0 + 8 * u < K)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][i], w[u][i], acc, 0, 0, 0);
     }
-    store_tile(y + mt * N, M - mt, N, n, h, [&](int v) __attribute__((always_inline)) { return acc[v]; });
+    return acc;
+}
+
+// One 32 x 32 tile of results from row mt on: without the operands' factor, and those that
+// are not finite formed again.  0 * r summed over the lane's sixteen is a NaN if any of
+// them is not finite, of rows past M too.
+template <bool BF, bool W32>
+__device__ __forceinline__ void dense_results(floatx16 &acc, int64_t mt, int64_t M, int64_t N, int64_t n, int h, const float *x,
+                                              const uint8_t *W, int64_t K) {
+    acc *= dense_down<W32>();
+    float z = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; v++) z = fmaf(acc[v], 0.f, z);
+    if (!__any(z != 0.f)) return;
+    bool bad = false;
+#pragma unroll
+    for (int v = 0; v < 16; v++) bad = bad || (mt + 8 * (v >> 2) + 4 * h + (v & 3) < M && n < N && !dense_finite(acc[v]));
+    if (!__any(bad)) return;
+    const floatx16 f = dense_tile<BF, W32>(x, W, K, M, N, mt, n);
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = dense_finite(acc[v]) ? acc[v] : f[v];
 }
 
 // x [M][K] -> pieces [3][rows][Kp] of 2^24 x (Kp = K up to a multiple of DK, zero filled);
@@ -568,31 +591,20 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm(const uint8_t *__rest
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] += low[i][j];
     float *y = out + (int64_t)z * g.split_stride;
-    if constexpr (TM * TN >= 4) {
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++)
-                dense_store<BF, false>(acc[i][j], y, m0 + 32 * (wm * TM + i), M, N, n0 + 32 * (wn * TN + j) + lr, h,
-                                       g.split_stride == 0, x, W, K);
-        return;
-    }
-    // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            const int64_t n = n0 + 32 * (wn * TN + j) + lr;
+            const int64_t mt = m0 + 32 * (wm * TM + i), n = n0 + 32 * (wn * TN + j) + lr;
+            if (g.split_stride == 0) dense_results<BF, false>(acc[i][j], mt, M, N, n, h, x, W, K);
+            if constexpr (TM * TN >= 4) {
+                store_tile(y + mt * N, M - mt, N, n, h, [&](int v) __attribute__((always_inline)) { return acc[i][j][v]; });
+            } else {  // (few stores, and partial sums that are read back: plain ones)
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int64_t m = m0 + 32 * (wm * TM + i) + 8 * (v >> 2) + 4 * h + (v & 3);
-                if (m >= M || n >= N) continue;
-                float r = acc[i][j][v];
-                if (g.split_stride == 0) {
-                    r *= dense_down<false>();
-                    if (!dense_finite(r)) r = dense_dot<BF>(x + m * K, W + n * K * 2, K);
+                for (int v = 0; v < 16; v++) {
+                    const int64_t m = mt + 8 * (v >> 2) + 4 * h + (v & 3);
+                    if (m < M && n < N) y[m * N + n] = acc[i][j][v];
                 }
-                y[m * N + n] = r;
             }
         }
 }
@@ -754,65 +766,75 @@ __global__ __launch_bounds__(64 * WM * WN) void k_dense_mm32(const uint8_t *__re
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] += low[i][j];
     float *y = out + (int64_t)z * g.split_stride;
-    if constexpr (TM * TN >= 4) {
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++)
-                dense_store<true, true>(acc[i][j], y, m0 + 32 * (wm * TM + i), M, N, n0 + 32 * (wn * TN + j) + lr, h,
-                                        g.split_stride == 0, x, W, K);
-        return;
-    }
-    // D layout of a 32 x 32 tile: lane holds column l%32, rows 8(v/4) + 4h + v%4
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            const int64_t n = n0 + 32 * (wn * TN + j) + lr;
+            const int64_t mt = m0 + 32 * (wm * TM + i), n = n0 + 32 * (wn * TN + j) + lr;
+            if (g.split_stride == 0) dense_results<true, true>(acc[i][j], mt, M, N, n, h, x, W, K);
+            if constexpr (TM * TN >= 4) {
+                store_tile(y + mt * N, M - mt, N, n, h, [&](int v) __attribute__((always_inline)) { return acc[i][j][v]; });
+            } else {  // (few stores, and partial sums that are read back: plain ones)
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int64_t m = m0 + 32 * (wm * TM + i) + 8 * (v >> 2) + 4 * h + (v & 3);
-                if (m >= M || n >= N) continue;
-                float r = acc[i][j][v];
-                if (g.split_stride == 0) {
-                    r *= dense_down<true>();
-                    if (!dense_finite(r)) r = dense_dot<true, true>(x + m * K, W + n * K * 4, K);
+                for (int v = 0; v < 16; v++) {
+                    const int64_t m = mt + 8 * (v >> 2) + 4 * h + (v & 3);
+                    if (m < M && n < N) y[m * N + n] = acc[i][j][v];
                 }
-                y[m * N + n] = r;
             }
         }
 }
 
-// y[m][n] = sum over the slices, in order; blockIdx.y: row m
-template <bool BF, bool W32 = false>
+// y[m][n] = the slices' sums added in order, without the operands' factor; a workgroup
+// takes 32 x 32 outputs, a wave eight rows of them, 16 bytes a lane.  What is not finite is
+// formed again by the first wave.
+template <bool BF, bool W32>
 __global__ __launch_bounds__(256) void k_dense_sum(const float *__restrict__ part, int S, int64_t M, int64_t N,
                                                    const float *__restrict__ x, const uint8_t *__restrict__ W, int64_t K,
                                                    float *__restrict__ y) {
-    const int64_t m = blockIdx.y, st = M * N;
-    const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (n >= N) return;
-    const float *p = part + m * N + n;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    if ((N & 3) == 0) {
-        for (int z0 = 0; z0 < S; z0 += 8) {
-            float4 v[8];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t mt = 32 * (int64_t)blockIdx.y, nt = 32 * (int64_t)blockIdx.x, st = M * N;
+    const int64_t m = mt + 8 * wave + (lane >> 3), n = nt + 4 * (lane & 7);
+    bool bad = false;
+    if (m < M && n < N) {
+        const float *p = part + m * N + n;
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+        if ((N & 3) == 0) {
+            for (int z0 = 0; z0 < S; z0 += 8) {
+                float4 v[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++)
-                if (z0 + j < S) v[j] = *reinterpret_cast<const float4 *>(p + (z0 + j) * st);
+                for (int j = 0; j < 8; j++)
+                    if (z0 + j < S) v[j] = *reinterpret_cast<const float4 *>(p + (z0 + j) * st);
 #pragma unroll
-            for (int j = 0; j < 8; j++)
-                if (z0 + j < S) { s[0] += v[j].x; s[1] += v[j].y; s[2] += v[j].z; s[3] += v[j].w; }
+                for (int j = 0; j < 8; j++)
+                    if (z0 + j < S) { s[0] += v[j].x; s[1] += v[j].y; s[2] += v[j].z; s[3] += v[j].w; }
+            }
+        } else {
+            for (int i = 0; i < 4 && n + i < N; i++)
+                for (int z = 0; z < S; z++) s[i] += p[z * st + i];
         }
-    } else {
-        for (int i = 0; i < 4 && n + i < N; i++)
-            for (int z = 0; z < S; z++) s[i] += p[z * st + i];
-    }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (n + i >= N) break;
-        float r = s[i] * dense_down<W32>();
-        if (!dense_finite(r)) r = dense_dot<BF, W32>(x + m * K, W + (n + i) * K * (W32 ? 4 : 2), K);
-        y[m * N + n + i] = r;
+        for (int i = 0; i < 4; i++) {
+            s[i] *= dense_down<W32>();
+            bad = bad || !dense_finite(s[i]);
+        }
+        float *o = y + m * N + n;
+        if ((N & 3) == 0 && !bad && (reinterpret_cast<uintptr_t>(y) & 15u) == 0) {
+            *reinterpret_cast<float4 *>(o) = make_float4(s[0], s[1], s[2], s[3]);
+        } else {
+            for (int i = 0; i < 4 && n + i < N; i++)
+                if (dense_finite(s[i])) o[i] = s[i];
+        }
+    }
+    if (!__syncthreads_or(bad) || wave) return;
+    const int64_t c = nt + (lane & 31);
+    const floatx16 f = dense_tile<BF, W32>(x, W, K, M, N, mt, c);
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        const int64_t r = mt + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+        if (r >= M || c >= N) continue;
+        float s = 0.f;
+        for (int z = 0; z < S; z++) s += part[z * st + r * N + c];
+        if (!dense_finite(s * dense_down<W32>())) y[r * N + c] = f[v];
     }
 }
 
@@ -865,7 +887,7 @@ static hipError_t dense_pieces(int type, const uint8_t *w, int64_t n, int64_t k,
     k_dense_pieces<<<(unsigned)m, 256, 0, st>>>(x, k, p.g.Kp, p.g.rows, a);
     const unsigned grid = (unsigned)(p.g.tiles_m * p.g.tiles_n * p.g.splits);
     auto go = [&](auto kern, int threads) { kern<<<grid, threads, 0, st>>>(w, n, k, a, x, m, out, p.g); };
-    const dim3 sg((unsigned)((n + 1023) / 1024), (unsigned)m);
+    const dim3 sg((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32));
     if (type == TYPE_F32) {
         if (p.bm == 32) go(k_dense_mm32<1, 4, 1, 1>, 256);
         else if (p.bm == 64) go(k_dense_mm32<2, 4, 1, 1>, 512);
@@ -877,13 +899,13 @@ static hipError_t dense_pieces(int type, const uint8_t *w, int64_t n, int64_t k,
         else if (p.bm == 64) go(k_dense_mm<false, 2, 4, 1, 1>, 512);
         else if (p.bn == 128) go(k_dense_mm<false, 2, 4, 2, 1>, 512);
         else go(k_dense_mm<false, 2, 4, 2, 2>, 512);
-        if (p.g.splits > 1) k_dense_sum<false><<<sg, 256, 0, st>>>(out, p.g.splits, m, n, x, w, k, y);
+        if (p.g.splits > 1) k_dense_sum<false, false><<<sg, 256, 0, st>>>(out, p.g.splits, m, n, x, w, k, y);
     } else {
         if (p.bm == 32) go(k_dense_mm<true, 1, 4, 1, 1>, 256);
         else if (p.bm == 64) go(k_dense_mm<true, 2, 4, 1, 1>, 512);
         else if (p.bn == 128) go(k_dense_mm<true, 4, 2, 1, 2>, 512);
         else go(k_dense_mm<true, 2, 4, 2, 2>, 512);
-        if (p.g.splits > 1) k_dense_sum<true><<<sg, 256, 0, st>>>(out, p.g.splits, m, n, x, w, k, y);
+        if (p.g.splits > 1) k_dense_sum<true, false><<<sg, 256, 0, st>>>(out, p.g.splits, m, n, x, w, k, y);
     }
     return hipGetLastError();
 }

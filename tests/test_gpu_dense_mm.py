@@ -217,3 +217,29 @@ def test_dense_mm_small_and_large_values(lbq, dev, t, m, n, k, xs, ws):
     # a result below the normal range has f32's fixed spacing there, 2^-149
     bound = np.maximum(2.0 ** -23 * max(4.0, (8 * k / 16) ** 0.5) * size, 2.0 ** -149)
     assert (np.abs(y - x @ w.T) <= bound).all()
+
+
+@pytest.mark.parametrize("t", [F16, BF16, F32])
+# one product a tile and slices of k; tiles of 32, 64, 128 rows and 128 x 256, short ones
+@pytest.mark.parametrize("m,n,k", [(20, 140, 64), (50, 70, 136), (40, 300, 2048), (300, 300, 1000), (1430, 4096, 72)])
+def test_dense_mm_nonfinite_batch(lbq, dev, t, m, n, k):
+    # x and W with NaN and infinities throughout; the finite outputs beside them keep their bits
+    rng = np.random.default_rng(29)
+    w = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    qm, wf = _weight(t, n, k, rng, dev, w)
+    clean = qm.forward(to_dev(x, dev)).cpu().numpy()
+    x2, w2 = x.copy(), w.copy()
+    x2[1::3, 7], x2[2::3, k - 1] = np.nan, np.inf
+    w2[3::5, 2], w2[:, k - 1] = -np.inf, np.where(np.arange(n) % 2, 0, w2[:, k - 1])
+    qm2, wd = _weight(t, n, k, rng, dev, w2)
+    with np.errstate(invalid="ignore"):
+        ref = (torch.from_numpy(x2).double() @ torch.from_numpy(wd).T).numpy()
+    y = qm2.forward(to_dev(x2, dev)).cpu().numpy()
+    fin = np.isfinite(ref)
+    assert np.array_equal(np.isnan(ref), np.isnan(y))
+    assert np.array_equal(ref[~fin & ~np.isnan(ref)], y[~fin & ~np.isnan(ref)])
+    same = fin & (np.arange(n) % 2 == 0)  # rows of W that did not change
+    assert np.array_equal(y[same], clean[same])
+    x2[:] = np.nan
+    assert np.isnan(qm2.forward(to_dev(x2, dev)).cpu().numpy()).all()
