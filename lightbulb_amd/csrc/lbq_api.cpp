@@ -36,18 +36,17 @@ struct lbq_ctx {
     uint8_t *noalloc_scratch;  // this device's `scratch`, from hipGetSymbolAddress
     lbq::Tuning tune;     // launch-plan overrides, read from the environment at lbq_init
     std::mutex mu;        // guards scratch growth
+    // Buffers that a larger one has replaced stay until the context goes: a captured graph
+    // may still use them.  Sizes double, so they add up to less than the ones in use.
+    std::vector<uint8_t *> outgrown;
     uint8_t *scratch;     // quantised activations (split layout)
     size_t scratch_bytes;
     uint8_t *ws;          // batched GEMM workspace (fp16 activations, split-k partials)
     size_t ws_bytes;
     uint8_t *tmp;         // gate and up outputs when their product is not fused
     size_t tmp_bytes;
-    // dense weights at m > 8: operand pieces and split-k partials.  Outgrown buffers
-    // stay until the context goes (their sizes double, so they add up to less than the
-    // current one): a captured graph may still use them.
-    uint8_t *dense_ws;
+    uint8_t *dense_ws;    // dense weights at m > 8: operand pieces and split-k partials
     size_t dense_ws_bytes;
-    std::vector<uint8_t *> dense_old;
     hipStream_t dense_stream;  // the last call's
     uint32_t *tile_counters;  // KS_COUNTERS zeroed words of the k-sliced GEMM (each launch leaves them zero)
 };
@@ -196,28 +195,39 @@ ActLayout act_layout(int act_type, int64_t m, int64_t k) {
     return L;
 }
 
-// Grows a context buffer to at least `bytes` (what: message tag).
-int ensure_buffer(uint8_t **buf, size_t *have, size_t bytes, const char *what) {
-    if (*have >= bytes) return LBQ_OK;
-    const size_t want = align_up(bytes > *have * 2 ? bytes : *have * 2, 1 << 20);
-    if (*buf) {
-        // in-flight kernels on any stream may still read the old buffer
-        hipError_t e = hipDeviceSynchronize();
-        if (e != hipSuccess) return hip_fail(e, "hipDeviceSynchronize");
-        (void)hipFree(*buf);
-        *buf = nullptr;
-        *have = 0;
+// Grows a context buffer to at least `bytes`; the one before stays (lbq_ctx::outgrown).
+// False where there is no memory: the buffer is as it was, and no message is left.
+bool grow_buffer(lbq_ctx *ctx, uint8_t **buf, size_t *have, size_t bytes) {
+    if (*have >= bytes) return true;
+    try {
+        ctx->outgrown.reserve(ctx->outgrown.size() + 1);
+    } catch (...) {
+        return false;
     }
+    size_t want = align_up(std::max(bytes, *have * 2), 1 << 20);
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, want);
-    if (e != hipSuccess) return fail(LBQ_ERR_OOM, "hipMalloc(%zu) for %s: %s", want, what, hipGetErrorString(e));
+    if (hipMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();
+        want = align_up(bytes, 1 << 20);
+        if (hipMalloc(&p, want) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    if (*buf) ctx->outgrown.push_back(*buf);
     *buf = static_cast<uint8_t *>(p);
     *have = want;
-    return LBQ_OK;
+    return true;
+}
+
+// The same as a status (what: message tag).
+int ensure_buffer(lbq_ctx *ctx, uint8_t **buf, size_t *have, size_t bytes, const char *what) {
+    if (grow_buffer(ctx, buf, have, bytes)) return LBQ_OK;
+    return fail(LBQ_ERR_OOM, "no %zu bytes of device memory for %s", bytes, what);
 }
 
 int ensure_scratch(lbq_ctx *ctx, size_t bytes) {
-    return ensure_buffer(&ctx->scratch, &ctx->scratch_bytes, bytes, "activation scratch");
+    return ensure_buffer(ctx, &ctx->scratch, &ctx->scratch_bytes, bytes, "activation scratch");
 }
 
 lbq::ActView view_of(uint8_t *base, const ActLayout &L, int64_t k) {
@@ -279,7 +289,7 @@ struct Scratch {
     }
     int ws(size_t bytes, uint8_t **out) {
         if (!fixed) {
-            const int s = ensure_buffer(&ctx->ws, &ctx->ws_bytes, bytes, "GEMM workspace");
+            const int s = ensure_buffer(ctx, &ctx->ws, &ctx->ws_bytes, bytes, "GEMM workspace");
             *out = ctx->ws;
             return s;
         }
@@ -416,22 +426,7 @@ uint8_t *dense_workspace(Scratch &sc, const lbq_weight *w, int64_t m, hipStream_
             (void)hipGetLastError();
             return nullptr;
         }
-        if (grow) {
-            const size_t want = align_up(std::max(need, 2 * c->dense_ws_bytes), 1 << 20);
-            void *p = nullptr;
-            try {
-                c->dense_old.reserve(c->dense_old.size() + 1);
-            } catch (...) {
-                return nullptr;
-            }
-            if (hipMalloc(&p, want) != hipSuccess) {
-                (void)hipGetLastError();
-                return nullptr;
-            }
-            if (c->dense_ws) c->dense_old.push_back(c->dense_ws);
-            c->dense_ws = static_cast<uint8_t *>(p);
-            c->dense_ws_bytes = want;
-        }
+        if (!grow_buffer(c, &c->dense_ws, &c->dense_ws_bytes, need)) return nullptr;
     }
     c->dense_stream = st;
     return c->dense_ws;
@@ -679,7 +674,7 @@ int lbq_ctx_destroy(lbq_ctx *ctx) {
     if (ctx->ws) (void)hipFree(ctx->ws);
     if (ctx->tmp) (void)hipFree(ctx->tmp);
     if (ctx->dense_ws) (void)hipFree(ctx->dense_ws);
-    for (uint8_t *p : ctx->dense_old) (void)hipFree(p);
+    for (uint8_t *p : ctx->outgrown) (void)hipFree(p);
     if (ctx->tile_counters) (void)hipFree(ctx->tile_counters);
     delete ctx;
     return LBQ_OK;
@@ -872,7 +867,7 @@ int group_f32(lbq_ctx *ctx, const lbq_weight *const *ws, int count, const float 
             wsb = std::max(wsb, mx[i] ? lbq::gemv_mx_workspace_bytes(w0->type, ws[i]->n, w0->k, (int)m)
                                       : lbq::gemm_workspace_bytes(w0->type, ws[i]->n, w0->k, m));
         }
-        int s = ensure_buffer(&ctx->ws, &ctx->ws_bytes, wsb, "GEMM workspace");
+        int s = ensure_buffer(ctx, &ctx->ws, &ctx->ws_bytes, wsb, "GEMM workspace");
         if (s) return s;
         bool in_kernel[LBQ_GROUP_MAX], all_in_kernel = true;
         for (int i = 0; i < count; i++) {
@@ -988,7 +983,7 @@ int gate_up_f32(lbq_ctx *ctx, const lbq_weight *w_gate, const lbq_weight *w_up, 
     if (m > 64 && !lbq::is_dense(w_gate->type) && lbq::gemm_pair_serves(w_gate->type, w_gate->n, w_gate->k, m)) {
         // one operand pre-pass, then both weights and the product in one launch
         std::lock_guard<std::mutex> lock(ctx->mu);
-        int s = ensure_buffer(&ctx->ws, &ctx->ws_bytes,
+        int s = ensure_buffer(ctx, &ctx->ws, &ctx->ws_bytes,
                               lbq::gemm_pair_workspace_bytes(w_gate->type, w_gate->n, w_gate->k, m), "GEMM workspace");
         if (s) return s;
         const int act_type = lbq::vec_dot_type(w_gate->type);
@@ -1014,7 +1009,7 @@ int gate_up_f32(lbq_ctx *ctx, const lbq_weight *w_gate, const lbq_weight *w_up, 
     const size_t half = ((size_t)m * (size_t)w_gate->n * sizeof(float) + 255) / 256 * 256;
     {
         std::lock_guard<std::mutex> lock(ctx->mu);
-        int s = ensure_buffer(&ctx->tmp, &ctx->tmp_bytes, 2 * half, "gate/up outputs");
+        int s = ensure_buffer(ctx, &ctx->tmp, &ctx->tmp_bytes, 2 * half, "gate/up outputs");
         if (s) return s;
     }
     float *gy = reinterpret_cast<float *>(ctx->tmp), *uy = reinterpret_cast<float *>(ctx->tmp + half);
@@ -1051,7 +1046,7 @@ int norm_into_tmp(lbq_ctx *ctx, const float *d_x, const float *d_w, float eps, i
     const size_t need = skip + (size_t)m * (size_t)k * sizeof(float);
     {
         std::lock_guard<std::mutex> lock(ctx->mu);
-        int s = ensure_buffer(&ctx->tmp, &ctx->tmp_bytes, need, "normalised activations");
+        int s = ensure_buffer(ctx, &ctx->tmp, &ctx->tmp_bytes, need, "normalised activations");
         if (s) return s;
     }
     *out = reinterpret_cast<float *>(ctx->tmp + skip);
