@@ -301,24 +301,18 @@ struct Scratch {
 
 // `bytes` of GEMM workspace for a path that has another to fall back on, or null: fixed
 // scratch that is too small, a stream under capture whose buffer would have to grow, or
-// no memory.  (The caller holds ctx->mu and has its activation scratch already.)
+// no memory.  (The caller holds ctx->mu, and has taken its activation scratch if it needs any.)
 uint8_t *optional_ws(Scratch &sc, size_t bytes, hipStream_t st) {
     if (!bytes) return nullptr;
-    if (sc.fixed) {
-        if (sc.act_used + bytes > sc.fixed_bytes) return nullptr;
-    } else if (sc.ctx->ws_bytes < bytes) {
+    if (sc.fixed) return sc.act_used + bytes <= sc.fixed_bytes ? sc.fixed + sc.act_used : nullptr;
+    if (sc.ctx->ws_bytes < bytes) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
             (void)hipGetLastError();
             return nullptr;
         }
     }
-    uint8_t *ws = nullptr;
-    if (sc.ws(bytes, &ws)) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    return ws;
+    return grow_buffer(sc.ctx, &sc.ctx->ws, &sc.ctx->ws_bytes, bytes) ? sc.ctx->ws : nullptr;
 }
 
 // Batch decode on the matrix cores for this weight and row count
