@@ -21,7 +21,9 @@
  *     [n][k / block_size] blocks, rows contiguous along k
  *     (GGUF ne0 = k; /root/reference/src/gguf/parser.rs:180-199).
  *   - A context owns per-device scratch (quantised activations, the batched
- *     GEMM's workspace, grown on demand, and 64 KiB of its tile counters).  Calls that share a context must be
+ *     GEMM's workspace, grown on demand, and 64 KiB of its tile counters).  A buffer
+ *     that has been outgrown stays until the context goes, for captured graphs that
+ *     use it.  Calls that share a context must be
  *     ordered on one stream (the reference runs every forward on one model
  *     thread, src/engine/model_runner.rs:236,383).  Weight handles are
  *     immutable and may be read concurrently.
@@ -160,10 +162,14 @@ int lbq_weight_info(const lbq_weight *w, uint32_t *ggml_type, int64_t *n, int64_
  * adds when y is plain device memory (hipMalloc; checked once per allocation),
  * else through partial sums in the workspace; either way y = a + b for the two
  * halves, the same bits for finite normal-range halves.  Dense F32/F16/BF16
- * weights are candle's dense variant: no quantisation, an f32 matmul (at
- * m > 8 x, and an F32 weight, as 16-bit operands that add up to it, x's in the context's scratch;
- * under a graph capture that would have to grow that scratch, the f32 matrix
- * cores).  m == 0 is a no-op. */
+ * weights are candle's dense variant: no quantisation, an f32 matmul.  At m > 8
+ * the 16-bit matrix cores form its products: x as three bf16 operands that add up
+ * to it (an F32 weight as three, an F16 weight as two), every product exact (F32: but
+ * for one part below 2^-32 of it), sums in f32.  The operands live in memory of the
+ * context, a buffer for each stream and for each graph capture, so dense calls
+ * need no order with calls on other streams; where there is none (no memory, more
+ * than 64 streams, captures that together would hold 1 GiB) the f32 matrix cores
+ * run instead.  m == 0 is a no-op. */
 int lbq_qmatmul_f32(lbq_ctx *ctx, const lbq_weight *w, const float *d_x, int64_t m, float *d_y, void *stream);
 
 /* lbq_qmatmul_f32's result (the same kernels, the same bits), allocating

@@ -45,9 +45,16 @@ struct lbq_ctx {
     size_t ws_bytes;
     uint8_t *tmp;         // gate and up outputs when their product is not fused
     size_t tmp_bytes;
-    uint8_t *dense_ws;    // dense weights at m > 8: operand pieces and split-k partials
-    size_t dense_ws_bytes;
-    hipStream_t dense_stream;  // the last call's
+    // dense weights at m > 8: operand pieces and split-k partials, a buffer for each stream and
+    // each (graph capture, stream) that calls (dense_workspace)
+    struct DenseBuffer {
+        hipStream_t stream;
+        bool captured;
+        unsigned long long capture;  // its id
+        uint8_t *p;
+        size_t bytes;
+    };
+    std::vector<DenseBuffer> dense;
     uint32_t *tile_counters;  // KS_COUNTERS zeroed words of the k-sliced GEMM (each launch leaves them zero)
 };
 
@@ -398,32 +405,57 @@ int run_dot(Scratch &sc, const lbq_weight *w, const lbq::ActView &av, int64_t m,
     return LBQ_OK;
 }
 
-// The operand workspace of a dense call, or null where the f32 kernel has to run
-// without one: types and m that have no such path, fixed scratch that is too small,
-// and a stream under capture whose buffer would have to be allocated.  The dense
-// path keeps its own buffer: a call on another stream than the last one's waits for
-// the device first, as the buffer may still be in use there.
+// This thread's allocations are allowed while it, or another thread, captures a graph
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~RelaxedCapture() {
+        if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+constexpr int DENSE_STREAMS = 64;
+constexpr size_t DENSE_CAPTURED_BYTES = (size_t)1 << 30;
+
+// The operand workspace of a dense call, or null where the f32 kernel has to run without
+// one: types and m that have no such path, fixed scratch that is too small, no memory.
+// A dense call needs no order with calls on other streams: each stream has its own buffer,
+// and each graph capture its own beside those, for the replays run beside eager calls and
+// other graphs.  Bounded: beyond DENSE_STREAMS streams, or DENSE_CAPTURED_BYTES for the
+// captures, which keep theirs until the context goes, null.  (The caller holds ctx->mu.)
 uint8_t *dense_workspace(Scratch &sc, const lbq_weight *w, int64_t m, hipStream_t st) {
     const size_t need = lbq::dense_workspace_bytes(w->type, w->n, w->k, m);
     if (!need) return nullptr;
     if (sc.fixed) return need <= sc.fixed_bytes ? sc.fixed : nullptr;
-    lbq_ctx *c = sc.ctx;
-    const bool grow = need > c->dense_ws_bytes, moved = c->dense_ws && st != c->dense_stream;
-    if (grow || moved) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        if (cap != hipStreamCaptureStatusNone) return grow ? nullptr : c->dense_ws;
-        if (moved && hipDeviceSynchronize() != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        if (!grow_buffer(c, &c->dense_ws, &c->dense_ws_bytes, need)) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(st, &cap, &id) != hipSuccess || cap == hipStreamCaptureStatusInvalidated) {
+        (void)hipGetLastError();
+        return nullptr;
     }
-    c->dense_stream = st;
-    return c->dense_ws;
+    const bool captured = cap == hipStreamCaptureStatusActive;
+    if (!captured) id = 0;
+    lbq_ctx *c = sc.ctx;
+    lbq_ctx::DenseBuffer *b = nullptr;
+    int streams = 0;
+    size_t held = 0;
+    for (auto &d : c->dense) {
+        if (d.stream == st && d.captured == captured && d.capture == id) b = &d;
+        if (d.captured) held += d.bytes;
+        else streams++;
+    }
+    if (b && b->bytes >= need) return b->p;
+    if (captured ? held + need > DENSE_CAPTURED_BYTES : !b && streams >= DENSE_STREAMS) return nullptr;
+    if (!b) {
+        try {
+            c->dense.push_back({st, captured, id, nullptr, 0});
+        } catch (...) {
+            return nullptr;
+        }
+        b = &c->dense.back();
+    }
+    RelaxedCapture relaxed;
+    return grow_buffer(c, &b->p, &b->bytes, need) ? b->p : nullptr;
 }
 
 // candle's dense variant: an f32 matmul, no activation quantisation.  `mu`: as forward's.
@@ -644,9 +676,6 @@ int lbq_init(int device, lbq_ctx **out_ctx) {
     c->ws_bytes = 0;
     c->tmp = nullptr;
     c->tmp_bytes = 0;
-    c->dense_ws = nullptr;
-    c->dense_ws_bytes = 0;
-    c->dense_stream = nullptr;
     c->tile_counters = nullptr;
     e = hipMalloc(&c->tile_counters, NOALLOC_COUNTER_BYTES);
     if (e == hipSuccess) e = hipMemset(c->tile_counters, 0, NOALLOC_COUNTER_BYTES);
@@ -667,7 +696,8 @@ int lbq_ctx_destroy(lbq_ctx *ctx) {
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     if (ctx->ws) (void)hipFree(ctx->ws);
     if (ctx->tmp) (void)hipFree(ctx->tmp);
-    if (ctx->dense_ws) (void)hipFree(ctx->dense_ws);
+    for (auto &d : ctx->dense)
+        if (d.p) (void)hipFree(d.p);
     for (uint8_t *p : ctx->outgrown) (void)hipFree(p);
     if (ctx->tile_counters) (void)hipFree(ctx->tile_counters);
     delete ctx;

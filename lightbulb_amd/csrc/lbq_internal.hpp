@@ -249,7 +249,7 @@ hipError_t launch_row_exponents(int type, const uint8_t *w, int64_t n, int64_t k
 // Dense F32 / F16 weights (candle's dense QMatMul variant): y[m][n] = x . W^T in
 // f32, W [n][k] in its file layout widened on the fly; k % 8 == 0.
 constexpr bool is_dense(int t) { return t == TYPE_F32 || t == TYPE_F16 || t == TYPE_BF16; }
-// F16 / BF16 at m > 8 take dense_workspace_bytes(type, n, k, m) bytes of device
+// At m > 8 these types take dense_workspace_bytes(type, n, k, m) bytes of device
 // memory at ws for x's operand pieces and split-k partials (the 16-bit matrix
 // cores); without it (nullptr, or 0 bytes asked) the f32 matrix-core kernel runs.
 size_t dense_workspace_bytes(int type, int64_t n, int64_t k, int64_t m);

@@ -243,3 +243,77 @@ def test_dense_mm_nonfinite_batch(lbq, dev, t, m, n, k):
     assert np.array_equal(y[same], clean[same])
     x2[:] = np.nan
     assert np.isnan(qm2.forward(to_dev(x2, dev)).cpu().numpy()).all()
+
+
+@pytest.mark.parametrize("t", [F16, F32])
+def test_dense_mm_streams_side_by_side(lbq, dev, t):
+    # many streams, a graph captured on one of them and replayed on another, none ordered
+    # against the others: every call's own result
+    rng = np.random.default_rng(31)
+    qm, w = _weight(t, 640, 2048, rng, dev)
+    xs = [rng.standard_normal((m, 2048)).astype(np.float32) for m in (40, 60, 130, 300)]
+    xd = [to_dev(x, dev) for x in xs]
+    want = [qm.forward(x).cpu().numpy() for x in xd]
+    for x, y in zip(xs, want):
+        _assert_rows(y, x.astype(np.float64) @ w.T, _bound(t, 2048))
+    streams = [torch.cuda.Stream() for _ in range(20)]
+    graphs = []
+    for i in (0, 2):  # two graphs from one stream, the second larger
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=streams[0]):
+            graphs.append((g, qm.forward(xd[i]), want[i]))
+    torch.cuda.synchronize()
+    for _ in range(4):
+        ys = []
+        for g, yg, _ in graphs:
+            yg.zero_()
+        torch.cuda.synchronize()
+        for j, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                if j in (1, 3):
+                    graphs[j // 2][0].replay()
+                ys += [(qm.forward(xd[i]), i) for i in ((j + 1) % 4, (j + 3) % 4)]
+        torch.cuda.synchronize()
+        for g, yg, ref in graphs:
+            assert np.array_equal(yg.cpu().numpy(), ref)
+        for y, i in ys:
+            assert np.array_equal(y.cpu().numpy(), want[i])
+
+
+def test_dense_mm_beside_a_capture(lbq, dev):
+    # a call that has to allocate, in another thread and on another stream than a capture in
+    # progress (whose mode forbids allocations elsewhere by default), does not end the capture
+    import threading
+
+    rng = np.random.default_rng(37)
+    qm, w = _weight(F16, 256, 1024, rng, dev)
+    x = rng.standard_normal((64, 1024)).astype(np.float32)
+    xd, y, ys = to_dev(x, dev), torch.empty(64, 256, device=dev), torch.empty(64, 256, device=dev)
+    want = qm.forward(xd).cpu().numpy()
+    other = torch.cuda.Stream()
+    ctx, h, rc = ctypes.c_void_p(), ctypes.c_void_p(), []
+    assert lbq.lbq_init(0, ctypes.byref(ctx)) == 0
+    data = qm.qtensor().data
+    assert lbq.lbq_weight_wrap_device(ctx, F16, 256, 1024, data.data_ptr(), data.numel(), ctypes.byref(h)) == 0
+    try:
+        def beside():
+            rc.append(lbq.lbq_qmatmul_f32(ctx, h, xd.data_ptr(), 64, ys.data_ptr(), ctypes.c_void_p(other.cuda_stream)))
+
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            th = threading.Thread(target=beside)
+            th.start()
+            th.join()
+            assert lbq.lbq_qmatmul_f32(ctx, h, xd.data_ptr(), 64, y.data_ptr(),
+                                       ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)) == 0
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(y.cpu().numpy(), want)
+        assert rc == [0] and np.array_equal(ys.cpu().numpy(), want)
+    finally:
+        torch.cuda.synchronize()
+        lbq.lbq_weight_destroy(h)
+        lbq.lbq_ctx_destroy(ctx)
