@@ -106,3 +106,37 @@ def test_square_group_mixes_kernels(oracle, lbq, dev):
         rows = [0, 200, m - 1]
         ref = oracle.qmatmul(t, raws[0][0], ns[0], k, xd.cpu().numpy()[rows], nthreads=8).astype(np.float64)
         assert_rows_close(qs[0].forward(xd)[rows].cpu().numpy(), ref, tight_bound(t, m))
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q4_K, Q6_K])
+@pytest.mark.parametrize("k", [512, 4352])
+@pytest.mark.parametrize("off", [0, 1])
+def test_norm_then_square_pair(oracle, lbq, dev, t, k, off, monkeypatch):
+    # the norm inside the pre-pass (off = 1: the norm weight only 4-byte aligned, a launch of
+    # its own) and the pair after it: the bits of the two products and the product launch
+    rng = np.random.default_rng(19 * t + k)
+    m, n = 300, 8300
+    (rg, gd), (ru, ud) = _blocks(oracle, rng, t, n, k, dev), _blocks(oracle, rng, t, n, k, dev)
+    x = (3.0 * rng.standard_normal((m, k))).astype(np.float32)
+    w = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    xd, wd = to_dev(x, dev), to_dev(np.concatenate([np.zeros(off), w]).astype(np.float32), dev)[off:]
+    outs = []
+
+    def run(L, ctx, hs):
+        y = torch.full((m, n), float("nan"), device=dev)
+        torch.cuda.synchronize()
+        assert L.lbq_rmsnorm_gate_up_silu_f32(ctx, hs[0], hs[1], xd.data_ptr(), wd.data_ptr(), 1e-5, m, y.data_ptr(), None) == 0
+        torch.cuda.synchronize()
+        outs.append(y.cpu().numpy())
+
+    _with_env(monkeypatch, {}, t, [gd, ud], n, k, run)
+    _with_env(monkeypatch, {"LBQ_GEMM_BIG": "square", "LBQ_GEMM_PAIR_OFF": "1"}, t, [gd, ud], n, k, run)
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    rows = [0, 128, 255, 256, m - 1]
+    x64 = x[rows].astype(np.float64)
+    xn = (x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-5) * w).astype(np.float32)
+    g = oracle.qmatmul(t, rg, n, k, xn, nthreads=8).astype(np.float64)
+    u = oracle.qmatmul(t, ru, n, k, xn, nthreads=8).astype(np.float64)
+    # the fp16 operands' bound of test_square_pair, and of x_norm rounded in f32 another
+    # way: codes at a tie move by one, 2^-7 of a block's largest for few of its values
+    assert_rows_close(outs[0][rows], g / (1.0 + np.exp(-g)) * u, 2e-3)
