@@ -450,32 +450,33 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float *__restrict__ x, co
     for (int64_t i = t; i < k; i += 256) y[m * k + i] = xr[i] / rms * w[i];
 }
 
-// The same for rows up to 256 P values: the row and the weight in registers, loaded once,
-// every load in flight before the first is used (no branch around a load), in the order of
-// k_rmsnorm's sum (the same bits).  Bound by one pass's latency, by memory from about a
-// thousand rows: k_rmsnorm's two passes of one load a step -> this, 512x4096 11.0 -> 5.9
-// us, 4096x4096 32.2 -> 21.3.  16-byte loads with sums of four neighbours took 5.6 and 20.7
-// but gave another last bit.
+// The same for 16-byte aligned rows of k % 4 == 0 up to 1024 P values: the row and the
+// weight in registers, loaded once, 16 bytes at a time, and a copy of the row in LDS for
+// the sum in k_rmsnorm's order (the same bits).  Bound by one pass's latency, by memory from
+// about a thousand rows; k_rmsnorm -> this: 32x4096 6.5 -> 3.6 us, 512x4096 7.9 -> 5.3,
+// 4096x4096 31.5 -> 20.3, 32x16384 20.2 -> 7.1 (sums of a thread's own values, in another
+// order, 3.1, 4.7, 20.1 and 5.2).
 template <int P>
-__global__ __launch_bounds__(256) void k_rmsnorm_r(const float *__restrict__ x, const float *__restrict__ w, float eps,
+__global__ __launch_bounds__(256) void k_rmsnorm_v(const float *__restrict__ x, const float *__restrict__ w, float eps,
                                                    int64_t k, float *__restrict__ y) {
+    __shared__ float4 row[256 * P];
     const int64_t m = blockIdx.x;
-    const int t = threadIdx.x;
-    const float *xr = x + m * k;
-    const int last = (int)k - 1;
-    float v[P], g[P];
+    const int t = threadIdx.x, k4 = (int)(k / 4);
+    const float4 *xr = reinterpret_cast<const float4 *>(x + m * k), *wr = reinterpret_cast<const float4 *>(w);
+    float4 v[P], g[P];
 #pragma unroll
-    for (int j = 0; j < P; j++) v[j] = xr[min(t + 256 * j, last)];
+    for (int j = 0; j < P; j++) v[j] = xr[min(t + 256 * j, k4 - 1)];
 #pragma unroll
-    for (int j = 0; j < P; j++) g[j] = w[min(t + 256 * j, last)];
-    float ss = 0.f;
+    for (int j = 0; j < P; j++) g[j] = wr[min(t + 256 * j, k4 - 1)];
 #pragma unroll
-    for (int j = 0; j < P; j++) ss = t + 256 * j <= last ? fmaf(v[j], v[j], ss) : ss;
-    const float rms = rms_of_256(ss, t, k, eps);
-    float *yr = y + m * k;
+    for (int j = 0; j < P; j++) row[t + 256 * j] = v[j];
+    __syncthreads();
+    const float rms = row_rms(reinterpret_cast<const float *>(row), t, k, eps);
+    float4 *yr = reinterpret_cast<float4 *>(y + m * k);
 #pragma unroll
     for (int j = 0; j < P; j++)
-        if (t + 256 * j <= last) yr[t + 256 * j] = v[j] / rms * g[j];
+        if (t + 256 * j < k4)
+            yr[t + 256 * j] = make_float4(v[j].x / rms * g[j].x, v[j].y / rms * g[j].y, v[j].z / rms * g[j].z, v[j].w / rms * g[j].w);
 }
 
 // candle's RmsNorm (f32) of each row and the Q8_K quantisation of the result in
@@ -564,11 +565,12 @@ hipError_t launch_rmsnorm_q8k(const float *x, const float *w, float eps, int64_t
 
 hipError_t launch_rmsnorm(const float *x, const float *w, float eps, int64_t m, int64_t k, float *y, hipStream_t st) {
     if (m <= 0) return hipSuccess;
-    if (k <= 16384) {
-        if (k <= 2048) k_rmsnorm_r<8><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
-        else if (k <= 4096) k_rmsnorm_r<16><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
-        else if (k <= 8192) k_rmsnorm_r<32><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
-        else k_rmsnorm_r<64><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
+    const uintptr_t all = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y);
+    if (k % 4 == 0 && k <= 16384 && !(all & 15u)) {
+        if (k <= 2048) k_rmsnorm_v<2><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
+        else if (k <= 4096) k_rmsnorm_v<4><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
+        else if (k <= 8192) k_rmsnorm_v<8><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
+        else k_rmsnorm_v<16><<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
         return hipGetLastError();
     }
     k_rmsnorm<<<(unsigned)m, 256, 0, st>>>(x, w, eps, k, y);
