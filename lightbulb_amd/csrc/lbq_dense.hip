@@ -411,7 +411,7 @@ __global__ __launch_bounds__(256) void k_dense_pieces(const float *__restrict__ 
     const float *xr = x + m * K;
     unsigned short *a = A + m * Kp;
     const int64_t ps = rows * Kp;
-    for (int64_t c = 8 * threadIdx.x; c < Kp; c += 2048) {
+    for (int64_t c = 8 * threadIdx.x; c < Kp; c += 8 * blockDim.x) {
         float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         if (c < K) load_x8(xr + c, xv, v);
         uint32_t pc[3][4];
@@ -844,16 +844,19 @@ struct DensePlan {
     DenseGrid g;
     size_t a_off, part_off, total;
 };
-// Tile by m (32, 64, 128 rows; 128 x 256 where such tiles fill the chip by themselves:
+// Tile by m (32, 64, 128 rows; 64 also where 128-row tiles would leave half the CUs idle and
+// k is too short for slices: F16 512x256 M = 1000 15.4 -> 11.7 us, M = 4000 22.5 -> 18.5, F32
+// 4096x256 M = 300 18.0 -> 13.6; 128 x 256 where such tiles fill the chip by themselves:
 // BF16 8192^2 M = 2048 945 -> 622 us, 14336x4096 M = 512 158 -> 143), then k split until the
 // resident workgroups (three of the 32-row tiles a CU, two of the 64-row, one of the
 // 128-row) are there, at least 256 values of k a slice.
 DensePlan dense_plan(int type, int64_t n, int64_t k, int64_t m) {
     DensePlan p;
     const bool w32 = type == TYPE_F32;
-    p.bm = m <= 32 ? 32 : m <= 64 ? 64 : 128;
-    p.bn = 128;
     const int64_t cus = num_cus();
+    const bool idle = ((m + 127) / 128) * ((n + 127) / 128) * 2 <= cus && k < 8 * DK;
+    p.bm = m <= 32 ? 32 : m <= 64 || idle ? 64 : 128;
+    p.bn = 128;
     if (p.bm == 128 && ((m + 127) / 128) * ((n + 255) / 256) * 4 >= 3 * cus) p.bn = 256;
     p.g.tiles_m = (int)((m + p.bm - 1) / p.bm);
     p.g.tiles_n = (int)((n + p.bn - 1) / p.bn);
@@ -876,6 +879,10 @@ DensePlan dense_plan(int type, int64_t n, int64_t k, int64_t m) {
 size_t dense_workspace_bytes(int type, int64_t n, int64_t k, int64_t m) {
     // the buffer resources: 128 rows of pieces, 256 of f32 weights within 2^31 bytes
     if (m <= 8 || k % 8 || k > (type == TYPE_F32 ? 1 << 20 : 1 << 22) || m > 65535) return 0;
+    // one stage and one launch of k_dense_gemm instead: 4096 x 64 M = 9 / 100 F16 8.9 / 10.2 -> 7.0 /
+    // 7.7 us; with more outputs its rate counts (16384 x 64 M = 4000, F16 / BF16 / F32, 131 / 131 / 148
+    // against 126 / 101 / 124)
+    if (k <= DK && m * n < (int64_t)1 << 22) return 0;
     return dense_plan(type, n, k, m).total;
 }
 
@@ -884,7 +891,7 @@ static hipError_t dense_pieces(int type, const uint8_t *w, int64_t n, int64_t k,
     const DensePlan p = dense_plan(type, n, k, m);
     unsigned short *a = reinterpret_cast<unsigned short *>(ws + p.a_off);
     float *out = p.g.splits > 1 ? reinterpret_cast<float *>(ws + p.part_off) : y;
-    k_dense_pieces<<<(unsigned)m, 256, 0, st>>>(x, k, p.g.Kp, p.g.rows, a);
+    k_dense_pieces<<<(unsigned)m, p.g.Kp >= 2048 ? 256 : p.g.Kp > 512 ? 128 : 64, 0, st>>>(x, k, p.g.Kp, p.g.rows, a);
     const unsigned grid = (unsigned)(p.g.tiles_m * p.g.tiles_n * p.g.splits);
     auto go = [&](auto kern, int threads) { kern<<<grid, threads, 0, st>>>(w, n, k, a, x, m, out, p.g); };
     const dim3 sg((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32));
