@@ -189,7 +189,7 @@ def test_dense_mm_f32_products(lbq, dev):
     # for the first pieces' sum and again for its sum with the others; what is left out is
     # 2^-32), values whose pieces are as large as they get
     rng = np.random.default_rng(23)
-    m, n, k = 300, 300, 8
+    m, n, k = 300, 300, 72
     bits = lambda s: (0x3f800000 | 0xff7f | (rng.integers(0, 128, s) << 16)).astype(np.uint32).view(np.float32)
     x, w = np.zeros((m, k), np.float32), np.zeros((n, k), np.float32)
     x[:, 5], w[:, 5] = bits(m), bits(n)
@@ -317,3 +317,16 @@ def test_dense_mm_beside_a_capture(lbq, dev):
         torch.cuda.synchronize()
         lbq.lbq_weight_destroy(h)
         lbq.lbq_ctx_destroy(ctx)
+
+
+@pytest.mark.parametrize("t", [F16, BF16, F32])
+# one stage of k and one value more; k without slices on 64-row tiles, their edges, and with slices
+@pytest.mark.parametrize("m,n,k", [(100, 520, 64), (4100, 1030, 64), (100, 520, 72), (129, 130, 504), (1000, 500, 256),
+                                   (129, 130, 512), (4000, 1100, 128)])
+def test_dense_mm_short_k(lbq, dev, t, m, n, k):
+    rng = np.random.default_rng(m + k)
+    qm, w = _weight(t, n, k, rng, dev)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    y = qm.forward(to_dev(x, dev)).cpu().numpy()
+    rows = sorted({0, 31, 32, 63, 64, 127, 128, m // 2, m - 1} & set(range(m)))
+    _assert_rows(y[rows], x[rows].astype(np.float64) @ w.T, _bound(t, k))
