@@ -647,7 +647,7 @@ def configs_bench(torch, qz, gen, dev, stream, prefill=None):
                                            "working_set_MB": ws_mb(f16),
                                            "frac_hbm": round(fb / us / 1e3 / HBM_PEAK_GBS, 4),
                                            "TFLOP/s": round(fl / us / 1e6, 1),
-                                           "path": "f32 GEMV (m <= 8) / two fp16 operands for x, v_mfma_f32_32x32x16_f16 GEMM"}
+                                           "path": "f32 GEMV (m <= 8) / three bf16 operands for x and two for the weight, v_mfma_f32_32x32x16_bf16 GEMM"}
         log(f"dense F16 M={M}: {us:.1f} us")
     del f16
     # Q8_0 batched (prefill of the same weight): M = 16 and 64 on the integer matrix

@@ -205,14 +205,17 @@ int lbq_qmatmul_group_f32(lbq_ctx *ctx, const lbq_weight *const *ws, int count, 
 /* The gate/up half of the reference's MLP forward (/root/reference/src/model/
  * mlp_wrapper.rs:190-194: `silu(gate_proj.forward(x)) * up_proj.forward(x)`):
  * d_out[m][n] = silu(x . Wg^T) * (x . Wu^T), silu(v) = v / (1 + exp(-v)) in f32.
- * The two products are computed exactly as lbq_qmatmul_f32 computes them.  At
- * m = 1, and for Q4_K / Q5_K weights of more than 8192 rows (and more than 32
+ * The two products are those of lbq_qmatmul_f32 on the same values.  At
+ * m = 1, for Q4_K / Q5_K weights of more than 8192 rows (and more than 32
  * rows per CU) at m = 5..32 -- m = 2..32 when k > 8192 -- (after one activation
- * quantisation), both weights stream through one launch and the product is
+ * quantisation), and for the MFMA types but Q4_1 / Q5_1 from m = 256 where tiles of 256
+ * rows by 128 outputs keep more than half the CUs busy (after one operand
+ * pre-pass), both weights run in one launch and the product is
  * formed in its epilogue, so neither product is written out; otherwise
- * the grouped path fills context memory and one elementwise launch combines it
- * (the m = 2..32 pair launch gives the same bits as that).  gate and up share the
- * ggml type, n and k. */
+ * the grouped path fills context memory and one elementwise launch combines it.
+ * The m = 2..32 pair launch gives the same bits as that; the one from m = 256 sums each
+ * output's k in one piece, and differs in f32 summation order where lbq_qmatmul_f32
+ * splits k.  gate and up share the ggml type, n and k. */
 int lbq_gate_up_silu_f32(lbq_ctx *ctx, const lbq_weight *w_gate, const lbq_weight *w_up, const float *d_x, int64_t m,
                          float *d_out, void *stream);
 
@@ -226,8 +229,11 @@ int lbq_gate_up_silu_f32(lbq_ctx *ctx, const lbq_weight *w_gate, const lbq_weigh
  * pre-quantised Q8_K activations (k-quants, k % 256 == 0 up to 16384, x and
  * norm_w 16-byte aligned; m <= 8, or Q4_K/Q5_K weights on the matrix-core batch
  * decode), the norm runs inside the one Q8_K quantisation launch, x_norm again
- * never written; otherwise x_norm goes to context memory first.
- * lbq_rmsnorm_f32 is the norm alone. */
+ * never written.  At m > 8, where every weight runs the MFMA GEMM behind a pre-pass by
+ * rows (k % 256 == 0 up to 16384, x and norm_w 16-byte aligned, not the k-sliced kernel
+ * of small m), the norm runs inside that pre-pass, with the bits of
+ * lbq_rmsnorm_f32 followed by the calls without a norm.  Otherwise x_norm goes to context
+ * memory first.  lbq_rmsnorm_f32 is the norm alone. */
 int lbq_rmsnorm_f32(const float *d_x, const float *d_w, float eps, int64_t m, int64_t k, float *d_y, void *stream);
 int lbq_rmsnorm_qmatmul_group_f32(lbq_ctx *ctx, const lbq_weight *const *ws, int count, const float *d_x,
                                   const float *d_norm_w, float eps, int64_t m, float *const *d_ys, void *stream);

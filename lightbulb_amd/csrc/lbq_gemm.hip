@@ -545,7 +545,10 @@ Plan plan_for(int type, int64_t n, int64_t k, int64_t m) {
     // square tile takes about 8.2 us per block of k with every CU busy, the wide and
     // tall tiles of half its size 5.0 (Q4_K 14336x4096 M = 2048 / 4096 302 / 590 ->
     // 261 / 545 us, Q8_0 8192^2 M = 2048 371 -> 329; with fewer tiles than half the
-    // CUs and k split they lose: 14336x4096 M = 512 76 -> 92)
+    // CUs and k split they lose: 14336x4096 M = 512 76 -> 92).  The line holds for the
+    // other types too: 6144x4096 M = 2048 Q2_K 148 -> 115, Q3_K 177 -> 129, Q4_0 149 -> 115, Q5_0
+    // 161 -> 120, Q5_K 161 -> 124, Q6_K 185 -> 153, and none of the eight slower at five
+    // shapes and M = 256 to 4096
     if (square_ok(type, k, m) && (!tu.gemm_big || tu.gemm_big == 3)) {
         const int64_t tiles = square_tiles(n, m, XBN), half = (int64_t)p.tiles_m * p.tiles_n * p.splits;
         const int64_t rs = (tiles + slots - 1) / slots * nb * 82, rh = (half + slots - 1) / slots * p.bps * 50;

@@ -9,7 +9,7 @@
 // exact), so an output takes one f32 FMA per block.  The offset types' m_w s_x of four
 // blocks is one more MFMA straight into the sums.  The arithmetic is the reference's but
 // for the f32 summation order: relative error against 64 bits as the integer decode
-// kernel's (Q8_0 5760x2880, M = 200: @@ERR), infinite and NaN scales included.
+// kernel's (Q8_0 5760x2880, M = 200: 7.6e-8), infinite and NaN scales included.
 //
 // These shapes ran the decode GEMV over chunks of 8 rows before: the weights read, and
 // a launch, per chunk.  Here a pre-pass (k_b32_ops) quantises x and writes the codes as
@@ -22,7 +22,7 @@
 // small m by the launches and the weight stream.  (With the activations as fp16 hi + lo
 // operands scaled by d_x, four MFMAs and four reads per block and tile, the LDS reads
 // held the kernel: 34.7 against 30.4 us at M = 200.)  Few tiles: k is split over
-// workgroups, partials added in order by k_b32_sum.
+// workgroups, partials added in order by k_split_sum.
 //
 // us per call, row chunks -> now: Q8_0 5760x2880 M = 9 / 32 / 64 / 200 19.6 / 52 / 101 /
 // 310 -> 17.4 / 18.3 / 22.5 / 36.0; Q5_0 4096x4128 M = 128 249 -> 35.3; Q4_0 8000x8160
