@@ -356,9 +356,10 @@ struct B32Plan {
     size_t a_off, d_off, s_off, part_off, total;
 };
 // Row tiles by m (32, 64 or 128 rows); k split until the resident workgroups (one a CU,
-// two of 32 or 64 rows) are there, at least two stages a slice -- one where the slices of
-// one stage still fit the CUs (Q8_0 4096x1056 M = 9 15.8 -> 12.7 us, 8192x544 14.4 -> 11.8;
-// elsewhere more slices only add partials: 5760x2880 M = 9 17.4 -> 21.0).
+// two of 32 or 64 rows) are there, at least two stages a slice -- one where up to sixteen
+// slices of one stage fit the CUs (Q8_0 4096x1056 M = 9 15.8 -> 12.7 us, 8192x544 14.4 ->
+// 11.8), or more of them half the CUs; elsewhere more slices only add partials: 5760x2880
+// M = 9 17.4 -> 21.0, 1024x8160 M = 40 20.0 -> 22.4.
 B32Plan b32_plan(int type, int64_t n, int64_t k, int64_t m) {
     B32Plan p;
     p.tm = m <= 32 ? 1 : m <= 64 ? 2 : 4;
@@ -366,7 +367,7 @@ B32Plan b32_plan(int type, int64_t n, int64_t k, int64_t m) {
     p.g.tiles_m = (int)((m + 32 * p.tm - 1) / (32 * p.tm));
     p.g.tiles_n = (int)((n + B32_BN - 1) / B32_BN);
     const int64_t tiles = (int64_t)p.g.tiles_m * p.g.tiles_n, slots = (int64_t)num_cus() * (p.tm == 4 ? 1 : 2);
-    const int64_t most = tiles * p.nst <= num_cus() ? p.nst : p.nst / 2;
+    const int64_t most = (p.nst <= 16 ? 1 : 2) * tiles * p.nst <= num_cus() ? p.nst : p.nst / 2;
     const int64_t s = std::max<int64_t>(1, std::min(slots / tiles, most));
     p.g.sps = (int)((p.nst + s - 1) / s);
     p.g.splits = (p.nst + p.g.sps - 1) / p.g.sps;
