@@ -168,8 +168,8 @@ int lbq_weight_info(const lbq_weight *w, uint32_t *ggml_type, int64_t *n, int64_
  * for one part below 2^-32 of it), sums in f32.  The operands live in memory of the
  * context, a buffer for each stream and for each graph capture, so dense calls
  * need no order with calls on other streams; where there is none (no memory, more
- * than 64 streams, captures that together would hold 1 GiB) the f32 matrix cores
- * run instead.  m == 0 is a no-op. */
+ * than 64 streams, hipStreamPerThread, captures that together would hold 1 GiB), and at
+ * k <= 64 with less than 2^22 outputs, the f32 matrix cores run instead.  m == 0 is a no-op. */
 int lbq_qmatmul_f32(lbq_ctx *ctx, const lbq_weight *w, const float *d_x, int64_t m, float *d_y, void *stream);
 
 /* lbq_qmatmul_f32's result (the same kernels, the same bits), allocating

@@ -427,6 +427,7 @@ uint8_t *dense_workspace(Scratch &sc, const lbq_weight *w, int64_t m, hipStream_
     const size_t need = lbq::dense_workspace_bytes(w->type, w->n, w->k, m);
     if (!need) return nullptr;
     if (sc.fixed) return need <= sc.fixed_bytes ? sc.fixed : nullptr;
+    if (st == hipStreamPerThread) return nullptr;  // one handle for a stream of each thread
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     if (hipStreamGetCaptureInfo(st, &cap, &id) != hipSuccess || cap == hipStreamCaptureStatusInvalidated) {
@@ -445,7 +446,8 @@ uint8_t *dense_workspace(Scratch &sc, const lbq_weight *w, int64_t m, hipStream_
         else streams++;
     }
     if (b && b->bytes >= need) return b->p;
-    if (captured ? held + need > DENSE_CAPTURED_BYTES : !b && streams >= DENSE_STREAMS) return nullptr;
+    const size_t want = std::max(need, b ? 2 * b->bytes : 0);  // (as grow_buffer)
+    if (captured ? held + want > DENSE_CAPTURED_BYTES : !b && streams >= DENSE_STREAMS) return nullptr;
     if (!b) {
         try {
             c->dense.push_back({st, captured, id, nullptr, 0});

@@ -330,3 +330,33 @@ def test_dense_mm_short_k(lbq, dev, t, m, n, k):
     y = qm.forward(to_dev(x, dev)).cpu().numpy()
     rows = sorted({0, 31, 32, 63, 64, 127, 128, m // 2, m - 1} & set(range(m)))
     _assert_rows(y[rows], x[rows].astype(np.float64) @ w.T, _bound(t, k))
+
+
+def test_dense_mm_per_thread_streams(lbq, dev):
+    # hipStreamPerThread: one handle, a stream of its own in each thread
+    import threading
+
+    from lightbulb_amd.quantized import context
+    rng = np.random.default_rng(41)
+    n, k = 1024, 2048
+    qm, w = _weight(F16, n, k, rng, dev)
+    xs = [rng.standard_normal((m, k)).astype(np.float32) for m in (300, 200, 100, 40)]
+    xd = [to_dev(x, dev) for x in xs]
+    ys = [torch.empty(x.shape[0], n, device=dev) for x in xs]
+    torch.cuda.synchronize()
+    rc = []
+
+    def calls(i):
+        for _ in range(5):
+            rc.append(lbq.lbq_qmatmul_f32(context(dev), qm._handle, xd[i].data_ptr(), xs[i].shape[0], ys[i].data_ptr(),
+                                          ctypes.c_void_p(2)))
+
+    threads = [threading.Thread(target=calls, args=(i,)) for i in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    assert rc == [0] * 20
+    for x, y in zip(xs, ys):  # k/2 sums of two products, one after the other
+        _assert_rows(y.cpu().numpy(), x.astype(np.float64) @ w.T, 2.0 ** -23 * (k / 2) ** 0.5)
